@@ -648,25 +648,70 @@ void launch_pack_chunks(const uint8_t* src, int64_t slot, const int32_t* lens, c
 }
 
 // ---------------------------------------------------------------------------
-// Arithmetic encoder (arith_coder.rs:26-136), one thread per chunk.
+// Arithmetic encoder (arith_coder.rs:26-136), one thread per chunk.  A chunk
+// is one chain of dependent steps, so the kernel is bound by that chain's
+// latency whatever the number of chunks.  A step takes its shifts in closed
+// form: after the k = clz(low ^ high) shifts that settle a leading bit (32 of
+// them when low == high), the leading bits differ, and the u following ones
+// of low & ~high behind them are the E3 shifts; an E3 shift leaves the leading
+// bits different, so no settled bit follows.  The divisions are one f64
+// estimate each (x / total formed ahead of the chain) with a branch-free
+// integer correction, the intervals are loaded ENC_AHEAD tokens ahead, and the
+// bits leave as whole words.  Measured against a loop per shift, pending bit
+// and correction: 11 chunks of 64 tokens 179 -> 34 us, 49 of 4096 16.3 -> 2.0
+// ms (4.0 -> 0.49 us a token), 38 thousand of 512 2.19 -> 0.29 ms.
 // ---------------------------------------------------------------------------
+constexpr int ENC_AHEAD = 8;  // intervals in flight per thread
+
 struct BitOut {
-    uint8_t* buf;
+    uint8_t* buf;  // 4-byte aligned
     long long cap, len;
-    unsigned cur;
-    int bit_pos;
+    unsigned long long acc;  // the low nacc bits are pending, the oldest on top
+    int nacc;                // < 32 between calls
     int overflow;
-    __device__ void bit(unsigned b) {
-        if (b) cur |= 1u << bit_pos;
-        if (--bit_pos < 0) {
-            if (len < cap) buf[len] = (uint8_t)cur;
+    // whole words leave in stream order (the most significant bit first)
+    __device__ __forceinline__ void flush_word() {
+        const unsigned w = (unsigned)(acc >> (nacc - 32));
+        if (len + 4 <= cap) {
+            *(unsigned*)(buf + len) = __builtin_bswap32(w);
+        } else {
+            for (int i = 0; i < 4; i++)
+                if (len + i < cap) buf[len + i] = (uint8_t)(w >> (24 - 8 * i));
+                else overflow = 1;
+        }
+        len += 4;
+        nacc -= 32;
+    }
+    // the low n bits of v, n <= 32
+    __device__ __forceinline__ void bits(unsigned v, int n) {
+        acc = (acc << n) | (n < 32 ? v & ((1u << n) - 1u) : v);
+        nacc += n;
+        if (nacc >= 32) flush_word();
+    }
+    __device__ __forceinline__ void bit(unsigned b) { bits(b, 1); }
+    __device__ __forceinline__ void run(unsigned b, unsigned n) {  // n copies of b
+        const unsigned v = b ? 0xFFFFFFFFu : 0u;
+        for (; n > 32; n -= 32) bits(v, 32);
+        bits(v, (int)n);
+    }
+    __device__ __forceinline__ void finish() {  // the partial word's bytes, zero-padded
+        while (nacc > 0) {
+            const unsigned b = nacc >= 8 ? (unsigned)(acc >> (nacc - 8)) : (unsigned)(acc << (8 - nacc));
+            if (len < cap) buf[len] = (uint8_t)b;
             else overflow = 1;
             len++;
-            cur = 0;
-            bit_pos = 7;
+            nacc -= 8;
         }
     }
 };
+
+// floor(x * range / total) with range = rm1 + 1 <= 2^32 and xt = x / total
+// rounded: the estimate is within one of the quotient, the remainder test exact
+__device__ __forceinline__ unsigned long long enc_div(unsigned x, double xt, unsigned rm1, double range, unsigned total) {
+    const unsigned long long q = (unsigned)fmin(xt * range, 4294967295.0);
+    const long long r = (long long)((unsigned long long)x * rm1 + x - q * total);
+    return q + (r >= (long long)total ? 1ull : 0ull) - (r < 0 ? 1ull : 0ull);
+}
 
 __global__ __launch_bounds__(64) void k_encode(const uint32_t* __restrict__ lohi, const int32_t* __restrict__ lens,
                                                int nb, int T, unsigned total, uint8_t* __restrict__ out,
@@ -675,42 +720,78 @@ __global__ __launch_bounds__(64) void k_encode(const uint32_t* __restrict__ lohi
     const int c = blockIdx.x * blockDim.x + threadIdx.x;
     if (c >= nb) return;
     const unsigned long long MASK = 0xFFFFFFFFull, HALF = 1ull << 31, QUART = 1ull << 30;
-    unsigned long long low = 0, high = MASK;
+    unsigned low = 0, high = 0xFFFFFFFFu;
     unsigned underflow = 0;
-    BitOut o{out + (size_t)c * slot, slot, 0, 0u, 7, 0};
+    BitOut o{out + (size_t)c * slot, slot, 0, 0ull, 0, 0};
     const double invT = 1.0 / (double)total;
     const int n = lens[c];
     const uint2* lh = (const uint2*)(lohi + (size_t)c * T * 2);
-    uint2 nxt = n > 0 ? lh[0] : make_uint2(0, 0);
-    for (int i = 0; i < n; i++) {
-        const uint2 cur = nxt;
-        if (i + 1 < n) nxt = lh[i + 1];  // prefetch the next interval
-        const unsigned long long range = high - low + 1;
-        high = low + udiv64_32((unsigned long long)cur.y * range, total, invT) - 1;
-        low = low + udiv64_32((unsigned long long)cur.x * range, total, invT);
-        for (;;) {
-            if (((low ^ high) & HALF) == 0) {
-                unsigned bitv = (unsigned)((low >> 31) & 1);
-                o.bit(bitv);
-                for (unsigned u = 0; u < underflow; u++) o.bit(bitv ^ 1u);
+    bool stuck = false;
+    auto step = [&](uint2 cur) {
+        if (stuck) return;
+        const unsigned rm1 = high - low;
+        const double range = (double)rm1 + 1.0;
+        const unsigned long long ql = enc_div(cur.x, (double)cur.x * invT, rm1, range, total);
+        const unsigned long long qh = enc_div(cur.y, (double)cur.y * invT, rm1, range, total);
+        const unsigned nl = low + (unsigned)ql, nh = low + (unsigned)qh - 1u;
+        if (ql < qh) {
+            const int k = __clz((int)(nl ^ nh));  // 32 when they are equal
+            if (k > 0) {
+                const unsigned b = nl >> 31;
+                o.bit(b);
+                if (underflow) o.run(b ^ 1u, underflow);
                 underflow = 0;
-                low = (low << 1) & MASK;
-                high = ((high << 1) & MASK) | 1;
-            } else if ((low & ~high & QUART) != 0) {
-                underflow += 1;
-                low = ((low << 1) ^ HALF) & MASK;
-                high = (((high ^ HALF) << 1) | HALF | 1) & MASK;
-            } else {
-                break;
+                // the k - 1 bits behind the first
+                if (k > 1) o.bits(nl >> (32 - k), k - 1);
+            }
+            const unsigned l1 = k < 32 ? nl << k : 0u;
+            const unsigned h1 = k < 32 ? (nh << k) | ((1u << k) - 1u) : 0xFFFFFFFFu;
+            // E3: bits 30, 29, .. of low & ~high
+            const int u = __clz((int)~((l1 & ~h1) << 1));
+            underflow += (unsigned)u;
+            low = (l1 << u) & 0x7FFFFFFFu;
+            high = (h1 << u) | ((1u << u) - 1u) | 0x80000000u;
+        } else {
+            // an empty interval (a total beyond the coder's range): the
+            // reference's shifts one by one; its range is 0 from here on, and
+            // no later symbol shifts anything
+            unsigned long long l = nl, h = nh;
+            stuck = true;
+            if (low + (unsigned)qh == 0u) return;  // high wrapped below 0: nothing to shift
+            for (;;) {
+                if (((l ^ h) & HALF) == 0) {
+                    const unsigned b = (unsigned)((l >> 31) & 1);
+                    o.bit(b);
+                    o.run(b ^ 1u, underflow);
+                    underflow = 0;
+                    l = (l << 1) & MASK;
+                    h = ((h << 1) & MASK) | 1;
+                } else if ((l & ~h & QUART) != 0) {
+                    underflow += 1;
+                    l = ((l << 1) ^ HALF) & MASK;
+                    h = (((h ^ HALF) << 1) | HALF | 1) & MASK;
+                } else {
+                    break;
+                }
             }
         }
+    };
+    uint2 cur[ENC_AHEAD], nxt[ENC_AHEAD];
+    auto load = [&](uint2* d, int i0) {
+#pragma unroll
+        for (int j = 0; j < ENC_AHEAD; j++) d[j] = lh[min(i0 + j, n - 1)];
+    };
+    if (n > 0) load(cur, 0);
+    for (int i0 = 0; i0 < n; i0 += ENC_AHEAD) {
+        load(nxt, i0 + ENC_AHEAD);
+#pragma unroll
+        for (int j = 0; j < ENC_AHEAD; j++)
+            if (i0 + j < n) step(cur[j]);
+#pragma unroll
+        for (int j = 0; j < ENC_AHEAD; j++) cur[j] = nxt[j];
     }
     o.bit(1u);  // finish(): terminating bit, then flush the partial byte
-    if (o.bit_pos < 7) {
-        if (o.len < o.cap) o.buf[o.len] = (uint8_t)o.cur;
-        else o.overflow = 1;
-        o.len++;
-    }
+    o.finish();
     out_lens[c] = (int32_t)o.len;
     if (o.overflow) atomicOr(err, 1);
 }
