@@ -7,7 +7,10 @@
  * entry point returns czip_status (0 = OK, negative = error class) and leaves
  * a message retrievable with czip_last_error().  A context owns one HIP
  * stream and all device memory it allocates; it is not thread-safe, but
- * several contexts may coexist (one per host thread / device).
+ * several contexts may coexist (one per host thread / device).  The device
+ * memory of a freed job or session stays with the context for its next ones
+ * (at most 1.25 times CZIP_SCRATCH_GB, 80 GB by default) until czip_destroy,
+ * or until an allocation of any context in the process would fail without it.
  *
  * The reference has no FFI; each entry point names the Rust API it stands in
  * for (file:line in the reference crate, rust/src).

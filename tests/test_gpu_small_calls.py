@@ -30,3 +30,52 @@ def test_encoder_chunk_lengths(pair, chunk):
     n = 67 * chunk + (chunk + 1) // 2
     toks = np.random.default_rng(chunk).integers(0, 1024, n).astype(np.uint32)
     assert gm.compress_chunks(toks, chunk) == om.compress_many(toks, chunk, threads=4)
+
+
+def test_job_memory_reuse(pair):
+    """Jobs of one context whose device memory comes back from earlier jobs of
+    other sizes, two of them alive at once, and a decode after a compress:
+    the bytes depend on nothing a block held before."""
+    gm, om = pair
+    rng = np.random.default_rng(5)
+    sizes = [(3000, 512), (40, 64), (9001, 128), (40, 64), (3000, 512), (700, 1024)]
+    ref = []
+    for n, chunk in sizes:
+        toks = rng.integers(0, 1024, n).astype(np.uint32)
+        ref.append((toks, chunk, om.compress_many(toks, chunk, threads=4)))
+    for toks, chunk, want in ref:
+        assert gm.compress_chunks(toks, chunk) == want
+        ntoks = [min(chunk, toks.size - i) for i in range(0, toks.size, chunk)]
+        assert np.array_equal(gm.decompress_chunks(want, ntoks), toks)
+    jobs = [gm.compress_plan(toks, chunk) for toks, chunk, _ in ref]
+    for j in jobs[::2] + jobs[1::2]:
+        j.run()
+    for j, (_, _, want) in zip(jobs, ref):
+        assert j.fetch() == want
+        j.free()
+
+
+def test_job_memory_threads(amd, pair):
+    """A context per thread, both taking and returning device memory at the same time."""
+    import threading
+    _, om = pair
+    toks = np.random.default_rng(6).integers(0, 1024, 5000).astype(np.uint32)
+    want = {c: om.compress_many(toks, c, threads=4) for c in (64, 200)}
+    bad = []
+
+    def work(c):
+        try:
+            gm = amd.Model(amd.ModelWeights(MODEL_PATH))
+            for _ in range(6):
+                if gm.compress_chunks(toks, c) != want[c]:
+                    bad.append(c)
+            gm.close()
+        except Exception as e:  # reported below
+            bad.append(e)
+
+    ts = [threading.Thread(target=work, args=(c,)) for c in want]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    assert not bad
