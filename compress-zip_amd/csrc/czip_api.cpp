@@ -35,6 +35,11 @@ constexpr int DEC_LANES_MAX = 4;  // most HIP streams a decode group is split ov
 // bytes span 256 bytes with 4-key blocks (1 KB with the prefill caches' 16-key blocks); the
 // decode attention reads this layout
 constexpr int DEC_VL = 2;
+// decode steps of at most this many (stream, head) rows take the attention
+// kernel with one row per wavefront (CZIP_ATTN_ROWS).  It gains up to 2.7x
+// while the rows leave SIMDs idle and loses once they queue: 4096 rows 118 ->
+// 64 ms (d512), 12288 rows 16.7 -> 18.3 (v001) and 81 -> 91 ms (d768)
+constexpr long long ATTN_ROWS_MAX = 8192;
 
 struct DevLayer {
     int8_t *attn_norm = nullptr, *post_attn_norm = nullptr, *ffn_norm = nullptr, *post_ffn_norm = nullptr;
@@ -199,6 +204,7 @@ struct czip_ctx {
     bool qkv_gemm = false;        // CZIP_QKV_GEMM: layer 0's QKV by the GEMM, not the per-token table
     double scratch_gb = 0;        // CZIP_SCRATCH_GB: a job's scratch budget
     int64_t decode_streams = 0;   // CZIP_DECODE_STREAMS: most streams per decode group (0: no cap)
+    long long attn_rows = ATTN_ROWS_MAX;  // CZIP_ATTN_ROWS
     int decode_lanes = 0;         // CZIP_DECODE_LANES: lanes per decode group (0: by group size)
     bool lut0_max = false;        // exp2_lut[0] == 65535: the heads' table step 0 is E(0) (HeadCdfArgs::e0)
     std::vector<Alloc> allocs;
@@ -520,6 +526,7 @@ extern "C" czip_status czip_create(const czip_model_desc* w, int device, czip_ct
     if (const char* e = getenv("CZIP_SCRATCH_GB")) c->scratch_gb = atof(e);
     c->pool.set_cap(c->scratch_gb * 1e9 * POOL_SCRATCH_SHARE);
     if (const char* e = getenv("CZIP_DECODE_STREAMS")) c->decode_streams = std::max(1ll, atoll(e));
+    if (const char* e = getenv("CZIP_ATTN_ROWS")) c->attn_rows = std::max(0ll, atoll(e));
     if (const char* e = getenv("CZIP_DECODE_LANES")) {
         const int n = atoi(e);
         if (n >= 1 && n <= DEC_LANES_MAX) c->decode_lanes = n;
@@ -1276,7 +1283,7 @@ static czip_status run_decompress(czip_job* j) {
                     a.q = Ln.r.q8; a.kc = kc; a.vc = vc; a.TP = TP; a.lens = Ln.ds.ntok; a.score_mult = L.score_mult;
                     a.sink = L.sink; a.lut = c->lut; a.etab = c->etab; a.out = Ln.r.attn; a.M = M; a.T = TP; a.H = H;
                     a.G = c->cfg.n_kv_heads; a.KH = c->KH; a.kv_mode = c->cfg.kv_mode; a.coef = 378194u;
-                    a.general = L.attn_general;
+                    a.general = L.attn_general; a.row_max = c->attn_rows;
                     { Timed t(c, "attn_decode"); launch_attn_decode(a, M, p, s); }
                     post_attention(c, Ln.r, l, M, s, nl > 1);
                 }
@@ -1450,7 +1457,7 @@ extern "C" czip_status czip_decode_step(czip_ctx* c, const uint32_t* tok_in, con
         a.q = j->q8; a.kc = kc; a.vc = vc; a.TP = TP; a.lens = j->d_ntok; a.score_mult = L.score_mult;
         a.sink = L.sink; a.lut = c->lut; a.etab = c->etab; a.out = j->attn; a.M = S; a.T = TP; a.H = c->cfg.n_heads; a.G = c->cfg.n_kv_heads;
         a.KH = c->KH; a.kv_mode = c->cfg.kv_mode; a.coef = 378194u;  // ATTN_COEF_Q24 (attention.rs:17-19)
-        a.general = L.attn_general;
+        a.general = L.attn_general; a.row_max = c->attn_rows;
         { Timed t(c, "attn_decode"); launch_attn_decode(a, S, p, s); }
         post_attention(c, row_bufs(c, j), l, S, s);
     }

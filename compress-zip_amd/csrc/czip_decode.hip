@@ -1,6 +1,7 @@
 // Batched autoregressive decode (decompression): one token per stream per
 // step, each stream a chunk of the .czip payload (main.rs:377-396), with an
 // arithmetic decoder per stream kept on the device (arith_coder.rs:139-264).
+#include "czip_attn_row.h"
 #include "czip_attn_tile.h"
 #include "czip_head.h"
 #include "czip_kernels.h"
@@ -309,12 +310,67 @@ __global__ __launch_bounds__(256, 3) void k_attn_decode(AttnArgs a, int p, int G
     });
 }
 
+// The same step with one wavefront per (stream, head) (czip_attn_row.h), four
+// independent wavefronts per workgroup; heads of one stream are neighbours,
+// so their K and V tiles come from L1 after the first.  The next tile's K and
+// V are requested before the current one is summed.
+template <bool GEN>
+__global__ __launch_bounds__(256) void k_attn_decode_row(AttnArgs a, int p) {
+    __shared__ __attribute__((aligned(16))) uint16_t etb[ETB_PAD];
+    __shared__ __attribute__((aligned(16))) AttnRowLds wl[4];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int item = (int)blockIdx.x * 4 + wave;
+    const int b = min(item / a.H, a.B - 1), h = item - (item / a.H) * a.H;
+    const bool act = item < a.B * a.H && p < a.lens[b];
+    const int g = a.kv_mode == 1 ? h * a.G / a.H : 0;
+    const size_t base = ((size_t)b * a.KH + g) * a.TP * 64;
+    const int8_t* kb = a.kc + base + lane * 64;
+    const int* vb = (const int*)(a.vc + base) + lane;  // block n of 4 keys (vt_off, vl = 2): word 64 n + lane
+    v4i k[4];
+    int v[16], q[16];
+    auto load = [&](int t0) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) k[i] = *(const v4i*)(kb + t0 * 64 + i * 16);
+#pragma unroll
+        for (int i = 0; i < 16; i++) v[i] = vb[(t0 / 4 + i) * 64];
+    };
+    if (act) {
+        const int* qp = (const int*)(a.q + ((size_t)b * a.H + h) * 64);
+#pragma unroll
+        for (int i = 0; i < 16; i++) q[i] = qp[i];
+        load(0);
+    }
+    for (int i = tid; i < ETB_PAD / 8; i += 256) ((uint4*)etb)[i] = ((const uint4*)a.etab)[i];
+    __syncthreads();
+    if (!act) return;  // no barrier follows
+    const double mscale = (double)a.score_mult[h] * (1.0 / 32768.0);
+    AttnRow st = attn_row_begin<GEN>(q, a.sink, mscale);
+    for (int t0 = 0; t0 <= p; t0 += 64) {
+        v4i kc[4];
+        int vc[16];
+#pragma unroll
+        for (int i = 0; i < 4; i++) kc[i] = k[i];
+#pragma unroll
+        for (int i = 0; i < 16; i++) vc[i] = v[i];
+        if (t0 + 64 <= p) load(t0 + 64);  // keys t0 + 64 .. + 127 stay inside TP
+        attn_row_tile<GEN>(q, kc, vc, mscale, min(p + 1 - t0, 64), etb, wl[wave], st);
+    }
+    a.out[((size_t)b * a.H + h) * 64 + lane] = attn_row_out(st);
+}
+
 void launch_attn_decode(const AttnArgs& a, int S, int p, hipStream_t s) {
     // heads per KV group: all of them in rust-compat mode (one KV head), H / G
     // in GQA mode (n_heads is a multiple of n_kv_heads); at most 16
     const int G = a.kv_mode == 1 ? a.H / a.G : a.H;
     AttnArgs g = a;
     g.B = S;
+    if ((long long)S * a.H <= a.row_max) {
+        const dim3 grid((unsigned)(((long long)S * a.H + 3) / 4));
+        if (a.general) hipLaunchKernelGGL(k_attn_decode_row<true>, grid, dim3(256), 0, s, g, p);
+        else hipLaunchKernelGGL(k_attn_decode_row<false>, grid, dim3(256), 0, s, g, p);
+        return;
+    }
     const bool two = 2 * G <= 16;
     const long long waves = (long long)(two ? (S + 1) / 2 : S) * a.KH;
     dim3 grid((unsigned)((waves + 3) / 4));

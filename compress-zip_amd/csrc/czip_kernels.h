@@ -73,6 +73,7 @@ struct AttnArgs {
     unsigned coef;
     int general;              // 1: scores may reach 2^30 or lut[0] != 65535 (wrapping score differences)
     int B;                    // chunks of the launch (set by launch_attention)
+    long long row_max = 0;    // decode: most (stream, head) rows taken by the one-row-per-wave kernel
 };
 
 // GEMM over full rows (N = d) with the residual + RMSNorm epilogue

@@ -79,3 +79,36 @@ def test_job_memory_threads(amd, pair):
     for t in ts:
         t.join()
     assert not bad
+
+
+# Decode steps of few rows take the one-row-per-wave attention kernel, which
+# every other decode test of a few streams therefore runs; here the same edge
+# cases through the kernel that packs streams or heads into a wave's rows.
+def test_decode_attention_tile_edge_cases(amd, orc, tmp_path, monkeypatch):
+    import test_gpu_parity as parity
+    monkeypatch.setenv("CZIP_ATTN_ROWS", "0")
+    parity.test_decompress_attention_edge_cases(amd, orc, tmp_path)
+
+
+def test_decode_attention_tile_wrap(amd, orc, tmp_path, monkeypatch):
+    import test_gpu_parity as parity
+    monkeypatch.setenv("CZIP_ATTN_ROWS", "0")
+    parity.test_vacc_wrap(amd, orc, tmp_path)
+
+
+@pytest.mark.parametrize("i", [0, 3, 7, 11, 16, 22, 28, 35])
+def test_decode_attention_tile_random_shapes(orc, tmp_path, monkeypatch, i):
+    import test_gpu_random_shapes as shapes
+    monkeypatch.setenv("CZIP_ATTN_ROWS", "0")
+    shapes.test_random_shape_roundtrip(orc, tmp_path, monkeypatch, i)
+
+
+@pytest.mark.parametrize("n", [1, 3, 4, 5, 63, 64, 65, 128, 129])
+def test_decode_attention_rows_key_counts(pair, n):
+    """Key counts around the 4-key blocks and the 64-key tiles, and stream
+    counts around a workgroup's four rows."""
+    gm, om = pair
+    toks = np.random.default_rng(100 + n).integers(0, 1024, 3 * n).astype(np.uint32)
+    chunks = om.compress_many(toks, n, threads=4)
+    for s in (1, 2, 3):
+        assert np.array_equal(gm.decompress_chunks(chunks[:s], [n] * s), toks[:s * n])
