@@ -40,11 +40,17 @@ constexpr int DEC_VL = 2;
 // while the rows leave SIMDs idle and loses once they queue: 4096 rows 118 ->
 // 64 ms (d512), 12288 rows 16.7 -> 18.3 (v001) and 81 -> 91 ms (d768)
 constexpr long long ATTN_ROWS_MAX = 8192;
+// GEMMs of at most this many rows split K over a workgroup's waves and the
+// columns over the chip (CZIP_SKINNY_ROWS).  Decode of 512 streams: d768 64
+// steps 72 -> 52 ms, d512 128 steps 52 -> 43, v001 256 steps 15.0 -> 14.4; of
+// 1024 streams d768 76 -> 73, d512 59.2 -> 59.6 ms
+constexpr int SKINNY_ROWS_MAX = 512;
 
 struct DevLayer {
     int8_t *attn_norm = nullptr, *post_attn_norm = nullptr, *ffn_norm = nullptr, *post_ffn_norm = nullptr;
     int8_t *qkv_w = nullptr, *out_w = nullptr, *up_w = nullptr, *down_w = nullptr, *sink = nullptr;
     int8_t *out_wf = nullptr, *down_wf = nullptr;  // fragment-major copies (row GEMM)
+    int8_t *qkv_wf = nullptr, *up_wf = nullptr;    // the same (GEMMs of few rows)
     int8_t* up_wf16 = nullptr;  // fragment-major, gate and up tiles interleaved per 16 features (fused FFN)
     int32_t* score_mult = nullptr;
     int qkv_mult, out_mult, up_mult, down_mult, qkv_shift, out_shift, up_shift, down_shift;
@@ -205,6 +211,7 @@ struct czip_ctx {
     double scratch_gb = 0;        // CZIP_SCRATCH_GB: a job's scratch budget
     int64_t decode_streams = 0;   // CZIP_DECODE_STREAMS: most streams per decode group (0: no cap)
     long long attn_rows = ATTN_ROWS_MAX;  // CZIP_ATTN_ROWS
+    int skinny_rows = SKINNY_ROWS_MAX;    // CZIP_SKINNY_ROWS
     int decode_lanes = 0;         // CZIP_DECODE_LANES: lanes per decode group (0: by group size)
     bool lut0_max = false;        // exp2_lut[0] == 65535: the heads' table step 0 is E(0) (HeadCdfArgs::e0)
     std::vector<Alloc> allocs;
@@ -392,10 +399,12 @@ void resolve_events(czip_ctx* c) {
 // the GEMM launches with the context's kernel switch
 void gemm(const czip_ctx* c, GemmArgs g, int epi, hipStream_t s) {
     g.tiled = c->gemm_tiled ? 1 : 0;
+    g.skinny_rows = c->skinny_rows;
     launch_gemm(g, epi, s);
 }
 void gemm_rn(const czip_ctx* c, RowGemmArgs a, hipStream_t s) {
     a.tiled = c->gemm_tiled ? 1 : 0;
+    a.skinny_rows = c->skinny_rows;
     launch_gemm_rn(a, s);
 }
 
@@ -527,6 +536,7 @@ extern "C" czip_status czip_create(const czip_model_desc* w, int device, czip_ct
     c->pool.set_cap(c->scratch_gb * 1e9 * POOL_SCRATCH_SHARE);
     if (const char* e = getenv("CZIP_DECODE_STREAMS")) c->decode_streams = std::max(1ll, atoll(e));
     if (const char* e = getenv("CZIP_ATTN_ROWS")) c->attn_rows = std::max(0ll, atoll(e));
+    if (const char* e = getenv("CZIP_SKINNY_ROWS")) c->skinny_rows = std::max(0, atoi(e));
     if (const char* e = getenv("CZIP_DECODE_LANES")) {
         const int n = atoi(e);
         if (n >= 1 && n <= DEC_LANES_MAX) c->decode_lanes = n;
@@ -560,6 +570,7 @@ extern "C" czip_status czip_create(const czip_model_desc* w, int device, czip_ct
         UP(D.ffn_norm, L.ffn_norm, d)
         UP(D.post_ffn_norm, L.post_ffn_norm, d)
         UP(D.qkv_w, L.qkv_w, (size_t)D.qkv_n * d)
+        if ((rc = upload_frag_major(C, &D.qkv_wf, L.qkv_w, (size_t)D.qkv_n, d))) return rc;
         UP(D.out_w, L.out_w, d * d)
         if ((rc = upload_frag_major(C, &D.out_wf, L.out_w, d, d))) return rc;
         // gate/up interleave in groups of 32 rows so one 64-wide GEMM tile holds matching pairs
@@ -568,6 +579,7 @@ extern "C" czip_status czip_create(const czip_model_desc* w, int device, czip_ct
             memcpy(&perm[(grp * 64 + 32) * d], L.up_w + (F + grp * 32) * d, 32 * d);
         }
         UP(D.up_w, perm.data(), 2 * F * d)
+        if ((rc = upload_frag_major(C, &D.up_wf, perm.data(), 2 * F, d))) return rc;
         UP(D.down_w, L.down_w, d * F)
         if ((rc = upload_frag_major(C, &D.down_wf, L.down_w, d, F))) return rc;
         if (c->ffn_fused) {
@@ -725,11 +737,11 @@ void post_attention(czip_ctx* c, const RowBufs& r, int l, int M, hipStream_t s, 
         set_requant(o, L.out_mult, L.out_shift);
         o.w1 = L.ffn_norm; o.w2 = L.post_attn_norm;
         o.x_in = l == 0 ? nullptr : r.x; o.tok = r.inp; o.embed = c->embed;
-        o.x_out = r.x; o.xn = r.xn; o.ws = r.rn_ws; o.ws_bytes = r.rn_ws_bytes;
+        o.x_out = r.x; o.xn = r.xn; o.ws = r.rn_ws; o.ws_bytes = r.rn_ws_bytes; o.y8 = r.y8;
         { Timed t(c, "gemm_o_norm"); gemm_rn(c, o, s); }
     } else {
         GemmArgs o{};
-        o.A = r.attn; o.W = L.out_w; o.M = M; o.N = d; o.K = d; o.out8 = r.y8; o.ldo = d;
+        o.A = r.attn; o.W = L.out_w; o.Wf = L.out_wf; o.M = M; o.N = d; o.K = d; o.out8 = r.y8; o.ldo = d;
         set_requant(o, L.out_mult, L.out_shift);
         { Timed t(c, "gemm_o"); gemm(c, o, EPI_REQ, s); }
         { Timed t(c, "row_norm"); launch_resid_norm(r.x, r.y8, L.ffn_norm, L.post_attn_norm, M, d, r.xn, s); }
@@ -753,7 +765,7 @@ void post_attention(czip_ctx* c, const RowBufs& r, int l, int M, hipStream_t s, 
         return;
     }
     GemmArgs u{};
-    u.A = r.xn; u.W = L.up_w; u.M = M; u.N = 2 * F; u.K = d; u.out8 = r.r8; u.ldo = F;
+    u.A = r.xn; u.W = L.up_w; u.Wf = L.up_wf; u.M = M; u.N = 2 * F; u.K = d; u.out8 = r.r8; u.ldo = F;
     set_requant(u, L.up_mult, L.up_shift);
     { Timed t(c, "gemm_up"); gemm(c, u, EPI_REGLU, s); }
     if (c->rn_fused) {
@@ -761,11 +773,11 @@ void post_attention(czip_ctx* c, const RowBufs& r, int l, int M, hipStream_t s, 
         dn.A = r.r8; dn.W = L.down_w; dn.Wf = L.down_wf; dn.M = M; dn.K = F; dn.d = d;
         set_requant(dn, L.down_mult, L.down_shift);
         dn.w1 = L.post_ffn_norm; dn.w2 = next;
-        dn.x_in = r.x; dn.x_out = last ? nullptr : r.x; dn.xn = r.xn; dn.ws = r.rn_ws; dn.ws_bytes = r.rn_ws_bytes;
+        dn.x_in = r.x; dn.x_out = last ? nullptr : r.x; dn.xn = r.xn; dn.ws = r.rn_ws; dn.ws_bytes = r.rn_ws_bytes; dn.y8 = r.y8;
         { Timed t(c, "gemm_down_norm"); gemm_rn(c, dn, s); }
     } else {
         GemmArgs dn{};
-        dn.A = r.r8; dn.W = L.down_w; dn.M = M; dn.N = d; dn.K = F; dn.out8 = r.y8; dn.ldo = d;
+        dn.A = r.r8; dn.W = L.down_w; dn.Wf = L.down_wf; dn.M = M; dn.N = d; dn.K = F; dn.out8 = r.y8; dn.ldo = d;
         set_requant(dn, L.down_mult, L.down_shift);
         { Timed t(c, "gemm_down"); gemm(c, dn, EPI_REQ, s); }
         { Timed t(c, "row_norm"); launch_resid_norm(r.x, r.y8, L.post_ffn_norm, next, M, d, r.xn, s); }
@@ -807,7 +819,7 @@ czip_status forward_batch(czip_ctx* c, czip_job* j, int nb, int T, bool head = t
     for (int l = 0; l < c->cfg.n_layers; l++) {
         const DevLayer& L = c->layers[(size_t)l];
         GemmArgs g{};
-        g.A = j->xn; g.W = L.qkv_w; g.M = M; g.N = L.qkv_n; g.K = d;
+        g.A = j->xn; g.W = L.qkv_w; g.Wf = L.qkv_wf; g.M = M; g.N = L.qkv_n; g.K = d;
         g.out8 = j->q8; g.ldo = d; set_requant(g, L.qkv_mult, L.qkv_shift);
         g.d = d; g.T = T; g.TP = pad64(T); g.pos = -1; g.kv_mode = c->cfg.kv_mode; g.G = c->cfg.n_kv_heads; g.KH = c->KH;
         g.kc = j->kc; g.vc = j->vc; g.rcos = c->rcos; g.rsin = c->rsin;
@@ -827,7 +839,7 @@ czip_status forward_batch(czip_ctx* c, czip_job* j, int nb, int T, bool head = t
     }
     if (head) {
         GemmArgs h{};
-        h.A = j->xn; h.W = c->head_w; h.M = M; h.N = V; h.K = d; h.out32 = j->logits; h.ldo = V;
+        h.A = j->xn; h.W = c->head_w; h.Wf = c->head_wf; h.M = M; h.N = V; h.K = d; h.out32 = j->logits; h.ldo = V;
         Timed t(c, "gemm_head");
         gemm(c, h, EPI_RAW, s);
     }
@@ -1269,7 +1281,7 @@ static czip_status run_decompress(czip_job* j) {
                     int8_t* kc = j->kc + (size_t)l * layer_kv + (size_t)Ln.r0 * stream_kv;
                     int8_t* vc = j->vc + (size_t)l * layer_kv + (size_t)Ln.r0 * stream_kv;
                     GemmArgs g{};
-                    g.A = Ln.r.xn; g.W = L.qkv_w; g.M = M; g.N = L.qkv_n; g.K = d;
+                    g.A = Ln.r.xn; g.W = L.qkv_w; g.Wf = L.qkv_wf; g.M = M; g.N = L.qkv_n; g.K = d;
                     g.out8 = Ln.r.q8; g.ldo = d; set_requant(g, L.qkv_mult, L.qkv_shift);
                     g.d = d; g.T = TP; g.TP = TP; g.pos = p; g.vl = DEC_VL; g.kv_mode = c->cfg.kv_mode; g.G = c->cfg.n_kv_heads;
                     g.KH = c->KH; g.kc = kc; g.vc = vc; g.rcos = c->rcos; g.rsin = c->rsin;
@@ -1295,7 +1307,7 @@ static czip_status run_decompress(czip_job* j) {
                     launch_head_dec(h, Ln.st, Ln.ds, s);
                 } else {
                     GemmArgs hd{};
-                    hd.A = Ln.r.xn; hd.W = c->head_w; hd.M = M; hd.N = V; hd.K = d;
+                    hd.A = Ln.r.xn; hd.W = c->head_w; hd.Wf = c->head_wf; hd.M = M; hd.N = V; hd.K = d;
                     hd.out32 = j->logits + (size_t)Ln.r0 * V; hd.ldo = V;
                     { Timed t(c, "gemm_head"); gemm(c, hd, EPI_RAW, s); }
                     {
@@ -1443,7 +1455,7 @@ extern "C" czip_status czip_decode_step(czip_ctx* c, const uint32_t* tok_in, con
         int8_t* kc = j->kc + (size_t)l * layer_kv;
         int8_t* vc = j->vc + (size_t)l * layer_kv;
         GemmArgs g{};
-        g.A = j->xn; g.W = L.qkv_w; g.M = S; g.N = L.qkv_n; g.K = d;
+        g.A = j->xn; g.W = L.qkv_w; g.Wf = L.qkv_wf; g.M = S; g.N = L.qkv_n; g.K = d;
         g.out8 = j->q8; g.ldo = d; set_requant(g, L.qkv_mult, L.qkv_shift);
         g.d = d; g.T = TP; g.TP = TP; g.pos = p; g.vl = DEC_VL; g.kv_mode = c->cfg.kv_mode; g.G = c->cfg.n_kv_heads;
         g.KH = c->KH; g.kc = kc; g.vc = vc; g.rcos = c->rcos; g.rsin = c->rsin;
@@ -1463,7 +1475,7 @@ extern "C" czip_status czip_decode_step(czip_ctx* c, const uint32_t* tok_in, con
     }
     {
         GemmArgs hd{};
-        hd.A = j->xn; hd.W = c->head_w; hd.M = S; hd.N = V; hd.K = d; hd.out32 = j->logits; hd.ldo = V;
+        hd.A = j->xn; hd.W = c->head_w; hd.Wf = c->head_wf; hd.M = S; hd.N = V; hd.K = d; hd.out32 = j->logits; hd.ldo = V;
         { Timed t(c, "gemm_head"); gemm(c, hd, EPI_RAW, s); }
         Timed t(c, "cdf");
         launch_cdf(j->logits, S, V, value_or_null ? j->d_val : nullptr, nullptr, 1, c->lut, c->cfg.coef_q24,
@@ -1520,6 +1532,9 @@ int32_t* carve_prefill(czip_ctx* c, czip_job* j, Carve& cv, int B, int T) {
     j->kc = cv.take<int8_t>(M * (size_t)c->KH * 64);
     j->vc = cv.take<int8_t>((size_t)B * pad64(T) * (size_t)c->KH * 64);
     j->logits = c->head_fused ? nullptr : cv.take<int32_t>(M * V);
+    // the few-row GEMMs' projection output, where the buffer has room for it
+    // (without it those launches take the row GEMM)
+    if (!j->y8 && M <= (size_t)c->skinny_rows && cv.off + M * d + 256 <= NOALLOC_SCRATCH_BYTES) j->y8 = cv.take<int8_t>(M * d);
     return err;
 }
 

@@ -73,9 +73,77 @@ __device__ __forceinline__ void qkv_row(const GemmArgs& a, int row, int c4, QkvR
     }
 }
 
+// ReGLU / QKV epilogue of one column pair: x holds columns col_base + 16 j +
+// c4 .. +3 of `row`, y the columns 32 further (col_base 64-aligned: one head /
+// one gate-up group; j is 0 or 1).
+template <int EPI, bool FAST>
+__device__ __forceinline__ void epi_pair(const GemmArgs& a, v4i x, v4i y, int row, int col_base, int j, int c4,
+                                         const QkvRow& q) {
+    const int i0 = j * 16 + c4;
+    if (EPI == EPI_REGLU) {
+        // W rows were permuted so that a 64-row group holds 32 gate rows then the
+        // matching 32 up rows: output feature f = col_base/2 + j*16 + c4 + r.
+        int o[4];
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const int g = rq<FAST>(x[r], a);
+            const int u = rq<FAST>(y[r], a);
+            const int gr = g > 0 ? g : 0;
+            o[r] = clamp127(rne_shr(gr * u, 7));  // reglu.rs:20-46 (|gr * u| <= 127^2)
+        }
+        *(unsigned*)(a.out8 + (size_t)row * a.ldo + (col_base >> 1) + i0) = pack4i(o[0], o[1], o[2], o[3]);
+        return;
+    }
+    // EPI_QKV: rotary pairs (i0 + r, i0 + r + 32)
+    const int p = q.p, b = q.b;
+    const int kcol = col_base - a.d;
+    int g = 0, isv = 0;
+    if (kcol >= 0) {
+        if (a.kv_mode == 1) { isv = kcol >= 64 * a.G; g = (isv ? kcol - 64 * a.G : kcol) >> 6; }
+        else isv = kcol >= 64;
+    }
+    int xq[4], yq[4], xv[4], yv[4];
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+        xv[r] = rq<FAST>(x[r], a);
+        yv[r] = rq<FAST>(y[r], a);
+        const int c = (int16_t)(r & 1 ? q.cs[j][r >> 1] >> 16 : q.cs[j][r >> 1] & 0xFFFFu);
+        const int sn = (int16_t)(r & 1 ? q.sn[j][r >> 1] >> 16 : q.sn[j][r >> 1] & 0xFFFFu);
+        const int xr = (int)((unsigned)(xv[r] * c) - (unsigned)(yv[r] * sn));
+        const int yr = (int)((unsigned)(xv[r] * sn) + (unsigned)(yv[r] * c));
+        if (kcol < 0) {
+            // Q: attention.rs:53-83 (>>15 then NET_SHIFT=1, two roundings)
+            xq[r] = clamp127(rne_shr(rne_shr(xr, 15), 1));
+            yq[r] = clamp127(rne_shr(rne_shr(yr, 15), 1));
+        } else {
+            // K: attention.rs:29-50 (|xr|, |yr| <= 2 * 127 * 32768)
+            xq[r] = clamp127(rne_shr(xr, 15));
+            yq[r] = clamp127(rne_shr(yr, 15));
+        }
+    }
+    if (kcol < 0) {
+        int8_t* qo = a.out8 + (size_t)row * a.ldo + col_base;
+        *(unsigned*)(qo + i0) = pack4i(xq[0], xq[1], xq[2], xq[3]);
+        *(unsigned*)(qo + i0 + 32) = pack4i(yq[0], yq[1], yq[2], yq[3]);
+    } else if (!isv) {
+        int8_t* k = a.kc + (((size_t)b * a.KH + g) * a.T + p) * 64;
+        *(unsigned*)(k + i0) = pack4i(xq[0], xq[1], xq[2], xq[3]);
+        *(unsigned*)(k + i0 + 32) = pack4i(yq[0], yq[1], yq[2], yq[3]);
+    } else {
+        // V^T in blocks of 2^vl keys (vt_off)
+        const int vl = a.vl;
+        int8_t* v = a.vc + ((size_t)b * a.KH + g) * 64 * a.TP + vt_off(p, 0, vl);
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            v[(i0 + r) << vl] = (int8_t)xv[r];
+            v[(i0 + r + 32) << vl] = (int8_t)yv[r];
+        }
+    }
+}
+
 // Epilogue of one 16-row x 64-column tile: acc[j] holds columns
-// col_base + 16 j + c4 .. +3 of `row` (col_base 64-aligned: one head / one
-// gate-up group).  The caller checks row < M and col_base < N.
+// col_base + 16 j + c4 .. +3 of `row` (col_base 64-aligned).  The caller
+// checks row < M and col_base < N.
 template <int EPI, bool FAST>
 __device__ __forceinline__ void epi_tile(const GemmArgs& a, const v4i* acc, int row, int col_base, int c4,
                                          const QkvRow& q) {
@@ -89,70 +157,9 @@ __device__ __forceinline__ void epi_tile(const GemmArgs& a, const v4i* acc, int 
         for (int j = 0; j < 4; j++)
             *(unsigned*)(a.out8 + (size_t)row * a.ldo + col_base + j * 16 + c4) =
                 pack4i(rq<FAST>(acc[j][0], a), rq<FAST>(acc[j][1], a), rq<FAST>(acc[j][2], a), rq<FAST>(acc[j][3], a));
-    } else if (EPI == EPI_REGLU) {
-        // W rows were permuted so that a 64-row group holds 32 gate rows then the
-        // matching 32 up rows: output feature f = col_base/2 + j*16 + c4 + r.
+    } else {
 #pragma unroll
-        for (int j = 0; j < 2; j++) {
-            int o[4];
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const int g = rq<FAST>(acc[j][r], a);
-                const int u = rq<FAST>(acc[j + 2][r], a);
-                const int gr = g > 0 ? g : 0;
-                o[r] = clamp127(rne_shr(gr * u, 7));  // reglu.rs:20-46 (|gr * u| <= 127^2)
-            }
-            *(unsigned*)(a.out8 + (size_t)row * a.ldo + (col_base >> 1) + j * 16 + c4) = pack4i(o[0], o[1], o[2], o[3]);
-        }
-    } else {  // EPI_QKV
-        const int p = q.p, b = q.b;
-        const int kcol = col_base - a.d;
-        int g = 0, isv = 0;
-        if (kcol >= 0) {
-            if (a.kv_mode == 1) { isv = kcol >= 64 * a.G; g = (isv ? kcol - 64 * a.G : kcol) >> 6; }
-            else isv = kcol >= 64;
-        }
-#pragma unroll
-        for (int j = 0; j < 2; j++) {
-            const int i0 = j * 16 + c4;  // rotary pairs (i0 + r, i0 + r + 32)
-            int xq[4], yq[4], xv[4], yv[4];
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                xv[r] = rq<FAST>(acc[j][r], a);
-                yv[r] = rq<FAST>(acc[j + 2][r], a);
-                const int c = (int16_t)(r & 1 ? q.cs[j][r >> 1] >> 16 : q.cs[j][r >> 1] & 0xFFFFu);
-                const int sn = (int16_t)(r & 1 ? q.sn[j][r >> 1] >> 16 : q.sn[j][r >> 1] & 0xFFFFu);
-                const int xr = (int)((unsigned)(xv[r] * c) - (unsigned)(yv[r] * sn));
-                const int yr = (int)((unsigned)(xv[r] * sn) + (unsigned)(yv[r] * c));
-                if (kcol < 0) {
-                    // Q: attention.rs:53-83 (>>15 then NET_SHIFT=1, two roundings)
-                    xq[r] = clamp127(rne_shr(rne_shr(xr, 15), 1));
-                    yq[r] = clamp127(rne_shr(rne_shr(yr, 15), 1));
-                } else {
-                    // K: attention.rs:29-50 (|xr|, |yr| <= 2 * 127 * 32768)
-                    xq[r] = clamp127(rne_shr(xr, 15));
-                    yq[r] = clamp127(rne_shr(yr, 15));
-                }
-            }
-            if (kcol < 0) {
-                int8_t* qo = a.out8 + (size_t)row * a.ldo + col_base;
-                *(unsigned*)(qo + i0) = pack4i(xq[0], xq[1], xq[2], xq[3]);
-                *(unsigned*)(qo + i0 + 32) = pack4i(yq[0], yq[1], yq[2], yq[3]);
-            } else if (!isv) {
-                int8_t* k = a.kc + (((size_t)b * a.KH + g) * a.T + p) * 64;
-                *(unsigned*)(k + i0) = pack4i(xq[0], xq[1], xq[2], xq[3]);
-                *(unsigned*)(k + i0 + 32) = pack4i(yq[0], yq[1], yq[2], yq[3]);
-            } else {
-                // V^T in blocks of 2^vl keys (vt_off)
-                const int vl = a.vl;
-                int8_t* v = a.vc + ((size_t)b * a.KH + g) * 64 * a.TP + vt_off(p, 0, vl);
-#pragma unroll
-                for (int r = 0; r < 4; r++) {
-                    v[(i0 + r) << vl] = (int8_t)xv[r];
-                    v[(i0 + r + 32) << vl] = (int8_t)yv[r];
-                }
-            }
-        }
+        for (int j = 0; j < 2; j++) epi_pair<EPI, FAST>(a, acc[j], acc[j + 2], row, col_base, j, c4, q);
     }
 }
 
@@ -536,6 +543,121 @@ __global__ __launch_bounds__(256, 2) void k_gemm_ws(GemmArgs a, int ncg) {
     }
 }
 
+// ---------------------------------------------------------------------------
+// GEMM of a few rows (decode steps of few streams, short prefills): bound by
+// the latency of the weights, which come from L2 or the memory behind it and
+// are used once.  A workgroup takes 16 RT rows and 16 output columns (QKV and
+// ReGLU: a pair of 16-column tiles 32 apart, what their epilogues join), its
+// waves split K, and every wave's operands (W fragment-major, A straight from
+// its rows) are requested at once, SKINNY_U K steps at a time.  The waves'
+// sums meet in LDS; wave i sums and finishes row tile i.  Per launch, events
+// included (d768 / 12 layers, 59 rows): QKV 14.3 -> 7.8 us, up + ReGLU 12.8 ->
+// 6.7, O + norms 22 -> 10.3, down + norms (K = 3072) 31 -> 13.9, head (V = 8192)
+// 15 -> 8.1; d512 down + norms at 512 rows 17.4 -> 12.4 (16-row row GEMM).
+// ---------------------------------------------------------------------------
+constexpr int SKINNY_U = 3;  // K steps of operands in flight per wave
+
+template <int EPI, bool FAST, int NW, int RT>
+__global__ __launch_bounds__(64 * NW) void k_gemm_skinny(GemmArgs a) {
+    constexpr int NT = EPI == EPI_QKV || EPI == EPI_REGLU ? 2 : 1;
+    static_assert(RT <= NW, "wave i finishes row tile i");
+    __shared__ v4i part[NW][RT * NT][64];
+    const int tid = threadIdx.x, lane = tid & 63, lr = lane & 15, c4 = (lane >> 4) * 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int m0 = blockIdx.y * 16 * RT;
+    // column tile (16 columns) of the workgroup, its pair two tiles further
+    const int ct = NT == 2 ? (int)(blockIdx.x >> 1) * 4 + (int)(blockIdx.x & 1) : (int)blockIdx.x;
+    const int nks = a.K / 64;
+    const __amdgpu_buffer_rsrc_t rA = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)(a.A + (size_t)m0 * a.K), (short)0, min(a.M - m0, 16 * RT) * a.K, BUF_DWORD3);
+    const __amdgpu_buffer_rsrc_t rW = __builtin_amdgcn_make_buffer_rsrc((void*)a.Wf, (short)0, a.N * a.K, BUF_DWORD3);
+    const int aoff = lr * a.K + (lane >> 4) * 16, woff = ct * nks * 1024 + lane * 16;
+    QkvRow qr;
+    if (EPI == EPI_QKV && wave < RT) qkv_row(a, m0 + wave * 16 + lr, c4, qr);
+    v4i acc[RT][NT];
+#pragma unroll
+    for (int i = 0; i < RT; i++)
+#pragma unroll
+        for (int t = 0; t < NT; t++) acc[i][t] = (v4i){0, 0, 0, 0};
+    for (int k0 = wave; k0 < nks; k0 += NW * SKINNY_U) {
+        v4i w[SKINNY_U][NT], x[SKINNY_U][RT];
+#pragma unroll
+        for (int u = 0; u < SKINNY_U; u++) {
+            const int ks = k0 + u * NW;
+            if (ks < nks) {
+#pragma unroll
+                for (int t = 0; t < NT; t++)
+                    w[u][t] = __builtin_amdgcn_raw_buffer_load_b128(rW, woff + 2 * t * nks * 1024, ks * 1024, 0);
+#pragma unroll
+                for (int i = 0; i < RT; i++)
+                    x[u][i] = __builtin_amdgcn_raw_buffer_load_b128(rA, aoff + i * 16 * a.K, ks * 64, 0);
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < SKINNY_U; u++)
+            if (k0 + u * NW < nks)
+#pragma unroll
+                for (int i = 0; i < RT; i++)
+#pragma unroll
+                    for (int t = 0; t < NT; t++)
+                        acc[i][t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(w[u][t], x[u][i], acc[i][t], 0, 0, 0);
+    }
+#pragma unroll
+    for (int i = 0; i < RT; i++)
+#pragma unroll
+        for (int t = 0; t < NT; t++) part[wave][i * NT + t][lane] = acc[i][t];
+    __syncthreads();
+    if (wave >= RT) return;  // no barrier follows
+    v4i y[NT];
+#pragma unroll
+    for (int t = 0; t < NT; t++) {
+        y[t] = part[0][wave * NT + t][lane];
+#pragma unroll
+        for (int w = 1; w < NW; w++) y[t] += part[w][wave * NT + t][lane];
+    }
+    const int row = m0 + wave * 16 + lr;
+    if (row >= a.M) return;
+    if constexpr (EPI == EPI_RAW) {
+        *(int4*)(a.out32 + (size_t)row * a.ldo + ct * 16 + c4) = make_int4(y[0][0], y[0][1], y[0][2], y[0][3]);
+    } else if constexpr (EPI == EPI_REQ) {
+        *(unsigned*)(a.out8 + (size_t)row * a.ldo + ct * 16 + c4) =
+            pack4i(rq<FAST>(y[0][0], a), rq<FAST>(y[0][1], a), rq<FAST>(y[0][2], a), rq<FAST>(y[0][3], a));
+    } else {
+        epi_pair<EPI, FAST>(a, y[0], y[1], row, (ct >> 2) * 64, ct & 1, c4, qr);
+    }
+}
+
+template <int EPI, bool FAST, int NW>
+static void launch_skinny_nw(const GemmArgs& a, hipStream_t s) {
+    const unsigned nx = (unsigned)(EPI == EPI_QKV || EPI == EPI_REGLU ? a.N / 32 : a.N / 16);
+    if (a.M <= 16)
+        hipLaunchKernelGGL((k_gemm_skinny<EPI, FAST, NW, 1>), dim3(nx, 1), dim3(64 * NW), 0, s, a);
+    else
+        hipLaunchKernelGGL((k_gemm_skinny<EPI, FAST, NW, 4>), dim3(nx, (unsigned)((a.M + 63) / 64)), dim3(64 * NW), 0, s, a);
+}
+
+template <int EPI, bool FAST>
+static void launch_skinny(const GemmArgs& a, hipStream_t s) {
+    // about SKINNY_U K steps a wave
+    const int nks = a.K / 64;
+    if (nks <= 4 * SKINNY_U) launch_skinny_nw<EPI, FAST, 4>(a, s);
+    else if (EPI == EPI_QKV || EPI == EPI_REGLU || nks <= 8 * SKINNY_U) launch_skinny_nw<EPI, FAST, 8>(a, s);
+    else launch_skinny_nw<EPI, FAST, 16>(a, s);
+}
+
+template <int EPI>
+static bool try_skinny(const GemmArgs& a, hipStream_t s) {
+    // every 64 rows read the weights again: the wide head stops paying sooner
+    // (512 rows, V = 8192: 21 -> 30 us; 256 rows 18.8 -> 17.8)
+    const int most = EPI == EPI_RAW ? a.skinny_rows / 2 : a.skinny_rows;
+    if (a.tiled || !a.Wf || a.a_rows || a.M <= 0 || a.M > most || a.N % 64 != 0 || a.K % 64 != 0 ||
+        (long long)a.N * a.K >= (1ll << 31))
+        return false;
+    if (a.rq_fast) launch_skinny<EPI, true>(a, s);
+    else launch_skinny<EPI, false>(a, s);
+    return true;
+}
+
 template <int EPI>
 static void launch_epi(const GemmArgs& a, dim3 grid, hipStream_t s) {
     if (a.rq_fast)
@@ -578,10 +700,10 @@ static bool try_ws(const GemmArgs& a, hipStream_t s) {
 
 void launch_gemm(const GemmArgs& a, int epi, hipStream_t s) {
     switch (epi) {
-        case EPI_RAW: if (try_ws<EPI_RAW>(a, s)) return; break;
-        case EPI_REQ: if (try_ws<EPI_REQ>(a, s)) return; break;
-        case EPI_QKV: if (try_ws<EPI_QKV>(a, s)) return; break;
-        default: if (try_ws<EPI_REGLU>(a, s)) return; break;
+        case EPI_RAW: if (try_skinny<EPI_RAW>(a, s) || try_ws<EPI_RAW>(a, s)) return; break;
+        case EPI_REQ: if (try_skinny<EPI_REQ>(a, s) || try_ws<EPI_REQ>(a, s)) return; break;
+        case EPI_QKV: if (try_skinny<EPI_QKV>(a, s) || try_ws<EPI_QKV>(a, s)) return; break;
+        default: if (try_skinny<EPI_REGLU>(a, s) || try_ws<EPI_REGLU>(a, s)) return; break;
     }
     const int ntm = (a.M + BM - 1) / BM, ntn = (a.N + BN - 1) / BN;
     dim3 grid((unsigned)(((ntm + NXCD - 1) / NXCD) * NXCD * ntn));
@@ -891,7 +1013,8 @@ __global__ __launch_bounds__(64 * NW) void k_gemm_rn16(RowGemmArgs a) {
 }
 
 // ---------------------------------------------------------------------------
-// Split-K row GEMM for few rows (decode with a few thousand streams): the
+// Split-K row GEMM for a few thousand rows whose K is too long for the 16-row
+// kernel (d_ff > 4096), and for fewer where the few-row GEMM is off: the
 // workgroup (row block, K slice) multiplies its K steps and stores the int32
 // partial sums; k_rn_splitk_epi then sums the slices and runs the row GEMM's
 // epilogue per row.  part: [splits][M][d].
@@ -1001,6 +1124,16 @@ static void launch_rn(const RowGemmArgs& a, hipStream_t s) {
 // d = 64 h columns over NW waves of CT 16-wide tiles: 8 waves where h is even
 // (few accumulators per wave, many waves to hide the W stream's latency)
 void launch_gemm_rn(const RowGemmArgs& a, hipStream_t s) {
+    if (a.y8 && !a.tiled && a.M > 0 && a.M <= a.skinny_rows) {
+        // few rows: the product over the whole chip, then the norms a wavefront per row
+        GemmArgs g{};
+        g.A = a.A; g.Wf = a.Wf; g.M = a.M; g.N = a.d; g.K = a.K; g.out8 = a.y8; g.ldo = a.d;
+        g.mult = a.mult; g.shift = a.shift; g.rq_scale = a.rq_scale; g.rq_fast = a.rq_fast; g.skinny_rows = a.skinny_rows;
+        if (try_skinny<EPI_REQ>(g, s)) {
+            launch_rn_rows(a, s);
+            return;
+        }
+    }
     if (!a.tiled && a.d == 384 && a.M > 0 && (long long)a.M * a.K < (1ll << 40) && !use_rn16(a)) {
         if (a.K == 384) { launch_rn_ws<8, 3, 6>(a, s); return; }
         if (a.K == 512) { launch_rn_ws<8, 3, 8>(a, s); return; }

@@ -207,6 +207,82 @@ void launch_rn_splitk_epi(const RowGemmArgs& a, const int32_t* part, int splits,
 }
 
 // ---------------------------------------------------------------------------
+// The same from the requantized projection (the few-row GEMM's output), one
+// wavefront per row: every load is requested before the first reduction.
+// ---------------------------------------------------------------------------
+template <int NG>  // 4-element groups per lane: d <= 256 NG
+__global__ __launch_bounds__(64) void k_rn_rows(RowGemmArgs a) {
+    const int row = blockIdx.x, lane = threadIdx.x;
+    const int d = a.d, ng = d >> 2;
+    const int8_t* erow = a.x_in ? nullptr : a.embed + (size_t)a.tok[row] * d;
+    unsigned yw[NG], w1w[NG], w2w[NG];
+    uint2 xw[NG];
+#pragma unroll
+    for (int j = 0; j < NG; j++) {
+        const int g = min(lane + 64 * j, ng - 1);
+        yw[j] = *(const unsigned*)(a.y8 + (size_t)row * d + 4 * g);
+        w1w[j] = *(const unsigned*)(a.w1 + 4 * g);
+        w2w[j] = *(const unsigned*)(a.w2 + 4 * g);
+        xw[j] = a.x_in ? *(const uint2*)(a.x_in + (size_t)row * d + 4 * g) : make_uint2(*(const unsigned*)(erow + 4 * g), 0u);
+    }
+    auto inv_rms = [&](unsigned ss) {
+        ss = wave_sum_u(ss);
+        return (double)inv_rms_q15_fast((int)(ss / (unsigned)d) + 1) * (1.0 / 32768.0);  // eps_scaled = 1 (rmsnorm.rs:80-83)
+    };
+    unsigned ss = 0;
+#pragma unroll
+    for (int j = 0; j < NG; j++) {
+        int y[4];
+        unpack4(yw[j], y);
+#pragma unroll
+        for (int k = 0; k < 4; k++) ss += lane + 64 * j < ng ? (unsigned)__mul24(y[k], y[k]) : 0u;
+    }
+    const double inv1 = inv_rms(ss);
+    int xc[NG][4];
+    ss = 0;
+#pragma unroll
+    for (int j = 0; j < NG; j++) {
+        const int g = lane + 64 * j;
+        int y[4], w1[4], xo[4];
+        unpack4(yw[j], y);
+        unpack4(w1w[j], w1);
+        if (a.x_in) {
+            xo[0] = (int16_t)(xw[j].x & 0xFFFFu); xo[1] = (int16_t)(xw[j].x >> 16);
+            xo[2] = (int16_t)(xw[j].y & 0xFFFFu); xo[3] = (int16_t)(xw[j].y >> 16);
+        } else {
+            unpack4(xw[j].x, xo);
+        }
+        int nv[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            nv[k] = xo[k] + rms_el(y[k], w1[k], inv1);
+            xc[j][k] = clamp127(nv[k]);
+            ss += g < ng ? (unsigned)__mul24(xc[j][k], xc[j][k]) : 0u;
+        }
+        if (a.x_out && g < ng)
+            *(uint2*)(a.x_out + (size_t)row * d + 4 * g) = make_uint2(((unsigned)nv[0] & 0xFFFFu) | ((unsigned)nv[1] << 16),
+                                                                    ((unsigned)nv[2] & 0xFFFFu) | ((unsigned)nv[3] << 16));
+    }
+    const double inv2 = inv_rms(ss);
+#pragma unroll
+    for (int j = 0; j < NG; j++) {
+        const int g = lane + 64 * j;
+        int w2[4];
+        unpack4(w2w[j], w2);
+        if (g < ng)
+            *(unsigned*)(a.xn + (size_t)row * d + 4 * g) =
+                pack4i(rms_el(xc[j][0], w2[0], inv2), rms_el(xc[j][1], w2[1], inv2), rms_el(xc[j][2], w2[2], inv2),
+                       rms_el(xc[j][3], w2[3], inv2));
+    }
+}
+
+void launch_rn_rows(const RowGemmArgs& a, hipStream_t s) {
+    const dim3 grid((unsigned)a.M);
+    if (a.d <= 512) hipLaunchKernelGGL(k_rn_rows<2>, grid, dim3(64), 0, s, a);
+    else hipLaunchKernelGGL(k_rn_rows<4>, grid, dim3(64), 0, s, a);
+}
+
+// ---------------------------------------------------------------------------
 // Layer 0's QKV from the per-token table.  One thread per (row, item): items
 // 0 .. 8H-1 are query rotary groups (head i / 8, dims 4 (i % 8) .. +3 paired
 // with +32), the next 8 NG key rotary groups, the last 16 NG value quads.

@@ -112,3 +112,19 @@ def test_decode_attention_rows_key_counts(pair, n):
     chunks = om.compress_many(toks, n, threads=4)
     for s in (1, 2, 3):
         assert np.array_equal(gm.decompress_chunks(chunks[:s], [n] * s), toks[:s * n])
+
+
+@pytest.mark.parametrize("heads,kv,d_ff", [(1, 1, 64), (5, 1, 1600), (6, 2, 128), (14, 7, 832), (16, 4, 3136)])
+def test_few_row_gemms(amd, orc, tmp_path, heads, kv, d_ff):
+    """The few-row GEMMs (and the row norms behind them) at row counts around
+    their 16- and 64-row tiles and past their last one, for K of 1, 5, 6, 13,
+    14, 16, 25 and 49 steps of 64 (all three wave counts, with and without a
+    remainder)."""
+    import test_gpu_parity as parity
+    from czip_amd import synth
+    path = synth.write_random_model(str(tmp_path / "m.czm"), d=64 * heads, n_layers=2, n_heads=heads, n_kv=kv,
+                                    d_ff=d_ff, vocab=1088, ctx=600, seed=300 + heads)
+    gm = amd.Model(amd.ModelWeights(path, amd.KV_GQA))
+    om = orc.Model.from_file(path, amd.KV_GQA)
+    for lens in ([1], [16], [17], [63], [32, 32], [13, 5, 13, 13, 13], [129], [256], [257], [512], [513]):
+        parity._check_logits(gm, om, max(lens), lens, 7 + len(lens), 1088)
