@@ -212,6 +212,7 @@ struct czip_ctx {
     int64_t decode_streams = 0;   // CZIP_DECODE_STREAMS: most streams per decode group (0: no cap)
     long long attn_rows = ATTN_ROWS_MAX;  // CZIP_ATTN_ROWS
     int skinny_rows = SKINNY_ROWS_MAX;    // CZIP_SKINNY_ROWS
+    int dec_fused_max = 0;        // most streams per group decoded by the whole-stream kernel (CZIP_DECODE_FUSED)
     int decode_lanes = 0;         // CZIP_DECODE_LANES: lanes per decode group (0: by group size)
     bool lut0_max = false;        // exp2_lut[0] == 65535: the heads' table step 0 is E(0) (HeadCdfArgs::e0)
     std::vector<Alloc> allocs;
@@ -540,6 +541,25 @@ extern "C" czip_status czip_create(const czip_model_desc* w, int device, czip_ct
     if (const char* e = getenv("CZIP_DECODE_LANES")) {
         const int n = atoi(e);
         if (n >= 1 && n <= DEC_LANES_MAX) c->decode_lanes = n;
+    }
+    {
+        // the whole-stream decode kernel: its shape, fast-path requantization, and a frequency total
+        // for which no interval is empty; not beside a switch that asks for one of the step kernels
+        bool ok = c->rn_fused && c->head_fused && w->n_layers == 1 && w->layers && w->target_total <= (1u << 30) &&
+                  decode_fused_supported(w->d_model, w->d_ff, w->vocab);
+        for (const char* e : {"CZIP_GEMM_TILED", "CZIP_QKV_GEMM", "CZIP_UNFUSED_FFN", "CZIP_FFN_MIN_ROWS", "CZIP_DECODE_LANES",
+                              "CZIP_ATTN_ROWS", "CZIP_SKINNY_ROWS"})
+            ok = ok && getenv(e) == nullptr;
+        if (ok) {
+            const czip_layer_desc& L = w->layers[0];
+            GemmArgs o{}, u{}, dn{};
+            o.K = w->d_model; set_requant(o, L.out_mult, L.out_shift);
+            u.K = w->d_model; set_requant(u, L.up_mult, L.up_shift);
+            dn.K = w->d_ff; set_requant(dn, L.down_mult, L.down_shift);
+            ok = o.rq_fast && u.rq_fast && dn.rq_fast;
+        }
+        c->dec_fused_max = ok ? DECODE_FUSED_MAX_STREAMS : 0;
+        if (const char* e = getenv("CZIP_DECODE_FUSED")) c->dec_fused_max = std::min(c->dec_fused_max, std::max(0, atoi(e)));
     }
     czip_ctx* C = c.get();
 #define UP(dst, src, n) if ((rc = upload(C, &dst, src, n))) return rc;
@@ -1218,6 +1238,26 @@ static czip_status run_decompress(czip_job* j) {
     const size_t layer_kv = (size_t)j->S * c->KH * TP * 64, stream_kv = (size_t)c->KH * TP * 64;
     for (int64_t g0 = 0; g0 < j->nchunks; g0 += j->S) {
         const int S = (int)std::min<int64_t>(j->S, j->nchunks - g0);
+        if (S <= c->dec_fused_max) {
+            const DevLayer& L = c->layers[0];
+            GemmArgs o{}, u{}, dn{};  // requantization scales (the fast path, checked at czip_create)
+            o.K = d; set_requant(o, L.out_mult, L.out_shift);
+            u.K = d; set_requant(u, L.up_mult, L.up_shift);
+            dn.K = c->cfg.d_ff; set_requant(dn, L.down_mult, L.down_shift);
+            FusedDecArgs f{};
+            f.ds = DecStreams{j->d_data, j->d_offs + g0, j->d_blen + g0, j->d_ntok + g0, j->d_tokens, j->d_toff + g0};
+            f.S = S; f.TP = TP; f.KH = c->KH; f.NKV = c->cfg.kv_mode == CZIP_KV_GQA ? c->cfg.n_kv_heads : 1;
+            f.kv_mode = c->cfg.kv_mode; f.G = c->cfg.n_kv_heads; f.qkv_n = L.qkv_n; f.F = c->cfg.d_ff;
+            f.tab = c->qkv_tab; f.embed = c->embed; f.rcos = c->rcos; f.rsin = c->rsin; f.kc = j->kc; f.vc = j->vc;
+            f.score_mult = L.score_mult; f.sink = L.sink; f.etab = c->etab;
+            f.out_wf = L.out_wf; f.up_wf = L.up_wf; f.down_wf = L.down_wf; f.head_wf = c->head_wf;
+            f.o_scale = o.rq_scale; f.up_scale = u.rq_scale; f.dn_scale = dn.rq_scale;
+            f.w_ffn = L.ffn_norm; f.w_post_attn = L.post_attn_norm; f.w_post_ffn = L.post_ffn_norm; f.w_final = c->final_norm;
+            f.lut = c->lut; f.coef = c->cfg.coef_q24; f.total = c->cfg.target_total;
+            Timed t(c, "dec_fused");
+            launch_decode_fused(f, d, L.attn_general, c->stream);
+            continue;
+        }
         const int nl = decode_lanes(c, S);
         for (int ln = 1; ln < nl; ln++) {
             if (c->lane_s[ln - 1]) continue;

@@ -126,7 +126,6 @@ __device__ __forceinline__ void attn_row_tile(const int* q, const v4i (&k)[4], c
         hi[4 * b] = h.x; hi[4 * b + 1] = h.y; hi[4 * b + 2] = h.z; hi[4 * b + 3] = h.w;
         lo[4 * b] = l.x; lo[4 * b + 1] = l.y; lo[4 * b + 2] = l.z; lo[4 * b + 3] = l.w;
     }
-    wave_lds_fence();
     // the segment being summed: sums of hi v, lo v and v over its blocks (a
     // block's keys outside the segment carry w = 0, bytes -128), and the
     // weight sum before it

@@ -372,6 +372,14 @@ __device__ __forceinline__ unsigned long long udiv64_32(unsigned long long a, un
     return q;
 }
 
+// floor(x * range / total) with range = rm1 + 1 <= 2^32 and xt = x / total
+// rounded: the estimate is within one of the quotient, the remainder test exact
+__device__ __forceinline__ unsigned long long coder_div(unsigned x, double xt, unsigned rm1, double range, unsigned total) {
+    const unsigned long long q = (unsigned)fmin(xt * range, 4294967295.0);
+    const long long r = (long long)((unsigned long long)x * rm1 + x - q * total);
+    return q + (r >= (long long)total ? 1ull : 0ull) - (r < 0 ? 1ull : 0ull);
+}
+
 __device__ __forceinline__ int wave_sum_i(int v) {
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
     return v;

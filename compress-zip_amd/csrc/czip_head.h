@@ -36,14 +36,16 @@ struct HeadLdsT {
     double row_y[HBM_ROWS];
 };
 
+__device__ __forceinline__ unsigned head_etab_entry(int t, const uint16_t* lut) {
+    const unsigned ip = (unsigned)t >> 8;
+    const unsigned x = ip >= 16u ? 1u : ((65536u >> ip) * (unsigned)lut[t & 255] + 0x8000u) >> 16;
+    return t == ETAB_N - 1 ? 65535u : (x < 1u ? 1u : (x > 65535u ? 65535u : x));
+}
+
 // The exp table of head_freqs, built once per workgroup.
 template <class Lds>
 __device__ __forceinline__ void head_etab_fill(Lds& L, const uint16_t* lut) {
-    for (int t = threadIdx.x; t < ETAB_N; t += 64 * HNW) {
-        const unsigned ip = (unsigned)t >> 8;
-        const unsigned x = ip >= 16u ? 1u : ((65536u >> ip) * (unsigned)lut[t & 255] + 0x8000u) >> 16;
-        L.etab[t] = t == ETAB_N - 1 ? 65535u : (x < 1u ? 1u : (x > 65535u ? 65535u : x));
-    }
+    for (int t = threadIdx.x; t < ETAB_N; t += 64 * HNW) L.etab[t] = head_etab_entry(t, lut);
 }
 
 // threadIdx.x with a value the compiler cannot follow across loop iterations

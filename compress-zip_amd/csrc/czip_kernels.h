@@ -235,4 +235,29 @@ struct HeadDecArgs {
 };
 void launch_head_dec(const HeadDecArgs& a, DecState st, DecStreams ds, hipStream_t s);
 
+
+// Every step of S streams of a one-layer model in one launch (the fused heads'
+// shapes, all three projections' requantization on the fast path, total <=
+// 2^30): the caches as the step kernels' (vt_off, vl = 2).
+struct FusedDecArgs {
+    DecStreams ds;
+    int S, R;                  // R: streams per workgroup (set by launch_decode_fused)
+    int TP, KH, NKV, kv_mode, G, qkv_n, F;  // NKV: KV heads in the table
+    const int8_t* tab;         // layer 0's Q/K/V per token (QkvTabArgs::tab)
+    const int8_t* embed;
+    const int16_t *rcos, *rsin;
+    int8_t *kc, *vc;
+    const int32_t* score_mult;
+    const int8_t* sink;
+    const uint16_t* etab;      // attention's exp table (attn_etab_host)
+    const int8_t *out_wf, *up_wf, *down_wf, *head_wf;  // fragment-major; up: 32 gate, 32 up rows alternating
+    double o_scale, up_scale, dn_scale;
+    const int8_t *w_ffn, *w_post_attn, *w_post_ffn, *w_final;
+    const uint16_t* lut;
+    unsigned coef, total;
+};
+constexpr int DECODE_FUSED_MAX_STREAMS = 256 * 16;
+bool decode_fused_supported(int d, int F, int V);
+void launch_decode_fused(const FusedDecArgs& a, int d, bool general, hipStream_t s);
+
 }  // namespace czip

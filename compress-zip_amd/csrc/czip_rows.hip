@@ -781,14 +781,6 @@ struct BitOut {
     }
 };
 
-// floor(x * range / total) with range = rm1 + 1 <= 2^32 and xt = x / total
-// rounded: the estimate is within one of the quotient, the remainder test exact
-__device__ __forceinline__ unsigned long long enc_div(unsigned x, double xt, unsigned rm1, double range, unsigned total) {
-    const unsigned long long q = (unsigned)fmin(xt * range, 4294967295.0);
-    const long long r = (long long)((unsigned long long)x * rm1 + x - q * total);
-    return q + (r >= (long long)total ? 1ull : 0ull) - (r < 0 ? 1ull : 0ull);
-}
-
 __global__ __launch_bounds__(64) void k_encode(const uint32_t* __restrict__ lohi, const int32_t* __restrict__ lens,
                                                int nb, int T, unsigned total, uint8_t* __restrict__ out,
                                                long long slot, int32_t* __restrict__ out_lens,
@@ -807,8 +799,8 @@ __global__ __launch_bounds__(64) void k_encode(const uint32_t* __restrict__ lohi
         if (stuck) return;
         const unsigned rm1 = high - low;
         const double range = (double)rm1 + 1.0;
-        const unsigned long long ql = enc_div(cur.x, (double)cur.x * invT, rm1, range, total);
-        const unsigned long long qh = enc_div(cur.y, (double)cur.y * invT, rm1, range, total);
+        const unsigned long long ql = coder_div(cur.x, (double)cur.x * invT, rm1, range, total);
+        const unsigned long long qh = coder_div(cur.y, (double)cur.y * invT, rm1, range, total);
         const unsigned nl = low + (unsigned)ql, nh = low + (unsigned)qh - 1u;
         if (ql < qh) {
             const int k = __clz((int)(nl ^ nh));  // 32 when they are equal

@@ -128,3 +128,54 @@ def test_few_row_gemms(amd, orc, tmp_path, heads, kv, d_ff):
     om = orc.Model.from_file(path, amd.KV_GQA)
     for lens in ([1], [16], [17], [63], [32, 32], [13, 5, 13, 13, 13], [129], [256], [257], [512], [513]):
         parity._check_logits(gm, om, max(lens), lens, 7 + len(lens), 1088)
+
+
+# The whole-stream decode kernel (one-layer models, V = 1024).  Up to 256
+# streams it takes one stream a workgroup, then two, ... sixteen; the streams
+# end at different steps, some before the first.
+FUSED_SHAPES = [  # d, kv heads, d_ff, kv mode, sink, general attention
+    (384, 1, 1024, "rust", False, False), (256, 2, 64, "gqa", True, False), (512, 4, 960, "gqa", False, False),
+    (512, 2, 1024, "rust", True, True), (256, 1, 320, "rust", False, True), (384, 3, 448, "gqa", True, False)]
+
+
+@pytest.mark.parametrize("i", range(len(FUSED_SHAPES)))
+def test_fused_decode_shapes(amd, orc, tmp_path, monkeypatch, i):
+    from test_gpu_parity import _write_model
+    from czip_amd import synth
+    d, n_kv, d_ff, kv, sink, general = FUSED_SHAPES[i]
+    t, meta = synth.random_model_tensors(d=d, n_layers=1, n_heads=d // 64, n_kv=n_kv, d_ff=d_ff, vocab=1024, ctx=256,
+                                         seed=400 + i, sink=sink)
+    if general:  # scores past 2^30 and an exp table whose first entry is not 65535
+        t["layers.0.attn.score_mult"] = np.resize(np.array([1 << 30, -(1 << 30), 1 << 27, -5], np.int32), d // 64)
+        t["lut.exp2"][0] = 65000
+    path = _write_model(str(tmp_path / "f.czm"), t, meta)
+    mode = amd.KV_GQA if kv == "gqa" else amd.KV_RUST_COMPAT
+    om = orc.Model.from_file(path, mode)
+    rng = np.random.default_rng(410 + i)
+    toks = synth.zipf_ids(5 * 200, 1024, seed=420 + i)
+    chunks = om.compress_many(toks, 200, threads=8)
+    gm = amd.Model(amd.ModelWeights(path, mode))
+    gm.set_profiling(True)
+    assert np.array_equal(gm.decompress_chunks(chunks, [200] * 5), toks)
+    assert gm.kernel_stats("dec_fused")[0] == 1  # the kernel under test ran
+    # many short streams of different lengths, some of them empty
+    for S in (257, 700, 4000):
+        lens = rng.integers(0, 6, S)
+        part = [toks[r:r + n] for r, n in zip(rng.integers(0, 900, S), lens)]
+        coded, seen = [], {}
+        for c in part:
+            k = c.tobytes()
+            if k not in seen:
+                seen[k] = om.compress_many(c, max(c.size, 1), threads=1)[0] if c.size else b""
+            coded.append(seen[k])
+        assert np.array_equal(gm.decompress_chunks(coded, lens), np.concatenate(part))
+
+
+def test_fused_decode_truncated_bytes(amd, pair):
+    """Streams cut short read zeros past their end, as the step kernels do."""
+    gm, om = pair
+    toks = np.random.default_rng(9).integers(0, 1024, 300).astype(np.uint32)
+    chunks = om.compress_many(toks, 60, threads=2)
+    for cut in (0, 1, 3, 7, 8, 9, 40):
+        part = [c[:cut] for c in chunks]
+        assert np.array_equal(gm.decompress_chunks(part, [60] * 5), om.decompress_many(part, [60] * 5))
