@@ -40,6 +40,17 @@ constexpr int DEC_VL = 2;
 // while the rows leave SIMDs idle and loses once they queue: 4096 rows 118 ->
 // 64 ms (d512), 12288 rows 16.7 -> 18.3 (v001) and 81 -> 91 ms (d768)
 constexpr long long ATTN_ROWS_MAX = 8192;
+// launches of at most this many rows, and at least one row for every 2500 bytes
+// of a layer's weights (and more than the few-row GEMMs take), run a layer after
+// its attention as one kernel (CZIP_TAIL_ROWS), where those weights fit an
+// XCD's L2: every workgroup streams them all.  Decode, separate kernels -> tail:
+// d512 (3.7 MB a layer) 128 steps of 768 rows 57.5 -> 57.9 ms, 2048 66.2 -> 63.5,
+// 4096 82.0 -> 71.3, 64 steps of 8192 64.5 -> 45.4; v001 (1.5 MB) 128 steps of
+// 8192 14.9 -> 11.7 ms, 20000 26.5 -> 24.5.  Prefill of d512: 1024 rows 0.60 ->
+// 0.63 ms, 8192 1.82 -> 1.62, 32768 3.81 -> 3.93; v001 704 rows 0.134 -> 0.127,
+// 18944 0.511 -> 0.505, 26752 0.277 -> 0.280, 65536 0.82 -> 0.84
+constexpr int64_t TAIL_ROWS_MAX = 20480;
+constexpr size_t TAIL_WEIGHTS_MAX = (size_t)4 << 20, TAIL_WEIGHT_BYTES_PER_ROW = 2500;
 // GEMMs of at most this many rows split K over a workgroup's waves and the
 // columns over the chip (CZIP_SKINNY_ROWS).  Decode of 512 streams: d768 64
 // steps 72 -> 52 ms, d512 128 steps 52 -> 43, v001 256 steps 15.0 -> 14.4; of
@@ -212,6 +223,8 @@ struct czip_ctx {
     int64_t decode_streams = 0;   // CZIP_DECODE_STREAMS: most streams per decode group (0: no cap)
     long long attn_rows = ATTN_ROWS_MAX;  // CZIP_ATTN_ROWS
     int skinny_rows = SKINNY_ROWS_MAX;    // CZIP_SKINNY_ROWS
+    int64_t tail_rows = 0;        // most and least rows of a launch whose layers end in the tail
+    int64_t tail_rows_min = 0;    // kernel (most 0: never)
     int dec_fused_max = 0;        // most streams per group decoded by the whole-stream kernel (CZIP_DECODE_FUSED)
     int decode_lanes = 0;         // CZIP_DECODE_LANES: lanes per decode group (0: by group size)
     bool lut0_max = false;        // exp2_lut[0] == 65535: the heads' table step 0 is E(0) (HeadCdfArgs::e0)
@@ -561,6 +574,24 @@ extern "C" czip_status czip_create(const czip_model_desc* w, int device, czip_ct
         c->dec_fused_max = ok ? DECODE_FUSED_MAX_STREAMS : 0;
         if (const char* e = getenv("CZIP_DECODE_FUSED")) c->dec_fused_max = std::min(c->dec_fused_max, std::max(0, atoi(e)));
     }
+    {
+        // the layer tail: its shapes, fast-path requantization, weights that stay in an L2
+        const size_t qn = w->kv_mode == CZIP_KV_GQA ? d + 2 * G * 64 : d + 128;
+        bool ok = c->rn_fused && w->layers && tail_supported(w->d_model, w->d_ff) && d * (qn + d + 3 * F) <= TAIL_WEIGHTS_MAX;
+        for (const char* e : {"CZIP_GEMM_TILED", "CZIP_UNFUSED_FFN", "CZIP_FFN_MIN_ROWS"}) ok = ok && getenv(e) == nullptr;
+        for (int l = 0; ok && l < w->n_layers; l++) {
+            const czip_layer_desc& L = w->layers[l];
+            GemmArgs q{}, o{}, u{}, dn{};
+            q.K = w->d_model; set_requant(q, L.qkv_mult, L.qkv_shift);
+            o.K = w->d_model; set_requant(o, L.out_mult, L.out_shift);
+            u.K = w->d_model; set_requant(u, L.up_mult, L.up_shift);
+            dn.K = w->d_ff; set_requant(dn, L.down_mult, L.down_shift);
+            ok = q.rq_fast && o.rq_fast && u.rq_fast && dn.rq_fast;
+        }
+        c->tail_rows = ok ? TAIL_ROWS_MAX : 0;
+        c->tail_rows_min = (int64_t)(d * (qn + d + 3 * F) / TAIL_WEIGHT_BYTES_PER_ROW);
+        if (const char* e = getenv("CZIP_TAIL_ROWS")) c->tail_rows = ok ? std::max(0ll, atoll(e)) : 0;
+    }
     czip_ctx* C = c.get();
 #define UP(dst, src, n) if ((rc = upload(C, &dst, src, n))) return rc;
     UP(c->embed, w->embed, V * d)
@@ -746,11 +777,31 @@ RowBufs row_bufs(const czip_ctx* c, const czip_job* j, int64_t r0 = 0, int ws_pa
                    j->rn_ws ? j->rn_ws + wb / 4 * (size_t)ws_part : nullptr, wb};
 }
 
-void post_attention(czip_ctx* c, const RowBufs& r, int l, int M, hipStream_t s, bool beside_lanes = false) {
+// next_qkv: the next layer's Q/K/V projection of a decode step (or nullptr);
+// returns whether it was done here.
+bool post_attention(czip_ctx* c, const RowBufs& r, int l, int M, hipStream_t s, bool beside_lanes = false,
+                    const GemmArgs* next_qkv = nullptr) {
     const int d = c->cfg.d_model, F = c->cfg.d_ff;
     const DevLayer& L = c->layers[(size_t)l];
     const bool last = l + 1 == c->cfg.n_layers;
     const int8_t* next = last ? c->final_norm : c->layers[(size_t)l + 1].attn_norm;
+    if (M > c->skinny_rows && M >= c->tail_rows_min && M <= c->tail_rows) {
+        GemmArgs o{}, u{}, dn{};  // requantization scales (the fast path, checked at czip_create)
+        o.K = d; set_requant(o, L.out_mult, L.out_shift);
+        u.K = d; set_requant(u, L.up_mult, L.up_shift);
+        dn.K = F; set_requant(dn, L.down_mult, L.down_shift);
+        TailArgs t{};
+        t.attn = r.attn; t.M = M; t.F = F; t.out_wf = L.out_wf; t.up_wf = L.up_wf; t.down_wf = L.down_wf;
+        t.o_scale = o.rq_scale; t.up_scale = u.rq_scale; t.dn_scale = dn.rq_scale;
+        t.w_ffn = L.ffn_norm; t.w_post_attn = L.post_attn_norm; t.w_post_ffn = L.post_ffn_norm; t.w_next = next;
+        t.x_in = l == 0 ? nullptr : r.x; t.tok = r.inp; t.embed = c->embed;
+        t.x_out = last ? nullptr : r.x;
+        if (next_qkv) t.qkv = *next_qkv;
+        t.xn = next_qkv ? nullptr : r.xn;
+        Timed tm(c, "layer_tail");
+        launch_layer_tail(t, d, s);
+        return next_qkv != nullptr;
+    }
     if (c->rn_fused) {
         RowGemmArgs o{};
         o.A = r.attn; o.W = L.out_w; o.Wf = L.out_wf; o.M = M; o.K = d; o.d = d;
@@ -782,7 +833,7 @@ void post_attention(czip_ctx* c, const RowBufs& r, int l, int M, hipStream_t s, 
         f.w1 = L.post_ffn_norm; f.w2 = next; f.x_in = r.x; f.x_out = last ? nullptr : r.x; f.xn_out = r.xn;
         Timed t(c, "ffn");
         launch_ffn(f, s);
-        return;
+        return false;
     }
     GemmArgs u{};
     u.A = r.xn; u.W = L.up_w; u.Wf = L.up_wf; u.M = M; u.N = 2 * F; u.K = d; u.out8 = r.r8; u.ldo = F;
@@ -802,6 +853,20 @@ void post_attention(czip_ctx* c, const RowBufs& r, int l, int M, hipStream_t s, 
         { Timed t(c, "gemm_down"); gemm(c, dn, EPI_REQ, s); }
         { Timed t(c, "row_norm"); launch_resid_norm(r.x, r.y8, L.post_ffn_norm, next, M, d, r.xn, s); }
     }
+    return false;
+}
+
+// Layer l's Q/K/V projection of a decode step: M streams at position p, their
+// caches in 4-key blocks
+GemmArgs decode_qkv_args(const czip_ctx* c, int l, const RowBufs& r, int M, int TP, int p, int8_t* kc, int8_t* vc) {
+    const DevLayer& L = c->layers[(size_t)l];
+    const int d = c->cfg.d_model;
+    GemmArgs g{};
+    g.A = r.xn; g.W = L.qkv_w; g.Wf = L.qkv_wf; g.M = M; g.N = L.qkv_n; g.K = d;
+    g.out8 = r.q8; g.ldo = d; set_requant(g, L.qkv_mult, L.qkv_shift);
+    g.d = d; g.T = TP; g.TP = TP; g.pos = p; g.vl = DEC_VL; g.kv_mode = c->cfg.kv_mode; g.G = c->cfg.n_kv_heads;
+    g.KH = c->KH; g.kc = kc; g.vc = vc; g.rcos = c->rcos; g.rsin = c->rsin;
+    return g;
 }
 
 // Layer 0's QKV: from the per-token table (RoPE + scatter), or the GEMM over
@@ -1316,18 +1381,18 @@ static czip_status run_decompress(czip_job* j) {
                     Timed t(c, "embed_norm");
                     launch_embed_norm(Ln.r.inp, c->embed, c->layers[0].attn_norm, M, d, Ln.r.x, Ln.r.xn, s);
                 }
+                bool have_qkv = false;
                 for (int l = 0; l < c->cfg.n_layers; l++) {
                     const DevLayer& L = c->layers[(size_t)l];
-                    int8_t* kc = j->kc + (size_t)l * layer_kv + (size_t)Ln.r0 * stream_kv;
-                    int8_t* vc = j->vc + (size_t)l * layer_kv + (size_t)Ln.r0 * stream_kv;
-                    GemmArgs g{};
-                    g.A = Ln.r.xn; g.W = L.qkv_w; g.Wf = L.qkv_wf; g.M = M; g.N = L.qkv_n; g.K = d;
-                    g.out8 = Ln.r.q8; g.ldo = d; set_requant(g, L.qkv_mult, L.qkv_shift);
-                    g.d = d; g.T = TP; g.TP = TP; g.pos = p; g.vl = DEC_VL; g.kv_mode = c->cfg.kv_mode; g.G = c->cfg.n_kv_heads;
-                    g.KH = c->KH; g.kc = kc; g.vc = vc; g.rcos = c->rcos; g.rsin = c->rsin;
+                    auto qkv_args = [&](int ly) {
+                        return decode_qkv_args(c, ly, Ln.r, M, TP, p, j->kc + (size_t)ly * layer_kv + (size_t)Ln.r0 * stream_kv,
+                                               j->vc + (size_t)ly * layer_kv + (size_t)Ln.r0 * stream_kv);
+                    };
+                    GemmArgs g = qkv_args(l);
+                    int8_t *kc = g.kc, *vc = g.vc;
                     if (l == 0) {
                         layer0_qkv(c, g, Ln.r.inp, s);
-                    } else {
+                    } else if (!have_qkv) {
                         Timed t(c, "gemm_qkv");
                         gemm(c, g, EPI_QKV, s);
                     }
@@ -1337,7 +1402,9 @@ static czip_status run_decompress(czip_job* j) {
                     a.G = c->cfg.n_kv_heads; a.KH = c->KH; a.kv_mode = c->cfg.kv_mode; a.coef = 378194u;
                     a.general = L.attn_general; a.row_max = c->attn_rows;
                     { Timed t(c, "attn_decode"); launch_attn_decode(a, M, p, s); }
-                    post_attention(c, Ln.r, l, M, s, nl > 1);
+                    GemmArgs nq{};
+                    if (l + 1 < c->cfg.n_layers) nq = qkv_args(l + 1);
+                    have_qkv = post_attention(c, Ln.r, l, M, s, nl > 1, l + 1 < c->cfg.n_layers ? &nq : nullptr);
                 }
                 if (c->head_fused) {
                     HeadDecArgs h{};
@@ -1490,18 +1557,18 @@ extern "C" czip_status czip_decode_step(czip_ctx* c, const uint32_t* tok_in, con
     const int TP = pad64(j->T);
     const size_t layer_kv = (size_t)S * c->KH * TP * 64;
     if (!c->rn_fused) { Timed t(c, "embed_norm"); launch_embed_norm(j->inp, c->embed, c->layers[0].attn_norm, S, d, j->x, j->xn, s); }
+    const RowBufs rows = row_bufs(c, j);
+    bool have_qkv = false;
     for (int l = 0; l < c->cfg.n_layers; l++) {
         const DevLayer& L = c->layers[(size_t)l];
-        int8_t* kc = j->kc + (size_t)l * layer_kv;
-        int8_t* vc = j->vc + (size_t)l * layer_kv;
-        GemmArgs g{};
-        g.A = j->xn; g.W = L.qkv_w; g.Wf = L.qkv_wf; g.M = S; g.N = L.qkv_n; g.K = d;
-        g.out8 = j->q8; g.ldo = d; set_requant(g, L.qkv_mult, L.qkv_shift);
-        g.d = d; g.T = TP; g.TP = TP; g.pos = p; g.vl = DEC_VL; g.kv_mode = c->cfg.kv_mode; g.G = c->cfg.n_kv_heads;
-        g.KH = c->KH; g.kc = kc; g.vc = vc; g.rcos = c->rcos; g.rsin = c->rsin;
+        auto qkv_args = [&](int ly) {
+            return decode_qkv_args(c, ly, rows, S, TP, p, j->kc + (size_t)ly * layer_kv, j->vc + (size_t)ly * layer_kv);
+        };
+        GemmArgs g = qkv_args(l);
+        int8_t *kc = g.kc, *vc = g.vc;
         if (l == 0) {
             layer0_qkv(c, g, j->inp, s);
-        } else {
+        } else if (!have_qkv) {
             Timed t(c, "gemm_qkv");
             gemm(c, g, EPI_QKV, s);
         }
@@ -1511,7 +1578,9 @@ extern "C" czip_status czip_decode_step(czip_ctx* c, const uint32_t* tok_in, con
         a.KH = c->KH; a.kv_mode = c->cfg.kv_mode; a.coef = 378194u;  // ATTN_COEF_Q24 (attention.rs:17-19)
         a.general = L.attn_general; a.row_max = c->attn_rows;
         { Timed t(c, "attn_decode"); launch_attn_decode(a, S, p, s); }
-        post_attention(c, row_bufs(c, j), l, S, s);
+        GemmArgs nq{};
+        if (l + 1 < c->cfg.n_layers) nq = qkv_args(l + 1);
+        have_qkv = post_attention(c, rows, l, S, s, false, l + 1 < c->cfg.n_layers ? &nq : nullptr);
     }
     {
         GemmArgs hd{};

@@ -38,27 +38,8 @@ constexpr int FMAXF = 1024;   // widest feed-forward
 constexpr int FV = 1024;      // vocabulary
 constexpr int FPAD = 16;      // row padding (words) of the int32 rows in LDS: 16 rows of 16-byte pieces in four passes
 
-// waits for and orders LDS only: loads of weights stay in flight across it
-__device__ __forceinline__ void lds_barrier() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
 __device__ __forceinline__ unsigned wave_total(unsigned x) {
     return (unsigned)__builtin_amdgcn_readlane((int)wave_scan(x, 0u, [](unsigned a, unsigned b) { return a + b; }), 63);
-}
-
-// fragment-major weights as a buffer: the lane's offset in a vector register,
-// the 1 KB piece (uniform) in a scalar one
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t weights_rsrc(const int8_t* Wf, int bytes) {
-    return __builtin_amdgcn_make_buffer_rsrc((void*)Wf, (short)0, bytes, BUF_DWORD3);
-}
-// N operands (1 KB each) from piece `pc` on
-template <int N>
-__device__ __forceinline__ void load_ops(v4i (&w)[N], __amdgpu_buffer_rsrc_t r, int pc, int lane) {
-#pragma unroll
-    for (int i = 0; i < N; i++) w[i] = __builtin_amdgcn_raw_buffer_load_b128(r, lane * 16, (pc + i) * 1024, 0);
 }
 
 // A stream's arithmetic decoder (arith_coder.rs:139-264), uniform over its

@@ -48,13 +48,6 @@ __device__ __forceinline__ void head_etab_fill(Lds& L, const uint16_t* lut) {
     for (int t = threadIdx.x; t < ETAB_N; t += 64 * HNW) L.etab[t] = head_etab_entry(t, lut);
 }
 
-// threadIdx.x with a value the compiler cannot follow across loop iterations
-__device__ __forceinline__ int opaque_tid() {
-    int t = (int)threadIdx.x;
-    asm volatile("" : "+v"(t));
-    return t;
-}
-
 // Requests the 64 x K block of A at row m0 into As by LDS DMA (no registers
 // held; rows past M read as 0): each wave instruction fills 1 KB, the 16 rows
 // 16 (q % 4) .. +16 of K step q / 4, lane l writing the 16 bytes at l * 16,

@@ -260,4 +260,25 @@ constexpr int DECODE_FUSED_MAX_STREAMS = 256 * 16;
 bool decode_fused_supported(int d, int F, int V);
 void launch_decode_fused(const FusedDecArgs& a, int d, bool general, hipStream_t s);
 
+
+// A layer's work after its attention in one launch, all requantizations on the
+// fast path: output projection + norms + residual, up + ReGLU, down + norms +
+// residual and, where qkv.Wf is set, the next layer's Q/K/V (EPI_QKV; its A is
+// not read).
+struct TailArgs {
+    const int8_t* attn;        // [M, d]
+    int M, F;
+    const int8_t *out_wf, *up_wf, *down_wf;  // fragment-major; up: 32 gate, 32 up rows alternating
+    double o_scale, up_scale, dn_scale;
+    const int8_t *w_ffn, *w_post_attn, *w_post_ffn, *w_next;
+    const int16_t* x_in;       // [M, d]; nullptr: the embedding rows of tok
+    const uint32_t* tok;
+    const int8_t* embed;
+    int16_t* x_out;            // [M, d] or nullptr
+    int8_t* xn;                // [M, d] normalized rows, or nullptr
+    GemmArgs qkv;
+};
+bool tail_supported(int d, int F);
+void launch_layer_tail(const TailArgs& a, int d, hipStream_t s);
+
 }  // namespace czip

@@ -21,7 +21,7 @@ CEILING_SOURCE = "czip_ceiling.hip"
 CEILING_LIB_PATH = os.path.join(ROOT, "libczip_ceiling.so")
 
 SOURCES = ["czip_rows.hip", "czip_gemm.hip", "czip_head.hip", "czip_attention.hip", "czip_decode.hip",
-           "czip_decode_fused.hip", "czip_ffn.hip",
+           "czip_decode_fused.hip", "czip_ffn.hip", "czip_tail.hip",
            "czip_api.cpp",
            "czm_loader.cpp", "czip_tokenizer.cpp", "czip_container.cpp"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")

@@ -179,3 +179,41 @@ def test_fused_decode_truncated_bytes(amd, pair):
     for cut in (0, 1, 3, 7, 8, 9, 40):
         part = [c[:cut] for c in chunks]
         assert np.array_equal(gm.decompress_chunks(part, [60] * 5), om.decompress_many(part, [60] * 5))
+
+
+@pytest.mark.parametrize("d,kv,d_ff,mode", [(256, 2, 64, "gqa"), (384, 1, 1024, "rust"), (512, 2, 2048, "gqa"), (512, 1, 704, "rust")])
+def test_layer_tail(amd, orc, tmp_path, monkeypatch, d, kv, d_ff, mode):
+    """A layer after its attention as one kernel: 16 rows a workgroup up to
+    4096 rows, then 32, with partial last workgroups; prefill (logits) and
+    decode steps (where it also projects the next layer's Q/K/V)."""
+    from czip_amd import synth
+    path = synth.write_random_model(str(tmp_path / "t.czm"), d=d, n_layers=2, n_heads=d // 64, n_kv=kv, d_ff=d_ff,
+                                    vocab=1024, ctx=64, seed=500 + d_ff)
+    m = amd.KV_GQA if mode == "gqa" else amd.KV_RUST_COMPAT
+    monkeypatch.setenv("CZIP_SKINNY_ROWS", "0")  # also below the few-row GEMMs' limit
+    monkeypatch.setenv("CZIP_TAIL_ROWS", "100000")
+    gm = amd.Model(amd.ModelWeights(path, m))
+    om = orc.Model.from_file(path, m)
+    gm.set_profiling(True)
+    rng = np.random.default_rng(d + d_ff)
+    least = d * ((d + 128 * (kv if mode == "gqa" else 1)) + d + 3 * d_ff) // 2500  # fewest rows that take it
+    for rows in (least + 1, 1537, 4096, 4097, 4131):
+        toks = rng.integers(0, 1024, 6 * rows).astype(np.uint32)  # chunks of 6: one row a stream when decoded
+        seen = gm.kernel_stats("layer_tail")[0]
+        chunks = gm.compress_chunks(toks[:rows], 6)
+        assert gm.kernel_stats("layer_tail")[0] > seen
+        assert chunks == om.compress_many(toks[:rows], 6, threads=8)
+        coded = gm.compress_chunks(toks, 6)
+        some = sorted({0, 15, 16, rows // 2, rows - 1})
+        assert [coded[i] for i in some] == om.compress_many(np.concatenate([toks[6 * i:6 * i + 6] for i in some]), 6, threads=8)
+        seen = gm.kernel_stats("layer_tail")[0]
+        assert np.array_equal(gm.decompress_chunks(coded, [6] * rows), toks)
+        assert gm.kernel_stats("layer_tail")[0] > seen
+
+
+def test_row_gemm_16_without_tail(amd, shipped, monkeypatch):
+    """The 16-row row GEMM behind the tail (shapes whose weights outgrow an L2 take it)."""
+    import test_gpu_parity as parity
+    monkeypatch.setenv("CZIP_TAIL_ROWS", "0")
+    gm = amd.Model(amd.ModelWeights(MODEL_PATH))
+    parity.test_small_launch_row_gemm(gm, shipped, 4, 512)
