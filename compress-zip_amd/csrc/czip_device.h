@@ -264,19 +264,23 @@ __device__ __forceinline__ int requant(int v, int mult, int shift) {
 
 // rmsnorm.rs:14-30: clamp(udiv_rne(2^23, isqrt32(mean_sq << 16)), 1, 32768)
 // (primitives.rs:80-97, 192-213) for mean_sq in [1, 2^16): the integer square
-// root by f64 sqrt with an exact correction, the round-half-even quotient by
-// an f64 estimate with an exact remainder test (2^23 / s, s in [256, 2^16)).
-// Checked against the reference algorithm on every mean_sq < 2^16.
+// root and the round-half-even quotient from f32 estimates, each within one of
+// the integer (the operand has 16 significant bits; root < 2^16 and quotient
+// <= 2^15 against relative errors of a few 2^-24) and corrected by its exact
+// remainder.  Checked against the reference algorithm on every mean_sq < 2^16
+// with both estimates off by up to four units in their last place.  A row norm
+// is a serial step of every projection, in f64 (sqrt, division and 64-bit
+// corrections) a several times longer one: layer tail of 19 thousand rows 71.5 ->
+// 68.4 us, whole-stream decode of 115 streams 12.22 -> 12.02 ms.
 __device__ __forceinline__ int inv_rms_q15_fast(int mean_sq) {
     const unsigned x = (unsigned)(mean_sq > 0 ? mean_sq : 1) << 16;
-    unsigned long long r = (unsigned long long)__builtin_sqrt((double)x);
-    if (r * r > x) r--;
-    if ((r + 1) * (r + 1) <= x) r++;
-    const unsigned d = (unsigned)r;
-    unsigned q = (unsigned)(8388608.0 / (double)d);
+    unsigned d = (unsigned)__builtin_amdgcn_sqrtf((float)x);
+    const int e = (int)(x - d * d);
+    d = e < 0 ? d - 1 : (e > (int)(2 * d) ? d + 1 : d);
+    unsigned q = (unsigned)(8388608.0f * __builtin_amdgcn_rcpf((float)d));
     int rem = (int)(8388608u - q * d);
     if (rem < 0) { q--; rem += (int)d; }
-    if (rem >= (int)d) { q++; rem -= (int)d; }
+    else if (rem >= (int)d) { q++; rem -= (int)d; }
     const unsigned tr = (unsigned)rem << 1;
     const unsigned inv = tr > d ? q + 1 : (tr == d ? q + (q & 1u) : q);
     return (int)(inv < 1u ? 1u : (inv > 32768u ? 32768u : inv));
