@@ -23,8 +23,7 @@ namespace czip {
 // or 4 four-wave workgroups per CU (15 or 16 waves at 128 VGPRs).  For rows
 // of one head, three waves per workgroup measured fastest on the 512-token
 // text chunks: 189 ms per compress step against 206 with two, 210 with four,
-// 237 with one and 242-248 with five, six or eight; the order in which a
-// chunk's row blocks are dispatched made no difference.
+// 237 with one and 242-248 with five, six or eight.
 // ---------------------------------------------------------------------------
 
 // NWV wavefronts per workgroup; HWG: the waves take the same 16 rows of NWV
@@ -39,15 +38,27 @@ __global__ __launch_bounds__(64 * NWV, 4) void k_attention(AttnArgs a) {
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int row = lane & 15, grp = lane >> 4;
     // 1-D grid, XCD-aware: workgroups go round-robin over the 8 XCDs; XCD x
-    // takes chunks x, x + 8, ..., all (query block, head) pairs of a chunk in a
+    // takes chunks x, x + 8, ..., all (query block, heads) pairs of a chunk in a
     // row, so a chunk's K/V tiles are fetched into one L2 only.
     const int nq = (a.T + QR - 1) / QR;
     const int per_chunk = nq * (HWG ? a.H / NWV : a.H);
+    // The chunks past the last multiple of eight are shared out over all XCDs
+    // by workgroup, and a chunk's last rows, which see the most keys, go first,
+    // all heads of a row block next to each other: few chunks otherwise leave
+    // XCDs idle behind the one with a chunk more.  49 chunks of 4096 tokens
+    // (d768) 65.6 -> 59.7 ms, 418 of 64 (v001) 64 -> 58 us, 37 of 512 95 -> 91
+    // us, 38 thousand of 512 66.6 -> 65.7 ms.
     const int xcd = (int)(blockIdx.x % 8u), jx = (int)(blockIdx.x / 8u);
-    const int b = (jx / per_chunk) * 8 + xcd;
-    if (b >= a.B) return;
-    const int q0 = ((jx % per_chunk) % nq) * QR;
-    const int h = HWG ? ((jx % per_chunk) / nq) * NWV + wave : (jx % per_chunk) / nq;
+    int b = (jx / per_chunk) * 8 + xcd, w = jx % per_chunk;
+    if ((jx / per_chunk) * 8 + 8 > a.B) {
+        const int f = (jx - (a.B / 8) * per_chunk) * 8 + xcd;
+        b = a.B / 8 * 8 + f / per_chunk;
+        w = f % per_chunk;
+        if (b >= a.B) return;
+    }
+    const int nhg = HWG ? a.H / NWV : a.H;
+    const int q0 = (nq - 1 - w / nhg) * QR;
+    const int h = HWG ? (w % nhg) * NWV + wave : w % nhg;
     const int T = a.T, len = a.lens[b];
     if (q0 >= len) return;
     for (int i = tid; i < ETB_PAD / 8; i += 64 * NWV) ((uint4*)etb)[i] = ((const uint4*)a.etab)[i];
@@ -145,7 +156,7 @@ template <bool GEN, int NWV, bool HWG>
 static void launch_attention_t(const AttnArgs& g, int B, hipStream_t s) {
     constexpr int QR = HWG ? 16 : 16 * NWV;
     const int nq = (g.T + QR - 1) / QR;
-    dim3 grid((unsigned)(((B + 7) / 8) * 8 * nq * (HWG ? g.H / NWV : g.H)));
+    dim3 grid((unsigned)(((long long)B * nq * (HWG ? g.H / NWV : g.H) + 7) / 8 * 8));
     hipLaunchKernelGGL((k_attention<GEN, NWV, HWG>), grid, dim3(64 * NWV), 0, s, g);
 }
 
