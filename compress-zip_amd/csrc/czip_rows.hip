@@ -733,9 +733,10 @@ void launch_pack_chunks(const uint8_t* src, int64_t slot, const int32_t* lens, c
 // bits different, so no settled bit follows.  The divisions are one f64
 // estimate each (x / total formed ahead of the chain) with a branch-free
 // integer correction, the intervals are loaded ENC_AHEAD tokens ahead, and the
-// bits leave as whole words.  Measured against a loop per shift, pending bit
-// and correction: 11 chunks of 64 tokens 179 -> 34 us, 49 of 4096 16.3 -> 2.0
-// ms (4.0 -> 0.49 us a token), 38 thousand of 512 2.19 -> 0.29 ms.
+// bits leave as whole words, a symbol's settled and pending bits in one append.
+// Measured against a loop per shift, pending bit and correction: 11 chunks of
+// 64 tokens 179 -> 27 us, 49 of 4096 16.3 -> 1.4 ms (4.0 -> 0.34 us a token), 38
+// thousand of 512 2.19 -> 0.22 ms.
 // ---------------------------------------------------------------------------
 constexpr int ENC_AHEAD = 8;  // intervals in flight per thread
 
@@ -805,12 +806,18 @@ __global__ __launch_bounds__(64) void k_encode(const uint32_t* __restrict__ lohi
         if (ql < qh) {
             const int k = __clz((int)(nl ^ nh));  // 32 when they are equal
             if (k > 0) {
+                // the first settled bit b, the pending bits (each 1 - b), the k - 1
+                // bits behind: b and n pending ones are the number 2^n - 1 + b
                 const unsigned b = nl >> 31;
-                o.bit(b);
-                if (underflow) o.run(b ^ 1u, underflow);
+                if (underflow + (unsigned)k <= 32u) {
+                    const unsigned head = ((1u << underflow) - 1u + b) << (k - 1);
+                    o.bits(head | ((nl >> (32 - k)) & ((1u << (k - 1)) - 1u)), (int)underflow + k);
+                } else {
+                    o.bit(b);
+                    o.run(b ^ 1u, underflow);
+                    if (k > 1) o.bits(nl >> (32 - k), k - 1);
+                }
                 underflow = 0;
-                // the k - 1 bits behind the first
-                if (k > 1) o.bits(nl >> (32 - k), k - 1);
             }
             const unsigned l1 = k < 32 ? nl << k : 0u;
             const unsigned h1 = k < 32 ? (nh << k) | ((1u << k) - 1u) : 0xFFFFFFFFu;
