@@ -56,6 +56,9 @@ constexpr size_t TAIL_WEIGHTS_MAX = (size_t)4 << 20, TAIL_WEIGHT_BYTES_PER_ROW =
 // steps 72 -> 52 ms, d512 128 steps 52 -> 43, v001 256 steps 15.0 -> 14.4; of
 // 1024 streams d768 76 -> 73, d512 59.2 -> 59.6 ms
 constexpr int SKINNY_ROWS_MAX = 512;
+// GEMMs of at least this many rows, where no W-stationary kernel takes them,
+// run 128 x 256 tiles with the weights straight from L2 (CZIP_WIDE_ROWS)
+constexpr int WIDE_ROWS_MIN = 4096;
 
 struct DevLayer {
     int8_t *attn_norm = nullptr, *post_attn_norm = nullptr, *ffn_norm = nullptr, *post_ffn_norm = nullptr;
@@ -223,6 +226,7 @@ struct czip_ctx {
     int64_t decode_streams = 0;   // CZIP_DECODE_STREAMS: most streams per decode group (0: no cap)
     long long attn_rows = ATTN_ROWS_MAX;  // CZIP_ATTN_ROWS
     int skinny_rows = SKINNY_ROWS_MAX;    // CZIP_SKINNY_ROWS
+    int wide_rows = WIDE_ROWS_MIN;        // CZIP_WIDE_ROWS
     int64_t tail_rows = 0;        // most and least rows of a launch whose layers end in the tail
     int64_t tail_rows_min = 0;    // kernel (most 0: never)
     int dec_fused_max = 0;        // most streams per group decoded by the whole-stream kernel (CZIP_DECODE_FUSED)
@@ -414,11 +418,13 @@ void resolve_events(czip_ctx* c) {
 void gemm(const czip_ctx* c, GemmArgs g, int epi, hipStream_t s) {
     g.tiled = c->gemm_tiled ? 1 : 0;
     g.skinny_rows = c->skinny_rows;
+    g.wide_rows = c->wide_rows;
     launch_gemm(g, epi, s);
 }
 void gemm_rn(const czip_ctx* c, RowGemmArgs a, hipStream_t s) {
     a.tiled = c->gemm_tiled ? 1 : 0;
     a.skinny_rows = c->skinny_rows;
+    a.wide_rows = c->wide_rows;
     launch_gemm_rn(a, s);
 }
 
@@ -550,6 +556,7 @@ extern "C" czip_status czip_create(const czip_model_desc* w, int device, czip_ct
     c->pool.set_cap(c->scratch_gb * 1e9 * POOL_SCRATCH_SHARE);
     if (const char* e = getenv("CZIP_DECODE_STREAMS")) c->decode_streams = std::max(1ll, atoll(e));
     if (const char* e = getenv("CZIP_ATTN_ROWS")) c->attn_rows = std::max(0ll, atoll(e));
+    if (const char* e = getenv("CZIP_WIDE_ROWS")) c->wide_rows = std::max(1, atoi(e));
     if (const char* e = getenv("CZIP_SKINNY_ROWS")) c->skinny_rows = std::max(0, atoi(e));
     if (const char* e = getenv("CZIP_DECODE_LANES")) {
         const int n = atoi(e);

@@ -448,6 +448,147 @@ __global__ __launch_bounds__(256, 2) void k_gemm_ws(GemmArgs a, int ncg) {
 }
 
 // ---------------------------------------------------------------------------
+// Tiled GEMM for many rows and any K: a workgroup of four waves takes 128 rows
+// x 256 columns, each wave all 128 rows of its 64 columns (8 x 4 MFMA tiles in
+// 128 accumulator registers, two workgroups a CU).  A goes through
+// double-buffered LDS, fetched two K steps ahead; W, which no two waves of a
+// workgroup share, comes fragment-major from L2 straight into registers a step
+// ahead.  A K step moves 24 KB from L2 and 40 KB through LDS for 128 MFMAs (a
+// 128 x 128 tile with both operands in LDS: 16 and 48 KB for 64, where LDS is
+// the limit), and only LDS is waited for at its barrier.  Column tiles of
+// WIDE_GROUP row blocks are neighbours, so that an XCD's workgroups share both
+// operands in its L2.  d768, 200 thousand rows, 12 layers, against k_gemm: up +
+// ReGLU 16.4 -> 10.8 ms (1.4 -> 2.1 POP/s), QKV 4.3 -> 3.1, head (V = 8192) 2.7 ->
+// 2.2; 4096 rows: up 0.42 -> 0.35, QKV 0.19 -> 0.22; 2048 rows 0.26 -> 0.29 and
+// 0.16 -> 0.20.  (K = 512: the W-stationary kernel is faster, up 14.9 against 18.4
+// ms at a million rows.)
+// ---------------------------------------------------------------------------
+constexpr int WIDE_BM = 128, WIDE_BN = 256;
+constexpr int WIDE_GROUP = 8;  // row blocks an XCD takes through all columns at a time
+
+template <int EPI, bool FAST>
+__global__ __launch_bounds__(256, 2) void k_gemm_wide(GemmArgs a) {
+    __shared__ __attribute__((aligned(16))) int8_t As[2][WIDE_BM * 64];
+    const int tid = threadIdx.x, lane = tid & 63, lr = lane & 15, c4 = (lane >> 4) * 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int ntn = (a.N + WIDE_BN - 1) / WIDE_BN;
+    const int xcd = (int)(blockIdx.x % NXCD), jx = (int)(blockIdx.x / NXCD);
+    const int grp_i = jx / (WIDE_GROUP * ntn), in_grp = jx - grp_i * WIDE_GROUP * ntn;
+    const int mt = (grp_i * WIDE_GROUP + in_grp % WIDE_GROUP) * NXCD + xcd;
+    const int m0 = mt * WIDE_BM, col_base = (in_grp / WIDE_GROUP) * WIDE_BN + wave * 64;
+    if (m0 >= a.M) return;  // the whole workgroup
+    const bool wlive = col_base < a.N;
+    const int nk = a.K / 64;
+    const __amdgpu_buffer_rsrc_t rA = tile_rsrc(a.A, a.M, a.K, m0);
+    const __amdgpu_buffer_rsrc_t rW = weights_rsrc(a.Wf, a.N * a.K);
+    const int voff = (tid >> 2) * a.K + (tid & 3) * 16, voff2 = voff + 64 * a.K;
+    const int wpc = (col_base >> 4) * nk;  // the wave's first 1 KB piece; column tile t at + t nk
+
+    v4i acc[8][4];
+#pragma unroll
+    for (int i = 0; i < 8; i++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) acc[i][j] = (v4i){0, 0, 0, 0};
+    TileRegs ta[2];
+    v4i w[2][4];
+    auto fetch_w = [&](v4i (&d)[4], int kt) {  // past the last step or column: other weights, or zeros
+#pragma unroll
+        for (int t = 0; t < 4; t++) d[t] = __builtin_amdgcn_raw_buffer_load_b128(rW, lane * 16, (wpc + t * nk + kt) * 1024, 0);
+    };
+    fetch_tile(rA, voff, voff2, 0, ta[0]);
+    fetch_tile(rA, voff, voff2, 64, ta[1]);
+    fetch_w(w[0], 0);
+    store_tile(ta[0], As[0], tid);
+    fetch_tile(rA, voff, voff2, 128, ta[0]);
+    lds_barrier();
+    // step kt (u = kt % 2): A of step kt + 1 from registers to LDS, W of kt + 1
+    // and A of kt + 3 requested, the products; past the last step the loads
+    // read other rows' bytes or zeros that nothing uses
+    auto step = [&](int kt, int u) {
+        v4i af[8];
+#pragma unroll
+        for (int i = 0; i < 8; i++) af[i] = *(const v4i*)(As[u] + lds64(i * 16 + lr, lane >> 4));
+        fetch_w(w[u ^ 1], kt + 1);
+        store_tile(ta[u ^ 1], As[u ^ 1], tid);
+        fetch_tile(rA, voff, voff2, (kt + 3) * 64, ta[u ^ 1]);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+#pragma unroll
+            for (int j = 0; j < 4; j++) acc[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(w[u][j], af[i], acc[i][j], 0, 0, 0);
+        }
+        lds_barrier();
+    };
+    int kt = 0;
+    for (; kt + 1 < nk; kt += 2) {
+        step(kt, 0);
+        step(kt + 1, 1);
+    }
+    if (kt < nk) step(kt, 0);
+    if (!wlive) return;  // no barrier follows
+
+    int role = 0, g = 0;
+    WsOut ro;
+    ro.r0 = m0;
+    {
+        const int ob = min(a.M - m0, WIDE_BM) * a.ldo * (EPI == EPI_RAW ? 4 : 1);
+        ro.o = EPI == EPI_RAW
+                   ? __builtin_amdgcn_make_buffer_rsrc((void*)(a.out32 + (size_t)m0 * a.ldo), (short)0, ob, BUF_DWORD3)
+                   : __builtin_amdgcn_make_buffer_rsrc((void*)(a.out8 + (size_t)m0 * a.ldo), (short)0, ob, BUF_DWORD3);
+    }
+    if (EPI == EPI_QKV) {
+        const int kcol = col_base - a.d;
+        if (kcol >= 0) {
+            int isv;
+            if (a.kv_mode == 1) { isv = kcol >= 64 * a.G; g = (isv ? kcol - 64 * a.G : kcol) >> 6; }
+            else isv = kcol >= 64;
+            role = isv ? 2 : 1;
+        }
+        // the caches from the block's first chunk (as the strips of k_gemm_ws)
+        const long long nb = a.pos >= 0 ? a.M : (a.M + a.T - 1) / a.T;
+        ro.b0 = a.pos >= 0 ? m0 : m0 / a.T;
+        const long long kb = (long long)a.KH * a.T * 64, vb = (long long)a.KH * 64 * a.TP;
+        ro.k = __builtin_amdgcn_make_buffer_rsrc((void*)(a.kc + ro.b0 * kb), (short)0,
+                                                 (int)min((nb - ro.b0) * kb, 0x7FFFFF00ll), BUF_DWORD3);
+        ro.v = __builtin_amdgcn_make_buffer_rsrc((void*)(a.vc + ro.b0 * vb), (short)0,
+                                                 (int)min((nb - ro.b0) * vb, 0x7FFFFF00ll), BUF_DWORD3);
+        ro.vl = a.vl;
+    }
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        const int row = m0 + i * 16 + lr;
+        WsTile t;
+        QkvRow qr;
+        if (EPI == EPI_QKV) qkv_row(a, row, c4, qr);
+        if (EPI != EPI_QKV || role == 0) {
+            epi_ws<EPI, FAST, 0>(a, ro, acc[i], row, col_base, c4, qr, g, t);
+            flush_ws<EPI, 0>(ro, t);
+        } else if (role == 1) {
+            epi_ws<EPI, FAST, 1>(a, ro, acc[i], row, col_base, c4, qr, g, t);
+            flush_ws<EPI, 1>(ro, t);
+        } else {
+            epi_ws<EPI, FAST, 2>(a, ro, acc[i], row, col_base, c4, qr, g, t);
+            flush_ws<EPI, 2>(ro, t);
+        }
+    }
+}
+
+template <int EPI>
+static bool try_wide(const GemmArgs& a, hipStream_t s) {
+    if (a.tiled || !a.Wf || a.a_rows || a.M < a.wide_rows || a.N % 64 != 0 || (long long)a.N * a.K >= (1ll << 31) - (1 << 20) ||
+        (long long)WIDE_BM * a.K >= (1ll << 31) || (long long)WIDE_BM * a.ldo * (EPI == EPI_RAW ? 4 : 1) >= (1ll << 31))
+        return false;
+    // 32-bit offsets into the caches from a block's first chunk
+    if (EPI == EPI_QKV && (((long long)WIDE_BM / a.T + 2) * a.KH * a.TP * 64 >= (1ll << 31) || a.T > a.TP || a.pos >= 0)) return false;
+    const int ntm = (a.M + WIDE_BM - 1) / WIDE_BM, ntn = (a.N + WIDE_BN - 1) / WIDE_BN;
+    const int groups = (ntm + NXCD * WIDE_GROUP - 1) / (NXCD * WIDE_GROUP);
+    const dim3 grid((unsigned)(groups * WIDE_GROUP * NXCD * ntn));
+    if (a.rq_fast) hipLaunchKernelGGL((k_gemm_wide<EPI, true>), grid, dim3(256), 0, s, a);
+    else hipLaunchKernelGGL((k_gemm_wide<EPI, false>), grid, dim3(256), 0, s, a);
+    return true;
+}
+
+// ---------------------------------------------------------------------------
 // GEMM of a few rows (decode steps of few streams, short prefills): bound by
 // the latency of the weights, which come from L2 or the memory behind it and
 // are used once.  A workgroup takes 16 RT rows and 16 output columns (QKV and
@@ -604,10 +745,10 @@ static bool try_ws(const GemmArgs& a, hipStream_t s) {
 
 void launch_gemm(const GemmArgs& a, int epi, hipStream_t s) {
     switch (epi) {
-        case EPI_RAW: if (try_skinny<EPI_RAW>(a, s) || try_ws<EPI_RAW>(a, s)) return; break;
-        case EPI_REQ: if (try_skinny<EPI_REQ>(a, s) || try_ws<EPI_REQ>(a, s)) return; break;
-        case EPI_QKV: if (try_skinny<EPI_QKV>(a, s) || try_ws<EPI_QKV>(a, s)) return; break;
-        default: if (try_skinny<EPI_REGLU>(a, s) || try_ws<EPI_REGLU>(a, s)) return; break;
+        case EPI_RAW: if (try_skinny<EPI_RAW>(a, s) || try_ws<EPI_RAW>(a, s) || try_wide<EPI_RAW>(a, s)) return; break;
+        case EPI_REQ: if (try_skinny<EPI_REQ>(a, s) || try_ws<EPI_REQ>(a, s) || try_wide<EPI_REQ>(a, s)) return; break;
+        case EPI_QKV: if (try_skinny<EPI_QKV>(a, s) || try_ws<EPI_QKV>(a, s) || try_wide<EPI_QKV>(a, s)) return; break;
+        default: if (try_skinny<EPI_REGLU>(a, s) || try_ws<EPI_REGLU>(a, s) || try_wide<EPI_REGLU>(a, s)) return; break;
     }
     const int ntm = (a.M + BM - 1) / BM, ntn = (a.N + BN - 1) / BN;
     dim3 grid((unsigned)(((ntm + NXCD - 1) / NXCD) * NXCD * ntn));
@@ -1034,6 +1175,24 @@ void launch_gemm_rn(const RowGemmArgs& a, hipStream_t s) {
         g.A = a.A; g.Wf = a.Wf; g.M = a.M; g.N = a.d; g.K = a.K; g.out8 = a.y8; g.ldo = a.d;
         g.mult = a.mult; g.shift = a.shift; g.rq_scale = a.rq_scale; g.rq_fast = a.rq_fast; g.skinny_rows = a.skinny_rows;
         if (try_skinny<EPI_REQ>(g, s)) {
+            launch_rn_rows(a, s);
+            return;
+        }
+    }
+    if (a.y8 && !a.tiled && a.d >= 768 && a.M >= 2 * a.wide_rows) {
+        // many rows: the product in 128 x 256 tiles and the norms apart move y
+        // (d bytes a row) out and back, and are faster still than 64 rows x d a
+        // workgroup with the weights streamed past every one of them.  d768,
+        // 200 thousand rows, 12 layers: O + norms 4.5 -> 3.3 ms, down + norms
+        // (K = 3072) 9.9 -> 6.4; 32 thousand rows 0.77 -> 0.67 and 1.57 -> 1.20;
+        // 4096 rows 0.22 -> 0.24 and 0.43 -> 0.44.  Not for d512, where these
+        // two kernels gain as much (26.3 -> 19.2 ms a million rows, 8 layers) but
+        // the call is at the card's power limit: the attention between them
+        // slows down by more (41 -> 47 ms; 86.3 -> 87.8 ms in all)
+        GemmArgs g{};
+        g.A = a.A; g.Wf = a.Wf; g.M = a.M; g.N = a.d; g.K = a.K; g.out8 = a.y8; g.ldo = a.d;
+        g.mult = a.mult; g.shift = a.shift; g.rq_scale = a.rq_scale; g.rq_fast = a.rq_fast; g.wide_rows = a.wide_rows;
+        if (try_wide<EPI_REQ>(g, s)) {
             launch_rn_rows(a, s);
             return;
         }

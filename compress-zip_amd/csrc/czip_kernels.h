@@ -36,8 +36,10 @@ struct GemmArgs {
     const int16_t* rcos;
     const int16_t* rsin;
     int tiled;        // 1: the tiled kernel only (no W-stationary one; a per-context test switch)
-    const int8_t* Wf = nullptr;  // W fragment-major (rowblock_mma), for launches of at most skinny_rows rows
-    int skinny_rows = 0;
+    // W fragment-major (rowblock_mma), for launches of at most skinny_rows rows
+    // and, for the K that have no W-stationary kernel, of at least wide_rows
+    const int8_t* Wf = nullptr;
+    int skinny_rows = 0, wide_rows = 0;
 };
 
 // The attention's exp table by table step t (exp_q16, lut.rs:213-235):
@@ -100,8 +102,8 @@ struct RowGemmArgs {
     int32_t* ws;           // optional workspace of ws_bytes for the split-K path (few rows)
     size_t ws_bytes;
     int tiled;             // 1: the tiled row kernel only (no W-stationary one; a per-context test switch)
-    int8_t* y8 = nullptr;  // [M, d] or nullptr: the projection output of launches of at most skinny_rows rows
-    int skinny_rows = 0;
+    int8_t* y8 = nullptr;  // [M, d] or nullptr: the projection output where product and norms are kernels of their own
+    int skinny_rows = 0, wide_rows = 0;
 };
 bool gemm_rn_supported(int d);
 // bytes of workspace the split-K row GEMM wants for M rows of width d (0: M is large enough without)

@@ -217,3 +217,22 @@ def test_row_gemm_16_without_tail(amd, shipped, monkeypatch):
     monkeypatch.setenv("CZIP_TAIL_ROWS", "0")
     gm = amd.Model(amd.ModelWeights(MODEL_PATH))
     parity.test_small_launch_row_gemm(gm, shipped, 4, 512)
+
+
+@pytest.mark.parametrize("heads,kv,d_ff,vocab", [(12, 4, 448, 1088), (10, 5, 192, 1024), (14, 2, 832, 2112), (8, 1, 1024, 1024)])
+def test_wide_gemms(amd, orc, tmp_path, monkeypatch, heads, kv, d_ff, vocab):
+    """The 128 x 256 tiles at row counts around their row blocks, for column
+    counts with a partial last tile and odd and even numbers of K steps (3, 7,
+    10, 13 and 14 of 64 among them), over ragged chunks; the norms behind them
+    where the row count asks for them."""
+    import test_gpu_parity as parity
+    from czip_amd import synth
+    path = synth.write_random_model(str(tmp_path / "w.czm"), d=64 * heads, n_layers=2, n_heads=heads, n_kv=kv,
+                                    d_ff=d_ff, vocab=vocab, ctx=600, seed=600 + heads)
+    monkeypatch.setenv("CZIP_SKINNY_ROWS", "0")
+    monkeypatch.setenv("CZIP_TAIL_ROWS", "0")
+    monkeypatch.setenv("CZIP_WIDE_ROWS", "1")
+    gm = amd.Model(amd.ModelWeights(path, amd.KV_GQA))
+    om = orc.Model.from_file(path, amd.KV_GQA)
+    for lens in ([1], [127], [64, 64], [129], [513], [200, 31, 200, 200]):
+        parity._check_logits(gm, om, max(lens), lens, 11 + len(lens), vocab)
