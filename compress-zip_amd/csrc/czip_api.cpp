@@ -1380,7 +1380,7 @@ static czip_status run_decompress(czip_job* j) {
                 const Lane& Ln = lanes[ln];
                 const hipStream_t s = Ln.s;
                 const int M = Ln.S;
-                {
+                if (c->head_fused || p == 0) {  // the unfused head leaves the next step's input itself
                     Timed t(c, "dec_prep");
                     launch_dec_prep(Ln.ds, Ln.st, M, p, c->head_fused && p > 0, c->cfg.target_total, Ln.r.inp, s);
                 }
@@ -1426,7 +1426,7 @@ static czip_status run_decompress(czip_job* j) {
                     { Timed t(c, "gemm_head"); gemm(c, hd, EPI_RAW, s); }
                     {
                         Timed t(c, "cdf_decode");
-                        launch_cdf_decode(hd.out32, M, V, c->lut, c->cfg.coef_q24, c->cfg.target_total, p, Ln.st, Ln.ds, s);
+                        launch_cdf_decode(hd.out32, M, V, c->lut, c->cfg.coef_q24, c->cfg.target_total, p, Ln.st, Ln.ds, Ln.r.inp, s);
                     }
                 }
             }

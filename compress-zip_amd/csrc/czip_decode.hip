@@ -40,29 +40,49 @@ void launch_dec_init(DecState st, DecStreams ds, int S, hipStream_t s) {
     hipLaunchKernelGGL(k_dec_init, dim3((unsigned)((S + 63) / 64)), dim3(64), 0, s, st, ds, S);
 }
 
+// A stream's decoder state and the 8 bytes of its chunk from the next bit's
+// byte on.  They come from three aligned words of the chunk buffer (which
+// carries 16 bytes of padding); bytes at or past the chunk's end read as 0
+// (arith_coder.rs:176-190).
+struct DecLoad {
+    unsigned low, high, code;
+    long long len, bp, start;
+    int bi;
+    unsigned w0, w1, w2;
+};
+
+__device__ __forceinline__ DecLoad dec_load(DecState st, DecStreams ds, int b) {
+    DecLoad d;
+    d.low = st.low[b];
+    d.high = st.high[b];
+    d.code = st.code[b];
+    d.len = ds.blen[b];
+    d.bp = st.byte_pos[b];
+    d.bi = st.bit_pos[b];
+    d.start = ds.offs[b] + d.bp;
+    const unsigned* w = (const unsigned*)(ds.data + (d.start & ~3ll));
+    d.w0 = w[0];
+    d.w1 = w[1];
+    d.w2 = w[2];
+    return d;
+}
+
 // The decoder step of a decoded symbol with interval [lo, hi) (arith_coder.rs:243-262):
-// narrow (low, high), then renormalize, reading the stream's bits from an
+// narrow (low, high), then renormalize, reading the stream's bits from the
 // 8-byte window: a step shifts at most 32 bits (each pass shifts a 0 into low
 // and a 1 into high; after 32 of them low = 0, high = 2^32 - 1 ends the loop).
-// The window comes from three aligned words of the chunk buffer (which carries
-// 16 bytes of padding); bytes at or past the chunk's end read as 0
-// (arith_coder.rs:176-190).
-__device__ __forceinline__ void dec_advance(DecState st, DecStreams ds, int b, unsigned lo, unsigned hi, unsigned total) {
-    const unsigned low = st.low[b], high = st.high[b], code = st.code[b];
+__device__ __forceinline__ void dec_advance(const DecLoad& d, DecState st, int b, unsigned lo, unsigned hi, unsigned total) {
+    const unsigned low = d.low, high = d.high;
     const unsigned long long range = (unsigned long long)high - low + 1;
     const double invT = 1.0 / (double)total;
     unsigned long long nh = low + udiv64_32((unsigned long long)hi * range, total, invT) - 1;
     unsigned long long nl = low + udiv64_32((unsigned long long)lo * range, total, invT);
-    unsigned long long cd = code;
-    const long long len = ds.blen[b];
-    const long long bp = st.byte_pos[b];
-    const int bi = st.bit_pos[b];
-    const long long start = ds.offs[b] + bp, base = start & ~3ll;
-    const unsigned* w = (const unsigned*)(ds.data + base);
-    const unsigned w0 = w[0], w1 = w[1], w2 = w[2];
-    const int sh = (int)(start - base) * 8;
-    const unsigned long long lo64 = ((unsigned long long)w1 << 32) | w0;
-    unsigned long long v = sh ? (lo64 >> sh) | ((unsigned long long)w2 << (64 - sh)) : lo64;  // bytes bp .. bp + 7
+    unsigned long long cd = d.code;
+    const long long len = d.len, bp = d.bp;
+    const int bi = d.bi;
+    const int sh = (int)(d.start & 3ll) * 8;
+    const unsigned long long lo64 = ((unsigned long long)d.w1 << 32) | d.w0;
+    unsigned long long v = sh ? (lo64 >> sh) | ((unsigned long long)d.w2 << (64 - sh)) : lo64;  // bytes bp .. bp + 7
     const long long nv = len - bp;
     if (nv < 8) v = nv <= 0 ? 0ull : v & ((1ull << (8 * nv)) - 1ull);
     const unsigned long long win = __builtin_bswap64(v);  // MSB first
@@ -101,7 +121,7 @@ __global__ void k_dec_prep(DecStreams ds, DecState st, int S, int p, int upd, un
     const int b = blockIdx.x * blockDim.x + threadIdx.x;
     if (b >= S) return;
     const int n = ds.ntok[b];
-    if (upd && p <= n) dec_advance(st, ds, b, st.pend_lo[b], st.pend_hi[b], total);
+    if (upd && p <= n) dec_advance(dec_load(st, ds, b), st, b, st.pend_lo[b], st.pend_hi[b], total);
     uint32_t t = 0u;
     if (p < n) t = p == 0 ? BOS_TOKEN : ds.tokens[ds.tok_offs[b] + p - 1];
     inp[b] = t;
@@ -397,12 +417,18 @@ void launch_attn_decode(const AttnArgs& a, int S, int p, hipStream_t s) {
 // Logits -> cumulative frequencies (softmax_cdf.rs:85-139) -> one decode step
 // (arith_coder.rs:195-264).  Same frequency arithmetic as the prefill CDF
 // kernel; the symbol is the first index whose cumulative frequency exceeds
-// value = ((code - low + 1) * total - 1) / range.
+// value = ((code - low + 1) * total - 1) / range.  Also leaves the next step's
+// forward input (main.rs:386-388) in inp.  A step of few streams is one
+// chain: the decoder's state and stream words are requested with the logits,
+// and a row takes as many waves as a workgroup holds.  V = 8192, against four
+// waves a row and stream bits read one by one: 59 streams 21.6 -> 13.5 us, 512
+// 31.5 -> 23.8; with four waves still, 1024 41.2 -> 26.5.
 // ---------------------------------------------------------------------------
 template <int WPR, int EPL>
 __global__ __launch_bounds__(64 * WPR) void k_cdf_decode(const int32_t* __restrict__ logits, int V,
                                                          const uint16_t* __restrict__ glut, unsigned coef,
-                                                         unsigned total, int p, DecState st, DecStreams ds) {
+                                                         unsigned total, int p, DecState st, DecStreams ds,
+                                                         uint32_t* __restrict__ inp) {
     __shared__ uint16_t lut[256];
     __shared__ int red_i[WPR];
     __shared__ unsigned red_u[WPR];
@@ -410,13 +436,27 @@ __global__ __launch_bounds__(64 * WPR) void k_cdf_decode(const int32_t* __restri
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int b = blockIdx.x;
     for (int i = tid; i < 256; i += 64 * WPR) lut[i] = glut[i];
-    if (p >= ds.ntok[b]) return;  // uniform per block
-    __syncthreads();
+    const int n = ds.ntok[b];
+    if (p >= n) {  // uniform per block
+        if (tid == 0) inp[b] = 0u;
+        return;
+    }
     const int i0 = tid * EPL;
     const int32_t* L = logits + (size_t)b * V;
     int lv[EPL];
+    if (i0 + EPL <= V) {
 #pragma unroll
-    for (int k = 0; k < EPL; k++) lv[k] = (i0 + k < V) ? L[i0 + k] : INT32_MIN;
+        for (int k = 0; k < EPL; k += 4) {
+            int4 v = *(const int4*)(L + i0 + k);
+            lv[k] = v.x; lv[k + 1] = v.y; lv[k + 2] = v.z; lv[k + 3] = v.w;
+        }
+    } else {
+#pragma unroll
+        for (int k = 0; k < EPL; k++) lv[k] = (i0 + k < V) ? L[i0 + k] : INT32_MIN;
+    }
+    const DecLoad dec = dec_load(st, ds, b);
+    const long long tok_off = ds.tok_offs[b];
+    __syncthreads();
     auto bmax = [&](int v) {
         v = wave_max_i(v);
         if (WPR == 1) return v;
@@ -495,10 +535,8 @@ __global__ __launch_bounds__(64 * WPR) void k_cdf_decode(const int32_t* __restri
         for (int w = 0; w < wave; w++) excl += red_u[w];
         __syncthreads();
     }
-    // decoder state
-    const unsigned long long low = st.low[b], high = st.high[b], code = st.code[b];
-    const unsigned long long range = high - low + 1;  // <= 2^32
-    const unsigned long long value = ((code - low + 1) * (unsigned long long)total - 1) / range;
+    const unsigned long long range = (unsigned long long)dec.high - dec.low + 1;  // <= 2^32
+    const unsigned long long value = (((unsigned long long)dec.code - dec.low + 1) * (unsigned long long)total - 1) / range;
     const unsigned v32 = (unsigned)value;
     // first i with v32 < cum_i, clamped to V-1 (arith_coder.rs:225-241)
     unsigned run = excl + (am < i0 ? rem : 0u);
@@ -520,47 +558,20 @@ __global__ __launch_bounds__(64 * WPR) void k_cdf_decode(const int32_t* __restri
     if (sym == best) { found[0] = lo_c; found[1] = hi_c; }
     __syncthreads();
     if (tid != 0) return;
-    const unsigned long long sl = found[0], sh = found[1];
-    const double invT = 1.0 / (double)total;
-    unsigned long long nh = low + udiv64_32(sh * range, total, invT) - 1;
-    unsigned long long nl = low + udiv64_32(sl * range, total, invT);
-    unsigned long long cd = code;
-    const uint8_t* data = ds.data + ds.offs[b];
-    const long long len = ds.blen[b];
-    long long bp = st.byte_pos[b];
-    int bi = st.bit_pos[b];
-    for (;;) {
-        if (((nl ^ nh) & DHALF) == 0) {
-            nl = (nl << 1) & DMASK;
-            nh = ((nh << 1) & DMASK) | 1;
-            cd = ((cd << 1) & DMASK) | read_bit(data, len, bp, bi);
-        } else if ((nl & ~nh & DQUART) != 0) {
-            nl = ((nl << 1) ^ DHALF) & DMASK;
-            nh = (((nh ^ DHALF) << 1) | DHALF | 1) & DMASK;
-            cd = (cd & DHALF) | ((cd << 1) & (DMASK >> 1)) | read_bit(data, len, bp, bi);
-        } else {
-            break;
-        }
-    }
-    st.low[b] = (uint32_t)nl;
-    st.high[b] = (uint32_t)nh;
-    st.code[b] = (uint32_t)cd;
-    st.byte_pos[b] = bp;
-    st.bit_pos[b] = bi;
-    ds.tokens[ds.tok_offs[b] + p] = (uint32_t)best;
+    dec_advance(dec, st, b, found[0], found[1], total);
+    ds.tokens[tok_off + p] = (uint32_t)best;
+    inp[b] = p + 1 < n ? (uint32_t)best : 0u;
 }
 
 void launch_cdf_decode(const int32_t* logits, int S, int V, const uint16_t* lut, unsigned coef, unsigned total, int p,
-                       DecState st, DecStreams ds, hipStream_t s) {
-    if (V <= 1024)
-        hipLaunchKernelGGL((k_cdf_decode<1, 16>), dim3((unsigned)S), dim3(64), 0, s, logits, V, lut, coef, total, p,
-                           st, ds);
-    else if (V <= 4096)
-        hipLaunchKernelGGL((k_cdf_decode<4, 16>), dim3((unsigned)S), dim3(256), 0, s, logits, V, lut, coef, total, p,
-                           st, ds);
-    else
-        hipLaunchKernelGGL((k_cdf_decode<4, 32>), dim3((unsigned)S), dim3(256), 0, s, logits, V, lut, coef, total, p,
-                           st, ds);
+                       DecState st, DecStreams ds, uint32_t* inp, hipStream_t s) {
+#define CZIP_CDF_DEC(W, E) \
+    hipLaunchKernelGGL((k_cdf_decode<W, E>), dim3((unsigned)S), dim3(64 * W), 0, s, logits, V, lut, coef, total, p, st, ds, inp)
+    const bool few = S <= CDF_FEW_ROWS;
+    if (V <= 1024) { if (few) CZIP_CDF_DEC(4, 4); else CZIP_CDF_DEC(1, 16); }
+    else if (V <= 4096) { if (few) CZIP_CDF_DEC(16, 4); else CZIP_CDF_DEC(4, 16); }
+    else { if (few) CZIP_CDF_DEC(16, 8); else CZIP_CDF_DEC(4, 32); }
+#undef CZIP_CDF_DEC
 }
 
 // ---------------------------------------------------------------------------

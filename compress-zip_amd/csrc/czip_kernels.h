@@ -183,6 +183,10 @@ void launch_attention(const AttnArgs& a, int B, hipStream_t s);
 // mode 0: (lo, hi) of targets; mode 1: full inclusive cumfreqs; mode 2:
 // targets are decoder values, out rows (sym, cum_lo, cum_hi).  Row r of the
 // launch is written at output row out_row0 + r.
+// Launches of at most this many rows (two workgroups of 16 waves a CU) give a
+// row to as many waves as hold its logits at 4 or 8 a lane: they are bound by
+// one row's chain of reductions
+constexpr int CDF_FEW_ROWS = 512;
 void launch_cdf(const int32_t* logits, int M, int V, const uint32_t* targets, const int32_t* lens, int T,
                 const uint16_t* lut, unsigned coef, unsigned total, int mode, uint32_t* out, int64_t out_row0,
                 hipStream_t s);
@@ -223,7 +227,7 @@ void launch_dec_prep(DecStreams ds, DecState st, int S, int p, bool upd, unsigne
 void launch_attn_decode(const AttnArgs& a, int S, int p, hipStream_t s);
 // logits -> cumulative frequencies -> one arithmetic-decode step (arith_coder.rs:195-264)
 void launch_cdf_decode(const int32_t* logits, int S, int V, const uint16_t* lut, unsigned coef, unsigned total,
-                       int p, DecState st, DecStreams ds, hipStream_t s);
+                       int p, DecState st, DecStreams ds, uint32_t* inp, hipStream_t s);
 // LM head + frequency table + symbol search + decoder step of S streams in one
 // kernel (head_cdf_supported(V)); A = the final-normalized rows [S, K]
 struct HeadDecArgs {

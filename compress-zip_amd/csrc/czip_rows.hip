@@ -647,15 +647,14 @@ __global__ __launch_bounds__(64 * WPR) void k_cdf(const int32_t* __restrict__ lo
 void launch_cdf(const int32_t* logits, int M, int V, const uint32_t* targets, const int32_t* lens, int T,
                 const uint16_t* lut, unsigned coef, unsigned total, int mode, uint32_t* out, int64_t out_row0,
                 hipStream_t s) {
-    if (V <= 1024)
-        hipLaunchKernelGGL((k_cdf<1, 16>), dim3((unsigned)M), dim3(64), 0, s, logits, V, targets, lens, T, lut, coef,
-                           total, mode, out, (long long)out_row0);
-    else if (V <= 4096)
-        hipLaunchKernelGGL((k_cdf<4, 16>), dim3((unsigned)M), dim3(256), 0, s, logits, V, targets, lens, T, lut, coef,
-                           total, mode, out, (long long)out_row0);
-    else
-        hipLaunchKernelGGL((k_cdf<4, 32>), dim3((unsigned)M), dim3(256), 0, s, logits, V, targets, lens, T, lut, coef,
-                           total, mode, out, (long long)out_row0);
+#define CZIP_CDF(W, E)                                                                                             \
+    hipLaunchKernelGGL((k_cdf<W, E>), dim3((unsigned)M), dim3(64 * W), 0, s, logits, V, targets, lens, T, lut, coef, \
+                       total, mode, out, (long long)out_row0)
+    const bool few = M <= CDF_FEW_ROWS;
+    if (V <= 1024) { if (few) CZIP_CDF(4, 4); else CZIP_CDF(1, 16); }
+    else if (V <= 4096) { if (few) CZIP_CDF(16, 4); else CZIP_CDF(4, 16); }
+    else { if (few) CZIP_CDF(16, 8); else CZIP_CDF(4, 32); }
+#undef CZIP_CDF
 }
 
 // ---------------------------------------------------------------------------

@@ -236,3 +236,27 @@ def test_wide_gemms(amd, orc, tmp_path, monkeypatch, heads, kv, d_ff, vocab):
     om = orc.Model.from_file(path, amd.KV_GQA)
     for lens in ([1], [127], [64, 64], [129], [513], [200, 31, 200, 200]):
         parity._check_logits(gm, om, max(lens), lens, 11 + len(lens), vocab)
+
+
+@pytest.mark.parametrize("vocab,env", [(1024, "CZIP_UNFUSED_HEAD"), (1088, None), (4096, None), (4160, None), (8192, None)])
+def test_decode_step_wave_counts(amd, orc, tmp_path, monkeypatch, vocab, env):
+    """The unfused head's decoder step with a row's logits over one, four and
+    sixteen waves (up to 512 rows, then more), at the edges of their vocabulary
+    ranges; streams that end at different steps and streams cut short."""
+    from czip_amd import synth
+    if env:
+        monkeypatch.setenv(env, "1")
+    path = synth.write_random_model(str(tmp_path / "c.czm"), d=128, n_layers=1, n_heads=2, n_kv=1, d_ff=64, vocab=vocab,
+                                    ctx=64, seed=700 + vocab)
+    gm = amd.Model(amd.ModelWeights(path, amd.KV_GQA))
+    om = orc.Model.from_file(path, amd.KV_GQA)
+    rng = np.random.default_rng(vocab)
+    toks = rng.integers(0, vocab, 24 * 13).astype(np.uint32)
+    coded = om.compress_many(toks, 13, threads=8)
+    for S in (24, 512, 513):
+        pick = rng.integers(0, 24, S)
+        lens = rng.integers(0, 14, S).astype(np.int32)
+        want = np.concatenate([toks[13 * c:13 * c + n] for c, n in zip(pick, lens)])
+        assert np.array_equal(gm.decompress_chunks([coded[c] for c in pick], lens), want)
+    cut = [c[:3 * i % (len(c) + 1)] for i, c in enumerate(coded)]
+    assert np.array_equal(gm.decompress_chunks(cut, [13] * 24), om.decompress_many(cut, [13] * 24))
