@@ -591,7 +591,7 @@ static bool try_wide(const GemmArgs& a, hipStream_t s) {
 // ---------------------------------------------------------------------------
 // GEMM of a few rows (decode steps of few streams, short prefills): bound by
 // the latency of the weights, which come from L2 or the memory behind it and
-// are used once.  A workgroup takes 16 RT rows and 16 output columns (QKV and
+// are used once.  A workgroup takes 16 RT rows (RT 1, 2 or 4) and 16 output columns (QKV and
 // ReGLU: a pair of 16-column tiles 32 apart, what their epilogues join), its
 // waves split K, and every wave's operands (W fragment-major, A straight from
 // its rows) are requested at once, SKINNY_U K steps at a time.  The waves'
@@ -601,6 +601,14 @@ static bool try_wide(const GemmArgs& a, hipStream_t s) {
 // 15 -> 8.1; d512 down + norms at 512 rows 17.4 -> 12.4 (16-row row GEMM).
 // ---------------------------------------------------------------------------
 constexpr int SKINNY_U = 3;  // K steps of operands in flight per wave
+// While 64-row workgroups do not cover the 256 CUs, 16 rows a workgroup, and
+// short of two a CU 32: a workgroup's time goes with the operand rows it reads
+// (64 rows of K = 3072: 196 KB beside 48 KB of weights), and the weights read
+// again are in the L2 (row tiles of one column tile are nx workgroups apart,
+// on one XCD where nx is a multiple of 8).  A step of d768, all layers, 64-row
+// workgroups -> these: 24 streams 422 -> 387 us, 96 505 -> 434, 256 587 -> 530,
+// 512 797 -> 725; d512 24 277 -> 252, 512 374 -> 363
+constexpr unsigned SKINNY_RT1_WGS = 256, SKINNY_RT2_WGS = 512;
 
 template <int EPI, bool FAST, int NW, int RT>
 __global__ __launch_bounds__(64 * NW) void k_gemm_skinny(GemmArgs a) {
@@ -675,8 +683,11 @@ __global__ __launch_bounds__(64 * NW) void k_gemm_skinny(GemmArgs a) {
 template <int EPI, bool FAST, int NW>
 static void launch_skinny_nw(const GemmArgs& a, hipStream_t s) {
     const unsigned nx = (unsigned)(EPI == EPI_QKV || EPI == EPI_REGLU ? a.N / 32 : a.N / 16);
-    if (a.M <= 16)
-        hipLaunchKernelGGL((k_gemm_skinny<EPI, FAST, NW, 1>), dim3(nx, 1), dim3(64 * NW), 0, s, a);
+    const unsigned wgs = nx * (unsigned)((a.M + 63) / 64);
+    if (a.M <= 16 || wgs < SKINNY_RT1_WGS)
+        hipLaunchKernelGGL((k_gemm_skinny<EPI, FAST, NW, 1>), dim3(nx, (unsigned)((a.M + 15) / 16)), dim3(64 * NW), 0, s, a);
+    else if (wgs < SKINNY_RT2_WGS)
+        hipLaunchKernelGGL((k_gemm_skinny<EPI, FAST, NW, 2>), dim3(nx, (unsigned)((a.M + 31) / 32)), dim3(64 * NW), 0, s, a);
     else
         hipLaunchKernelGGL((k_gemm_skinny<EPI, FAST, NW, 4>), dim3(nx, (unsigned)((a.M + 63) / 64)), dim3(64 * NW), 0, s, a);
 }
