@@ -52,10 +52,13 @@ constexpr long long ATTN_ROWS_MAX = 8192;
 constexpr int64_t TAIL_ROWS_MAX = 20480;
 constexpr size_t TAIL_WEIGHTS_MAX = (size_t)4 << 20, TAIL_WEIGHT_BYTES_PER_ROW = 2500;
 // GEMMs of at most this many rows split K over a workgroup's waves and the
-// columns over the chip (CZIP_SKINNY_ROWS).  Decode of 512 streams: d768 64
-// steps 72 -> 52 ms, d512 128 steps 52 -> 43, v001 256 steps 15.0 -> 14.4; of
-// 1024 streams d768 76 -> 73, d512 59.2 -> 59.6 ms
-constexpr int SKINNY_ROWS_MAX = 512;
+// columns over the chip (CZIP_SKINNY_ROWS); half of it where the layer tail
+// takes over below it.  A step-wise decode step, other kernels -> these: d768
+// 513 streams 1141 -> 768 us, 768 1134 -> 970, 1024 1175 -> 1078; d512 513
+// 470 -> 380, 768 485 -> 429, 1024 496 -> 490; v001, against the tail, 513
+// 106 -> 106, 768 102 -> 110.  Compressing as many tokens in chunks of 256: d512
+// 520 732 -> 677, 1024 740 -> 723 us; d768 520 1271 -> 1253, 1024 1292 -> 1327
+constexpr int SKINNY_ROWS_MAX = 1024;
 // GEMMs of at least this many rows, where no W-stationary kernel takes them,
 // run 128 x 256 tiles with the weights straight from L2 (CZIP_WIDE_ROWS)
 constexpr int WIDE_ROWS_MIN = 4096;
@@ -597,6 +600,7 @@ extern "C" czip_status czip_create(const czip_model_desc* w, int device, czip_ct
         }
         c->tail_rows = ok ? TAIL_ROWS_MAX : 0;
         c->tail_rows_min = (int64_t)(d * (qn + d + 3 * F) / TAIL_WEIGHT_BYTES_PER_ROW);
+        if (ok && c->tail_rows_min < SKINNY_ROWS_MAX && getenv("CZIP_SKINNY_ROWS") == nullptr) c->skinny_rows = SKINNY_ROWS_MAX / 2;
         if (const char* e = getenv("CZIP_TAIL_ROWS")) c->tail_rows = ok ? std::max(0ll, atoll(e)) : 0;
     }
     czip_ctx* C = c.get();

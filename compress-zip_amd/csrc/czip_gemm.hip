@@ -596,9 +596,10 @@ static bool try_wide(const GemmArgs& a, hipStream_t s) {
 // waves split K, and every wave's operands (W fragment-major, A straight from
 // its rows) are requested at once, SKINNY_U K steps at a time.  The waves'
 // sums meet in LDS; wave i sums and finishes row tile i.  Per launch, events
-// included (d768 / 12 layers, 59 rows): QKV 14.3 -> 7.8 us, up + ReGLU 12.8 ->
-// 6.7, O + norms 22 -> 10.3, down + norms (K = 3072) 31 -> 13.9, head (V = 8192)
-// 15 -> 8.1; d512 down + norms at 512 rows 17.4 -> 12.4 (16-row row GEMM).
+// included (d768 / 12 layers), tiled kernels -> these: 59 rows QKV 14.3 -> 6.4
+// us, up + ReGLU 12.8 -> 6.8, O + norms 22.2 -> 10.1, down + norms (K = 3072)
+// 31.4 -> 10.1, head (V = 8192) 14.8 -> 8.0; 512 rows QKV 18.7 -> 8.8, up 15.1
+// -> 15.8, O + norms 15.0 -> 11.8, down + norms 33.8 -> 18.5.
 // ---------------------------------------------------------------------------
 constexpr int SKINNY_U = 3;  // K steps of operands in flight per wave
 // While 64-row workgroups do not cover the 256 CUs, 16 rows a workgroup, and
@@ -705,7 +706,7 @@ template <int EPI>
 static bool try_skinny(const GemmArgs& a, hipStream_t s) {
     // every 64 rows read the weights again: the wide head stops paying sooner
     // (512 rows, V = 8192: 21 -> 30 us; 256 rows 18.8 -> 17.8)
-    const int most = EPI == EPI_RAW ? a.skinny_rows / 2 : a.skinny_rows;
+    const int most = EPI == EPI_RAW ? std::min(a.skinny_rows, 256) : a.skinny_rows;
     if (a.tiled || !a.Wf || a.a_rows || a.M <= 0 || a.M > most || a.N % 64 != 0 || a.K % 64 != 0 ||
         (long long)a.N * a.K >= (1ll << 31))
         return false;

@@ -260,3 +260,16 @@ def test_decode_step_wave_counts(amd, orc, tmp_path, monkeypatch, vocab, env):
         assert np.array_equal(gm.decompress_chunks([coded[c] for c in pick], lens), want)
     cut = [c[:3 * i % (len(c) + 1)] for i, c in enumerate(coded)]
     assert np.array_equal(gm.decompress_chunks(cut, [13] * 24), om.decompress_many(cut, [13] * 24))
+
+
+@pytest.mark.parametrize("heads,kv,d_ff", [(4, 2, 4160), (12, 4, 448)])
+def test_few_row_gemms_row_limit(amd, orc, tmp_path, heads, kv, d_ff):
+    """Row counts up to the few-row GEMMs' limit of 1024 and just past it."""
+    import test_gpu_parity as parity
+    from czip_amd import synth
+    path = synth.write_random_model(str(tmp_path / "l.czm"), d=64 * heads, n_layers=2, n_heads=heads, n_kv=kv,
+                                    d_ff=d_ff, vocab=1088, ctx=600, seed=800 + heads)
+    gm = amd.Model(amd.ModelWeights(path, amd.KV_GQA))
+    om = orc.Model.from_file(path, amd.KV_GQA)
+    for lens in ([520], [385, 385], [512, 300], [513, 512]):
+        parity._check_logits(gm, om, max(lens), lens, 17 + len(lens), 1088)
