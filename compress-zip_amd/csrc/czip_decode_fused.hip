@@ -373,11 +373,16 @@ __global__ __launch_bounds__(64 * FNW) void k_decode_fused(FusedDecArgs a) {
             const int lane = opaque_tid() & 63, lr = lane & 15, grp = lane >> 4, c4 = grp * 4;
             const int nk = a.F / 64;
             v4i w[2][FK];
-            load_ops(w[0], r_down, tile0 * nk + half * FK, lane);
+            auto load = [&](v4i (&d)[FK], int tile) {  // past the last K step: the last one, times zeros
+#pragma unroll
+                for (int s = 0; s < FK; s++)
+                    d[s] = __builtin_amdgcn_raw_buffer_load_b128(r_down, lane * 16, (tile * nk + min(half * FK + s, nk - 1)) * 1024, 0);
+            };
+            load(w[0], tile0);
             lds_barrier();
 #pragma unroll
             for (int i = 0; i < NT; i++) {
-                if (i + 1 < NT) load_ops(w[(i + 1) & 1], r_down, (tile0 + 8 * (i + 1)) * nk + half * FK, lane);
+                if (i + 1 < NT) load(w[(i + 1) & 1], tile0 + 8 * (i + 1));
                 v4i acc = {0, 0, 0, 0};
 #pragma unroll
                 for (int s = 0; s < FK; s++)

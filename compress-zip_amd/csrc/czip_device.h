@@ -416,7 +416,9 @@ __device__ __forceinline__ void lds_barrier() {
 }
 
 // fragment-major weights as a buffer: the lane's offset in a vector register,
-// the 1 KB piece (uniform) in a scalar one
+// the 1 KB piece (uniform) in a scalar one.  The range check is specified for
+// the vector offset only, so a piece must lie inside the weights: requests
+// ahead of their use stay at the last one.
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t weights_rsrc(const int8_t* Wf, int bytes) {
     return __builtin_amdgcn_make_buffer_rsrc((void*)Wf, (short)0, bytes, BUF_DWORD3);
 }

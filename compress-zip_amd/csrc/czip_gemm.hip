@@ -482,7 +482,8 @@ __global__ __launch_bounds__(256, 2) void k_gemm_wide(GemmArgs a) {
     const __amdgpu_buffer_rsrc_t rA = tile_rsrc(a.A, a.M, a.K, m0);
     const __amdgpu_buffer_rsrc_t rW = weights_rsrc(a.Wf, a.N * a.K);
     const int voff = (tid >> 2) * a.K + (tid & 3) * 16, voff2 = voff + 64 * a.K;
-    const int wpc = (col_base >> 4) * nk;  // the wave's first 1 KB piece; column tile t at + t nk
+    // the wave's first 1 KB piece, column tile t at + t nk (a wave past the last column: the last ones, unused)
+    const int wpc = (min(col_base, a.N - 64) >> 4) * nk;
 
     v4i acc[8][4];
 #pragma unroll
@@ -491,26 +492,28 @@ __global__ __launch_bounds__(256, 2) void k_gemm_wide(GemmArgs a) {
         for (int j = 0; j < 4; j++) acc[i][j] = (v4i){0, 0, 0, 0};
     TileRegs ta[2];
     v4i w[2][4];
-    auto fetch_w = [&](v4i (&d)[4], int kt) {  // past the last step or column: other weights, or zeros
+    // past the last step: the last one, unused
+    auto fetch_w = [&](v4i (&d)[4], int kt) {
+        kt = min(kt, nk - 1);
 #pragma unroll
         for (int t = 0; t < 4; t++) d[t] = __builtin_amdgcn_raw_buffer_load_b128(rW, lane * 16, (wpc + t * nk + kt) * 1024, 0);
     };
-    fetch_tile(rA, voff, voff2, 0, ta[0]);
-    fetch_tile(rA, voff, voff2, 64, ta[1]);
+    auto fetch_a = [&](TileRegs& d, int kt) { fetch_tile(rA, voff, voff2, min(kt, nk - 1) * 64, d); };
+    fetch_a(ta[0], 0);
+    fetch_a(ta[1], 1);
     fetch_w(w[0], 0);
     store_tile(ta[0], As[0], tid);
-    fetch_tile(rA, voff, voff2, 128, ta[0]);
+    fetch_a(ta[0], 2);
     lds_barrier();
     // step kt (u = kt % 2): A of step kt + 1 from registers to LDS, W of kt + 1
-    // and A of kt + 3 requested, the products; past the last step the loads
-    // read other rows' bytes or zeros that nothing uses
+    // and A of kt + 3 requested, the products
     auto step = [&](int kt, int u) {
         v4i af[8];
 #pragma unroll
         for (int i = 0; i < 8; i++) af[i] = *(const v4i*)(As[u] + lds64(i * 16 + lr, lane >> 4));
         fetch_w(w[u ^ 1], kt + 1);
         store_tile(ta[u ^ 1], As[u ^ 1], tid);
-        fetch_tile(rA, voff, voff2, (kt + 3) * 64, ta[u ^ 1]);
+        fetch_a(ta[u ^ 1], kt + 3);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int i = 0; i < 8; i++) {

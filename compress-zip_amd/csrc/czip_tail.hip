@@ -198,14 +198,15 @@ __global__ __launch_bounds__(64 * TNW) void k_layer_tail(TailArgs a) {
             }
         }
     };
-    auto load_pair = [&](v4i (&wa)[KS], v4i (&wb)[KS], __amdgpu_buffer_rsrc_t rw, int g) {
-        const int pc = ((g >> 1) * 4 + (g & 1)) * KS;  // past the last pair: other rows of the weights, or zeros
+    auto load_pair = [&](v4i (&wa)[KS], v4i (&wb)[KS], __amdgpu_buffer_rsrc_t rw, int g, int np) {
+        g = min(g, np - 1);  // past the last pair: the last one, unused
+        const int pc = ((g >> 1) * 4 + (g & 1)) * KS;
         load_ops(wa, rw, pc, lane);
         load_ops(wb, rw, pc + 2 * KS, lane);
     };
     v4i wa[2][KS], wb[2][KS];  // the wave's first pair is requested by the caller
     auto pairs = [&](__amdgpu_buffer_rsrc_t rw, int np, auto emit) {
-        auto load = [&](int u, int g) { load_pair(wa[u], wb[u], rw, g); };
+        auto load = [&](int u, int g) { load_pair(wa[u], wb[u], rw, g, np); };
         lds_barrier();
         for (int g = wave; g < np; g += 2 * TNW) {
             v4i ya[RT], yb[RT];
@@ -232,7 +233,7 @@ __global__ __launch_bounds__(64 * TNW) void k_layer_tail(TailArgs a) {
                 for (int t = 0; t < CT; t++) acc[i][t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wo[t][s], af, acc[i][t], 0, 0, 0);
             }
         }
-        load_pair(wa[0], wb[0], r_up, wave);  // in flight during the norms
+        load_pair(wa[0], wb[0], r_up, wave, a.F / 16);  // in flight during the norms
         norms(acc, a.o_scale, w1[0], w2[0], nullptr);
     }
 
@@ -257,12 +258,13 @@ __global__ __launch_bounds__(64 * TNW) void k_layer_tail(TailArgs a) {
 #pragma unroll
             for (int t = 0; t < CT; t++) acc[i][t] = (v4i){0, 0, 0, 0};
         auto load = [&](v4i (&d)[CT], int kt) {
+            kt = min(kt, nk - 1);  // past the last step: the last one, unused
 #pragma unroll
             for (int t = 0; t < CT; t++)
                 d[t] = __builtin_amdgcn_raw_buffer_load_b128(r_down, lane * 16, ((wave * CT + t) * nk + kt) * 1024, 0);
         };
 #pragma unroll
-        for (int u = 0; u < P - 1; u++) load(w[u], u);  // past nk: other rows of the weights, or zeros
+        for (int u = 0; u < P - 1; u++) load(w[u], u);
         lds_barrier();
         for (int k0 = 0; k0 < nk; k0 += P) {
 #pragma unroll
@@ -278,7 +280,7 @@ __global__ __launch_bounds__(64 * TNW) void k_layer_tail(TailArgs a) {
                 }
             }
         }
-        if (QKV) load_pair(wa[0], wb[0], weights_rsrc(a.qkv.Wf, a.qkv.N * D), wave);
+        if (QKV) load_pair(wa[0], wb[0], weights_rsrc(a.qkv.Wf, a.qkv.N * D), wave, a.qkv.N / 32);
         norms(acc, a.dn_scale, w1[1], w2[1], a.xn);
     }
     if (a.x_out) {
