@@ -751,7 +751,8 @@ czip_status alloc_scratch(czip_ctx* c, czip_job* j, int BC, int T, bool logits =
     if ((rc = dalloc(c, j->allocs, &j->attn, M * d))) return rc;
     if ((rc = dalloc(c, j->allocs, &j->y8, M * d))) return rc;
     if ((rc = dalloc(c, j->allocs, &j->r8, M * F))) return rc;
-    if ((rc = dalloc(c, j->allocs, &j->kc, M * (size_t)c->KH * 64))) return rc;
+    // the attention's last key tile reads up to 63 rows past a head's T
+    if ((rc = dalloc(c, j->allocs, &j->kc, M * (size_t)c->KH * 64 + 63 * 64))) return rc;
     if ((rc = dalloc(c, j->allocs, &j->vc, (size_t)BC * pad64(T) * (size_t)c->KH * 64))) return rc;
     if (logits && (rc = dalloc(c, j->allocs, &j->logits, M * V))) return rc;
     return CZIP_OK;
@@ -1649,7 +1650,7 @@ int32_t* carve_prefill(czip_ctx* c, czip_job* j, Carve& cv, int B, int T) {
     j->attn = cv.take<int8_t>(M * d);
     j->y8 = c->rn_fused ? nullptr : cv.take<int8_t>(M * d);
     j->r8 = cv.take<int8_t>(M * F);
-    j->kc = cv.take<int8_t>(M * (size_t)c->KH * 64);
+    j->kc = cv.take<int8_t>(M * (size_t)c->KH * 64);  // the last key tile's rows past T lie in vc (at least 64 rows)
     j->vc = cv.take<int8_t>((size_t)B * pad64(T) * (size_t)c->KH * 64);
     j->logits = c->head_fused ? nullptr : cv.take<int32_t>(M * V);
     // the few-row GEMMs' projection output, where the buffer has room for it

@@ -95,11 +95,12 @@ __global__ __launch_bounds__(64 * NWV, 4) void k_attention(AttnArgs a) {
     // visible keys end in its first half
     const bool half_last = (last & 63) < 32;
     // K [T][64] and V^T [TP/16][64][16] of the chunk's KV head: buffer loads
-    // with the tile offset in the scalar operand; keys past T read as 0 (the
-    // resource's range check) and are never visible.
+    // with the tile offset in the scalar operand.  Keys past T, of the last
+    // tile, are other bytes (the next head's keys, or what lies behind the
+    // cache: its buffers hold at least 63 more rows) and are never visible.
     const int8_t* Kg = a.kc + ((size_t)b * a.KH + g) * T * 64;
     const int8_t* Vg = a.vc + ((size_t)b * a.KH + g) * 64 * a.TP;
-    const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc((void*)Kg, (short)0, T * 64, BUF_DWORD3);
+    const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc((void*)Kg, (short)0, a.TP * 64, BUF_DWORD3);
     const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc((void*)Vg, (short)0, a.TP * 64, BUF_DWORD3);
     // key kperm<KT>(blk, row) = the row's base + 4 blk; V^T of dim row (+ 16
     // db), keys 16 grp .. +16 of the tile

@@ -27,8 +27,8 @@ CASES = [
     "tail 40 512 1024 1", "tail 40 512 704 1", "tail 40 384 1024 0", "tail 17 256 64 1", "tail 17 256 4096 1", "tail 4100 256 64 1",
     # whole-stream decode: feed-forwards short of its K steps
     "fused 3 384 1024", "fused 3 512 960", "fused 2 384 448", "fused 1 256 64",
-    # prefill attention of whole tiles
-    "attention 9 512 6", "attention 3 64 5",
+    # prefill attention: whole tiles, last tiles short of 64 and of 32 keys
+    "attention 9 512 6", "attention 3 64 5", "attention 3 100 4", "attention 2 93 6", "attention 1 1 5",
 ]
 
 
