@@ -417,18 +417,24 @@ void resolve_events(czip_ctx* c) {
     c->pending.clear();
 }
 
+void count_gemm(czip_ctx* c, GemmKernel k) {
+    if (!c->profiling) return;
+    if (k == GEMM_FEW_ROWS) c->stats["few_row_gemm"].launches++;
+    if (k == GEMM_WIDE) c->stats["wide_gemm"].launches++;
+}
+
 // the GEMM launches with the context's kernel switch
-void gemm(const czip_ctx* c, GemmArgs g, int epi, hipStream_t s) {
+void gemm(czip_ctx* c, GemmArgs g, int epi, hipStream_t s) {
     g.tiled = c->gemm_tiled ? 1 : 0;
     g.skinny_rows = c->skinny_rows;
     g.wide_rows = c->wide_rows;
-    launch_gemm(g, epi, s);
+    count_gemm(c, launch_gemm(g, epi, s));
 }
-void gemm_rn(const czip_ctx* c, RowGemmArgs a, hipStream_t s) {
+void gemm_rn(czip_ctx* c, RowGemmArgs a, hipStream_t s) {
     a.tiled = c->gemm_tiled ? 1 : 0;
     a.skinny_rows = c->skinny_rows;
     a.wide_rows = c->wide_rows;
-    launch_gemm_rn(a, s);
+    count_gemm(c, launch_gemm_rn(a, s));
 }
 
 czip_status check_config(czip_ctx* c, const czip_model_desc& w) {

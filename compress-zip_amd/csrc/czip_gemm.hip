@@ -758,20 +758,22 @@ static bool try_ws(const GemmArgs& a, hipStream_t s) {
     }
 }
 
-void launch_gemm(const GemmArgs& a, int epi, hipStream_t s) {
-    switch (epi) {
-        case EPI_RAW: if (try_skinny<EPI_RAW>(a, s) || try_ws<EPI_RAW>(a, s) || try_wide<EPI_RAW>(a, s)) return; break;
-        case EPI_REQ: if (try_skinny<EPI_REQ>(a, s) || try_ws<EPI_REQ>(a, s) || try_wide<EPI_REQ>(a, s)) return; break;
-        case EPI_QKV: if (try_skinny<EPI_QKV>(a, s) || try_ws<EPI_QKV>(a, s) || try_wide<EPI_QKV>(a, s)) return; break;
-        default: if (try_skinny<EPI_REGLU>(a, s) || try_ws<EPI_REGLU>(a, s) || try_wide<EPI_REGLU>(a, s)) return; break;
-    }
+template <int EPI>
+static GemmKernel launch_gemm_epi(const GemmArgs& a, hipStream_t s) {
+    if (try_skinny<EPI>(a, s)) return GEMM_FEW_ROWS;
+    if (try_ws<EPI>(a, s)) return GEMM_OTHER;
+    if (try_wide<EPI>(a, s)) return GEMM_WIDE;
     const int ntm = (a.M + BM - 1) / BM, ntn = (a.N + BN - 1) / BN;
-    dim3 grid((unsigned)(((ntm + NXCD - 1) / NXCD) * NXCD * ntn));
+    launch_epi<EPI>(a, dim3((unsigned)(((ntm + NXCD - 1) / NXCD) * NXCD * ntn)), s);
+    return GEMM_OTHER;
+}
+
+GemmKernel launch_gemm(const GemmArgs& a, int epi, hipStream_t s) {
     switch (epi) {
-        case EPI_RAW: launch_epi<EPI_RAW>(a, grid, s); break;
-        case EPI_REQ: launch_epi<EPI_REQ>(a, grid, s); break;
-        case EPI_QKV: launch_epi<EPI_QKV>(a, grid, s); break;
-        default: launch_epi<EPI_REGLU>(a, grid, s); break;
+        case EPI_RAW: return launch_gemm_epi<EPI_RAW>(a, s);
+        case EPI_REQ: return launch_gemm_epi<EPI_REQ>(a, s);
+        case EPI_QKV: return launch_gemm_epi<EPI_QKV>(a, s);
+        default: return launch_gemm_epi<EPI_REGLU>(a, s);
     }
 }
 
@@ -1183,7 +1185,7 @@ static void launch_rn(const RowGemmArgs& a, hipStream_t s) {
 
 // d = 64 h columns over NW waves of CT 16-wide tiles: 8 waves where h is even
 // (few accumulators per wave, many waves to hide the W stream's latency)
-void launch_gemm_rn(const RowGemmArgs& a, hipStream_t s) {
+GemmKernel launch_gemm_rn(const RowGemmArgs& a, hipStream_t s) {
     if (a.y8 && !a.tiled && a.M > 0 && a.M <= a.skinny_rows) {
         // few rows: the product over the whole chip, then the norms a wavefront per row
         GemmArgs g{};
@@ -1191,7 +1193,7 @@ void launch_gemm_rn(const RowGemmArgs& a, hipStream_t s) {
         g.mult = a.mult; g.shift = a.shift; g.rq_scale = a.rq_scale; g.rq_fast = a.rq_fast; g.skinny_rows = a.skinny_rows;
         if (try_skinny<EPI_REQ>(g, s)) {
             launch_rn_rows(a, s);
-            return;
+            return GEMM_FEW_ROWS;
         }
     }
     if (a.y8 && !a.tiled && a.d >= 768 && a.M >= 2 * a.wide_rows) {
@@ -1209,12 +1211,12 @@ void launch_gemm_rn(const RowGemmArgs& a, hipStream_t s) {
         g.mult = a.mult; g.shift = a.shift; g.rq_scale = a.rq_scale; g.rq_fast = a.rq_fast; g.wide_rows = a.wide_rows;
         if (try_wide<EPI_REQ>(g, s)) {
             launch_rn_rows(a, s);
-            return;
+            return GEMM_WIDE;
         }
     }
     if (!a.tiled && a.d == 384 && a.M > 0 && (long long)a.M * a.K < (1ll << 40) && !use_rn16(a)) {
-        if (a.K == 384) { launch_rn_ws<8, 3, 6>(a, s); return; }
-        if (a.K == 512) { launch_rn_ws<8, 3, 8>(a, s); return; }
+        if (a.K == 384) { launch_rn_ws<8, 3, 6>(a, s); return GEMM_OTHER; }
+        if (a.K == 512) { launch_rn_ws<8, 3, 8>(a, s); return GEMM_OTHER; }
     }
     switch (a.d / 64) {
         case 4: launch_rn<8, 2>(a, s); break;
@@ -1227,6 +1229,7 @@ void launch_gemm_rn(const RowGemmArgs& a, hipStream_t s) {
         case 14: launch_rn<8, 7>(a, s); break;
         default: launch_rn<16, 4>(a, s); break;
     }
+    return GEMM_OTHER;
 }
 
 }  // namespace czip

@@ -42,6 +42,9 @@ struct GemmArgs {
     int skinny_rows = 0, wide_rows = 0;
 };
 
+// the kernel that a GEMM launch took, for the context's launch counts
+enum GemmKernel { GEMM_OTHER, GEMM_FEW_ROWS, GEMM_WIDE };
+
 // The attention's exp table by table step t (exp_q16, lut.rs:213-235):
 // E(t) = max(1, ((lut[t % 256] << 16 >> (t / 256)) + 2^15) >> 16) for
 // t < 4096, and entry 4096 stands for every larger step (a shift by 16 or more
@@ -111,7 +114,7 @@ size_t gemm_rn_ws_bytes(int M, int d);
 // the row GEMM's epilogue from the requantized projection a.y8
 void launch_rn_rows(const RowGemmArgs& a, hipStream_t s);
 void launch_rn_splitk_epi(const RowGemmArgs& a, const int32_t* part, int splits, hipStream_t s);
-void launch_gemm_rn(const RowGemmArgs& a, hipStream_t s);
+GemmKernel launch_gemm_rn(const RowGemmArgs& a, hipStream_t s);
 
 // The FFN of one layer in one kernel (model.rs:438-468 from the pre-FFN norm's
 // output): xn_out = rmsnorm(clamp(x), w2) with x = x_in + rmsnorm(requant(
@@ -178,7 +181,7 @@ void launch_embed_norm(const uint32_t* inp, const int8_t* embed, const int8_t* w
                        int16_t* x, int8_t* xn, hipStream_t s);
 void launch_resid_norm(int16_t* x, const int8_t* y8, const int8_t* w1, const int8_t* w2, int M, int d,
                        int8_t* xn, hipStream_t s);
-void launch_gemm(const GemmArgs& a, int epi, hipStream_t s);
+GemmKernel launch_gemm(const GemmArgs& a, int epi, hipStream_t s);
 void launch_attention(const AttnArgs& a, int B, hipStream_t s);
 // mode 0: (lo, hi) of targets; mode 1: full inclusive cumfreqs; mode 2:
 // targets are decoder values, out rows (sym, cum_lo, cum_hi).  Row r of the

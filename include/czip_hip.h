@@ -263,10 +263,13 @@ void        czip_buffer_free(void* p);
 /* ---- instrumentation: per-kernel HIP-event timing on the context stream. ---- */
 void        czip_set_profiling(czip_ctx* ctx, int32_t on);
 /* Kernel names: "prep","embed_norm","gemm_qkv","attention","gemm_o_norm",
- * "gemm_up","gemm_down_norm","head_cdf","encode"; where a fused kernel has no
+ * "gemm_up","gemm_down_norm","head_cdf","encode", "ffn" or "layer_tail" for a
+ * layer's FFN, or all of it after the attention, in one launch; where a fused kernel has no
  * instance for the model shape: "gemm_o","gemm_down","row_norm","gemm_head",
  * "cdf"; decode: "dec_init","dec_prep","attn_decode","head_dec" (or, unfused,
- * "gemm_head","cdf_decode"), or "dec_fused" for every step in one launch. */
+ * "gemm_head","cdf_decode"), or "dec_fused" for every step in one launch.
+ * "few_row_gemm" and "wide_gemm" count the GEMMs among them (under the names
+ * above, with their time) that ran by the few-row kernel or in 128 x 256 tiles. */
 czip_status czip_kernel_stats(czip_ctx* ctx, const char* name, int64_t* launches, double* total_ms);
 void        czip_reset_stats(czip_ctx* ctx);
 

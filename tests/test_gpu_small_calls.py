@@ -126,8 +126,12 @@ def test_few_row_gemms(amd, orc, tmp_path, heads, kv, d_ff):
                                     d_ff=d_ff, vocab=1088, ctx=600, seed=300 + heads)
     gm = amd.Model(amd.ModelWeights(path, amd.KV_GQA))
     om = orc.Model.from_file(path, amd.KV_GQA)
+    gm.set_profiling(True)
     for lens in ([1], [16], [17], [63], [32, 32], [13, 5, 13, 13, 13], [129], [256], [257], [512], [513]):
+        seen = gm.kernel_stats("few_row_gemm")[0]
         parity._check_logits(gm, om, max(lens), lens, 7 + len(lens), 1088)
+        if max(lens) <= 512:  # QKV of the second layer, O, up and down of both, and the head up to 256 rows
+            assert gm.kernel_stats("few_row_gemm")[0] - seen == (8 if len(lens) * max(lens) <= 256 else 7)
 
 
 # The whole-stream decode kernel (one-layer models, V = 1024).  Up to 256
@@ -219,12 +223,18 @@ def test_row_gemm_16_without_tail(amd, shipped, monkeypatch):
     parity.test_small_launch_row_gemm(gm, shipped, 4, 512)
 
 
-@pytest.mark.parametrize("heads,kv,d_ff,vocab", [(12, 4, 448, 1088), (10, 5, 192, 1024), (14, 2, 832, 2112), (8, 1, 1024, 1024)])
-def test_wide_gemms(amd, orc, tmp_path, monkeypatch, heads, kv, d_ff, vocab):
+# projections of a layer that take the 128 x 256 tiles: QKV (not layer 0's,
+# which comes from the table) and up of two layers, the head, and O and down
+# where their own rule (d >= 768 with a row kernel) or the lack of a row
+# kernel (11 and 13 heads) sends them there
+@pytest.mark.parametrize("heads,kv,d_ff,vocab,per_pass", [
+    (12, 4, 192, 1088, 8), (14, 2, 832, 2112, 8), (11, 1, 448, 1024, 8), (13, 13, 320, 1088, 8), (10, 5, 192, 1024, 4)])
+def test_wide_gemms(amd, orc, tmp_path, monkeypatch, heads, kv, d_ff, vocab, per_pass):
     """The 128 x 256 tiles at row counts around their row blocks, for column
-    counts with a partial last tile and odd and even numbers of K steps (3, 7,
-    10, 13 and 14 of 64 among them), over ragged chunks; the norms behind them
-    where the row count asks for them."""
+    counts with a partial last tile and numbers of K steps of 64 odd and even:
+    10 to 14 for QKV, ReGLU and the head (11 and 13 among them), 3, 5, 7 and 13
+    for the down projection, over ragged chunks; the norms behind them where
+    the row count asks for them."""
     import test_gpu_parity as parity
     from czip_amd import synth
     path = synth.write_random_model(str(tmp_path / "w.czm"), d=64 * heads, n_layers=2, n_heads=heads, n_kv=kv,
@@ -234,8 +244,13 @@ def test_wide_gemms(amd, orc, tmp_path, monkeypatch, heads, kv, d_ff, vocab):
     monkeypatch.setenv("CZIP_WIDE_ROWS", "1")
     gm = amd.Model(amd.ModelWeights(path, amd.KV_GQA))
     om = orc.Model.from_file(path, amd.KV_GQA)
+    gm.set_profiling(True)
     for lens in ([1], [127], [64, 64], [129], [513], [200, 31, 200, 200]):
+        seen = gm.kernel_stats("wide_gemm")[0]
         parity._check_logits(gm, om, max(lens), lens, 11 + len(lens), vocab)
+        # (the row kernels' rule asks for twice the rows: one row is too few)
+        n = per_pass if per_pass == 4 or heads in (11, 13) or len(lens) * max(lens) >= 2 else 4
+        assert gm.kernel_stats("wide_gemm")[0] - seen == n
 
 
 @pytest.mark.parametrize("vocab,env", [(1024, "CZIP_UNFUSED_HEAD"), (1088, None), (4096, None), (4160, None), (8192, None)])
