@@ -1,5 +1,8 @@
-"""GPU parity of the kernels whose sizes a small call decides, against the
-oracle: the arithmetic encoder's load groups."""
+"""GPU parity of the kernels that a call's size chooses, at the sizes around
+their limits, against the oracle: the arithmetic encoder's load groups, decode
+attention by rows, few-row GEMMs, whole-stream decode, layer tail, 128 x 256
+tiles and the wave counts of the unfused decoder step; and device memory that
+jobs hand on."""
 import numpy as np
 import pytest
 
@@ -81,9 +84,38 @@ def test_job_memory_threads(amd, pair):
     assert not bad
 
 
-# Decode steps of few rows take the one-row-per-wave attention kernel, which
-# every other decode test of a few streams therefore runs; here the same edge
-# cases through the kernel that packs streams or heads into a wave's rows.
+# Decode steps of few rows take the one-row-per-wave attention kernel; one-layer
+# models of 1024 tokens decode as a whole instead (CZIP_DECODE_FUSED=0: step by
+# step).  The attention's edge cases through the row kernel, and through the
+# kernel that packs streams or heads into a wave's rows (CZIP_ATTN_ROWS=0).
+def test_decode_attention_row_edge_cases(amd, orc, tmp_path, monkeypatch):
+    import test_gpu_parity as parity
+    monkeypatch.setenv("CZIP_DECODE_FUSED", "0")
+    parity.test_decompress_attention_edge_cases(amd, orc, tmp_path)
+
+
+@pytest.mark.parametrize("sink", [False, True])
+@pytest.mark.parametrize("kv,n_kv", [("rust", 1), ("gqa", 2)])
+def test_decode_attention_row_general(amd, orc, tmp_path, sink, kv, n_kv):
+    """Two layers whose scores pass 2^30 and wrap in their differences, an exp
+    table whose first entry is not 65535, with and without a sink."""
+    from test_gpu_parity import _write_model
+    from czip_amd import synth
+    t, meta = synth.random_model_tensors(d=256, n_layers=2, n_heads=4, n_kv=n_kv, d_ff=128, vocab=1024, ctx=256,
+                                         seed=430 + n_kv, sink=sink)
+    for l in range(2):
+        t[f"layers.{l}.attn.score_mult"] = np.array([1 << 30, -(1 << 30), 1 << 27, -5], np.int32)
+    t["lut.exp2"][0] = 65000
+    path = _write_model(str(tmp_path / "g.czm"), t, meta)
+    mode = amd.KV_GQA if kv == "gqa" else amd.KV_RUST_COMPAT
+    gm, om = amd.Model(amd.ModelWeights(path, mode)), orc.Model.from_file(path, mode)
+    gm.set_profiling(True)
+    toks = synth.zipf_ids(3 * 150 - 41, 1024, seed=431)
+    chunks = om.compress_many(toks, 150, threads=4)
+    assert np.array_equal(gm.decompress_chunks(chunks, [150, 150, 109]), toks)
+    assert gm.kernel_stats("dec_fused")[0] == 0 and gm.kernel_stats("attn_decode")[0] == 2 * 150
+
+
 def test_decode_attention_tile_edge_cases(amd, orc, tmp_path, monkeypatch):
     import test_gpu_parity as parity
     monkeypatch.setenv("CZIP_ATTN_ROWS", "0")
@@ -104,14 +136,21 @@ def test_decode_attention_tile_random_shapes(orc, tmp_path, monkeypatch, i):
 
 
 @pytest.mark.parametrize("n", [1, 3, 4, 5, 63, 64, 65, 128, 129])
-def test_decode_attention_rows_key_counts(pair, n):
+def test_decode_attention_rows_key_counts(amd, pair, monkeypatch, n):
     """Key counts around the 4-key blocks and the 64-key tiles, and stream
-    counts around a workgroup's four rows."""
-    gm, om = pair
+    counts around a workgroup's four rows: step by step, and the whole-stream
+    kernel's own rows."""
+    _, om = pair
     toks = np.random.default_rng(100 + n).integers(0, 1024, 3 * n).astype(np.uint32)
     chunks = om.compress_many(toks, n, threads=4)
-    for s in (1, 2, 3):
-        assert np.array_equal(gm.decompress_chunks(chunks[:s], [n] * s), toks[:s * n])
+    for fused in (0, 4096):
+        monkeypatch.setenv("CZIP_DECODE_FUSED", str(fused))
+        gm = amd.Model(amd.ModelWeights(MODEL_PATH))
+        gm.set_profiling(True)
+        for s in (1, 2, 3):
+            assert np.array_equal(gm.decompress_chunks(chunks[:s], [n] * s), toks[:s * n])
+        assert gm.kernel_stats("dec_fused")[0] == (3 if fused else 0)
+        assert gm.kernel_stats("attn_decode")[0] == (0 if fused else 3 * n)
 
 
 @pytest.mark.parametrize("heads,kv,d_ff", [(1, 1, 64), (5, 1, 1600), (6, 2, 128), (14, 7, 832), (16, 4, 3136)])
@@ -221,6 +260,29 @@ def test_row_gemm_16_without_tail(amd, shipped, monkeypatch):
     monkeypatch.setenv("CZIP_TAIL_ROWS", "0")
     gm = amd.Model(amd.ModelWeights(MODEL_PATH))
     parity.test_small_launch_row_gemm(gm, shipped, 4, 512)
+
+
+# The kernels of more rows at launches that the few-row GEMMs, the layer tail
+# and the whole-stream decode take by default: the shapes of the random-shape
+# tests, and decode steps on both sides of the 16-row row GEMM's least rows
+@pytest.mark.parametrize("i", [1, 5, 9, 13, 19, 24, 27, 33, 39, 44, 52, 61, 69, 74, 80, 88])
+def test_random_shapes_many_row_kernels(orc, tmp_path, monkeypatch, i):
+    import test_gpu_random_shapes as shapes
+    monkeypatch.setenv("CZIP_SKINNY_ROWS", "0")
+    monkeypatch.setenv("CZIP_TAIL_ROWS", "0")
+    shapes.test_random_shape_roundtrip(orc, tmp_path, monkeypatch, i)
+
+
+@pytest.mark.parametrize("n_chunks", [1600, 369, 368])
+def test_decode_steps_many_row_kernels(amd, shipped, monkeypatch, n_chunks):
+    import test_gpu_parity as parity
+    monkeypatch.setenv("CZIP_SKINNY_ROWS", "0")
+    monkeypatch.setenv("CZIP_TAIL_ROWS", "0")
+    gm = amd.Model(amd.ModelWeights(MODEL_PATH))
+    gm.set_profiling(True)
+    parity.test_small_launch_row_gemm(gm, shipped, n_chunks, 64)
+    for name in ("dec_fused", "layer_tail", "few_row_gemm"):
+        assert gm.kernel_stats(name)[0] == 0
 
 
 # projections of a layer that take the 128 x 256 tiles: QKV (not layer 0's,
