@@ -461,12 +461,15 @@ __global__ __launch_bounds__(256, 2) void k_gemm_ws(GemmArgs a, int ncg) {
 // ReGLU 16.4 -> 10.8 ms (1.4 -> 2.1 POP/s), QKV 4.3 -> 3.1, head (V = 8192) 2.7 ->
 // 2.2; 4096 rows: up 0.42 -> 0.35, QKV 0.19 -> 0.22; 2048 rows 0.26 -> 0.29 and
 // 0.16 -> 0.20.  (K = 512: the W-stationary kernel is faster, up 14.9 against 18.4
-// ms at a million rows.)
+// ms at a million rows.)  Fast requantization only (try_wide).  A whole pass of 2
+// layers, 4096 / 65536 rows: d640 449 -> 443 us / 2.33 -> 2.12 ms, d704 511 -> 488
+// / 2.75 -> 2.36, d768 487 -> 474 / 2.90 -> 2.31, d896 543 -> 532 / 3.62 -> 2.86,
+// d1024 586 -> 566 / 4.12 -> 3.27.
 // ---------------------------------------------------------------------------
 constexpr int WIDE_BM = 128, WIDE_BN = 256;
 constexpr int WIDE_GROUP = 8;  // row blocks an XCD takes through all columns at a time
 
-template <int EPI, bool FAST>
+template <int EPI>
 __global__ __launch_bounds__(256, 2) void k_gemm_wide(GemmArgs a) {
     __shared__ __attribute__((aligned(16))) int8_t As[2][WIDE_BM * 64];
     const int tid = threadIdx.x, lane = tid & 63, lr = lane & 15, c4 = (lane >> 4) * 4;
@@ -564,13 +567,13 @@ __global__ __launch_bounds__(256, 2) void k_gemm_wide(GemmArgs a) {
         QkvRow qr;
         if (EPI == EPI_QKV) qkv_row(a, row, c4, qr);
         if (EPI != EPI_QKV || role == 0) {
-            epi_ws<EPI, FAST, 0>(a, ro, acc[i], row, col_base, c4, qr, g, t);
+            epi_ws<EPI, true, 0>(a, ro, acc[i], row, col_base, c4, qr, g, t);
             flush_ws<EPI, 0>(ro, t);
         } else if (role == 1) {
-            epi_ws<EPI, FAST, 1>(a, ro, acc[i], row, col_base, c4, qr, g, t);
+            epi_ws<EPI, true, 1>(a, ro, acc[i], row, col_base, c4, qr, g, t);
             flush_ws<EPI, 1>(ro, t);
         } else {
-            epi_ws<EPI, FAST, 2>(a, ro, acc[i], row, col_base, c4, qr, g, t);
+            epi_ws<EPI, true, 2>(a, ro, acc[i], row, col_base, c4, qr, g, t);
             flush_ws<EPI, 2>(ro, t);
         }
     }
@@ -578,6 +581,10 @@ __global__ __launch_bounds__(256, 2) void k_gemm_wide(GemmArgs a) {
 
 template <int EPI>
 static bool try_wide(const GemmArgs& a, hipStream_t s) {
+    // only the fast requantization: the general one's 64-bit arithmetic on 128
+    // accumulators a lane spills (2 layers, d640 4096 rows 508 -> 578 us, d768 65
+    // thousand 3.38 -> 3.75 ms, d1024 4.61 -> 5.17)
+    if (EPI != EPI_RAW && !a.rq_fast) return false;
     if (a.tiled || !a.Wf || a.a_rows || a.M < a.wide_rows || a.N % 64 != 0 || (long long)a.N * a.K >= (1ll << 31) - (1 << 20) ||
         (long long)WIDE_BM * a.K >= (1ll << 31) || (long long)WIDE_BM * a.ldo * (EPI == EPI_RAW ? 4 : 1) >= (1ll << 31))
         return false;
@@ -586,8 +593,7 @@ static bool try_wide(const GemmArgs& a, hipStream_t s) {
     const int ntm = (a.M + WIDE_BM - 1) / WIDE_BM, ntn = (a.N + WIDE_BN - 1) / WIDE_BN;
     const int groups = (ntm + NXCD * WIDE_GROUP - 1) / (NXCD * WIDE_GROUP);
     const dim3 grid((unsigned)(groups * WIDE_GROUP * NXCD * ntn));
-    if (a.rq_fast) hipLaunchKernelGGL((k_gemm_wide<EPI, true>), grid, dim3(256), 0, s, a);
-    else hipLaunchKernelGGL((k_gemm_wide<EPI, false>), grid, dim3(256), 0, s, a);
+    hipLaunchKernelGGL((k_gemm_wide<EPI>), grid, dim3(256), 0, s, a);
     return true;
 }
 

@@ -315,6 +315,25 @@ def test_wide_gemms(amd, orc, tmp_path, monkeypatch, heads, kv, d_ff, vocab, per
         assert gm.kernel_stats("wide_gemm")[0] - seen == n
 
 
+def test_general_requantization_leaves_the_wide_tiles(amd, orc, tmp_path, monkeypatch):
+    """Projections off the fast requantization path (|mult| >= 2^26) keep the
+    128 x 128 tiles, which are faster there; the head has none and does not."""
+    import test_gpu_parity as parity
+    from czip_amd import synth
+    t, meta = synth.random_model_tensors(d=768, n_layers=2, n_heads=12, n_kv=4, d_ff=192, vocab=1088, ctx=600, seed=650)
+    for l in range(2):
+        for nm in ("attn.qkv", "attn.out", "ffn.up", "ffn.down"):
+            t[f"layers.{l}.{nm}.mult"] = np.array(int(t[f"layers.{l}.{nm}.mult"]) << 17, np.int32)
+            t[f"layers.{l}.{nm}.shift"] = np.array(int(t[f"layers.{l}.{nm}.shift"]) + 17, np.int8)
+    path = parity._write_model(str(tmp_path / "g.czm"), t, meta)
+    monkeypatch.setenv("CZIP_SKINNY_ROWS", "0")
+    monkeypatch.setenv("CZIP_WIDE_ROWS", "1")
+    gm, om = parity._model_pair(amd, orc, path, amd.KV_GQA)
+    gm.set_profiling(True)
+    parity._check_logits(gm, om, 200, [200, 31], 651, 1088)
+    assert gm.kernel_stats("wide_gemm")[0] == 1
+
+
 @pytest.mark.parametrize("vocab,env", [(1024, "CZIP_UNFUSED_HEAD"), (1088, None), (4096, None), (4160, None), (8192, None)])
 def test_decode_step_wave_counts(amd, orc, tmp_path, monkeypatch, vocab, env):
     """The unfused head's decoder step with a row's logits over one, four and
