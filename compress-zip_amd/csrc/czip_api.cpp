@@ -56,9 +56,19 @@ constexpr size_t TAIL_WEIGHTS_MAX = (size_t)4 << 20, TAIL_WEIGHT_BYTES_PER_ROW =
 // takes over below it.  A step-wise decode step, other kernels -> these: d768
 // 513 streams 1141 -> 768 us, 768 1134 -> 970, 1024 1175 -> 1078; d512 513
 // 470 -> 380, 768 485 -> 429, 1024 496 -> 490; v001, against the tail, 513
-// 106 -> 106, 768 102 -> 110.  Compressing as many tokens in chunks of 256: d512
-// 520 732 -> 677, 1024 740 -> 723 us; d768 520 1271 -> 1253, 1024 1292 -> 1327
-constexpr int SKINNY_ROWS_MAX = 1024;
+// 106 -> 106, 768 102 -> 110.
+// Past SKINNY_WIDE_ROWS rows the 16-row row GEMM of a model of SKINNY_WIDE_D or
+// wider is ahead where the weights lie in a cache: in a prefill, whose layers
+// follow each other at once, and in decode steps of models whose weights are
+// small.  Compressing in chunks of 256, other kernels -> these: d512 (8 layers)
+// 768 tokens 655 -> 597 us, 1024 662 -> 650; d768 (12) 768 1198 -> 1163, 896 1203
+// -> 1252, 1024 1201 -> 1250; d640 (2) 768 248 -> 237, 1024 248 -> 258; d1024 (2)
+// 321 -> 307, 323 -> 349; d704 (2, no row GEMM) 288 -> 261, 292 -> 271.  Decode
+// steps of 800 and 1024 streams: d640 (12 layers, 71 MB) 920 -> 795, 883 -> 878
+// us; d1024 (12) 1419 -> 1289, 1459 -> 1454; d768 (2 layers, 17 MB) 212 -> 208, 224
+// -> 231; d1024 (2, 31 MB) 1024 streams 264 -> 289
+constexpr int SKINNY_ROWS_MAX = 1024, SKINNY_WIDE_ROWS = 768, SKINNY_WIDE_D = 640;
+constexpr size_t SKINNY_SMALL_WEIGHTS = (size_t)48 << 20;
 // GEMMs of at least this many rows, where no W-stationary kernel takes them,
 // run 128 x 256 tiles with the weights straight from L2 (CZIP_WIDE_ROWS)
 constexpr int WIDE_ROWS_MIN = 4096;
@@ -228,7 +238,8 @@ struct czip_ctx {
     double scratch_gb = 0;        // CZIP_SCRATCH_GB: a job's scratch budget
     int64_t decode_streams = 0;   // CZIP_DECODE_STREAMS: most streams per decode group (0: no cap)
     long long attn_rows = ATTN_ROWS_MAX;  // CZIP_ATTN_ROWS
-    int skinny_rows = SKINNY_ROWS_MAX;    // CZIP_SKINNY_ROWS
+    // most rows of the few-row GEMMs in a prefill and in a decode step (CZIP_SKINNY_ROWS: both)
+    int skinny_rows_prefill = SKINNY_ROWS_MAX, skinny_rows_decode = SKINNY_ROWS_MAX;
     int wide_rows = WIDE_ROWS_MIN;        // CZIP_WIDE_ROWS
     int64_t tail_rows = 0;        // most and least rows of a launch whose layers end in the tail
     int64_t tail_rows_min = 0;    // kernel (most 0: never)
@@ -260,7 +271,7 @@ struct czip_ctx {
 
 struct czip_job {
     czip_ctx* ctx = nullptr;
-    int kind = 0;  // 0 compress
+    int kind = 0;  // 0 prefill (compress, rows in and out), 1 decompress, 2 decode session
     int64_t n_tokens = 0, nchunks = 0;
     int T = 0, BC = 0;
     int64_t slot = 0;
@@ -423,16 +434,17 @@ void count_gemm(czip_ctx* c, GemmKernel k) {
     if (k == GEMM_WIDE) c->stats["wide_gemm"].launches++;
 }
 
-// the GEMM launches with the context's kernel switch
-void gemm(czip_ctx* c, GemmArgs g, int epi, hipStream_t s) {
+// the GEMM launches with the context's kernel switches; skinny_rows: the pass's
+// limit of the few-row kernel (0: never)
+void gemm(czip_ctx* c, GemmArgs g, int epi, int skinny_rows, hipStream_t s) {
     g.tiled = c->gemm_tiled ? 1 : 0;
-    g.skinny_rows = c->skinny_rows;
+    g.skinny_rows = skinny_rows;
     g.wide_rows = c->wide_rows;
     count_gemm(c, launch_gemm(g, epi, s));
 }
-void gemm_rn(czip_ctx* c, RowGemmArgs a, hipStream_t s) {
+void gemm_rn(czip_ctx* c, RowGemmArgs a, int skinny_rows, hipStream_t s) {
     a.tiled = c->gemm_tiled ? 1 : 0;
-    a.skinny_rows = c->skinny_rows;
+    a.skinny_rows = skinny_rows;
     a.wide_rows = c->wide_rows;
     count_gemm(c, launch_gemm_rn(a, s));
 }
@@ -566,7 +578,6 @@ extern "C" czip_status czip_create(const czip_model_desc* w, int device, czip_ct
     if (const char* e = getenv("CZIP_DECODE_STREAMS")) c->decode_streams = std::max(1ll, atoll(e));
     if (const char* e = getenv("CZIP_ATTN_ROWS")) c->attn_rows = std::max(0ll, atoll(e));
     if (const char* e = getenv("CZIP_WIDE_ROWS")) c->wide_rows = std::max(1, atoi(e));
-    if (const char* e = getenv("CZIP_SKINNY_ROWS")) c->skinny_rows = std::max(0, atoi(e));
     if (const char* e = getenv("CZIP_DECODE_LANES")) {
         const int n = atoi(e);
         if (n >= 1 && n <= DEC_LANES_MAX) c->decode_lanes = n;
@@ -606,7 +617,12 @@ extern "C" czip_status czip_create(const czip_model_desc* w, int device, czip_ct
         }
         c->tail_rows = ok ? TAIL_ROWS_MAX : 0;
         c->tail_rows_min = (int64_t)(d * (qn + d + 3 * F) / TAIL_WEIGHT_BYTES_PER_ROW);
-        if (ok && c->tail_rows_min < SKINNY_ROWS_MAX && getenv("CZIP_SKINNY_ROWS") == nullptr) c->skinny_rows = SKINNY_ROWS_MAX / 2;
+        if (c->rn_fused && w->d_model >= SKINNY_WIDE_D) {
+            c->skinny_rows_prefill = SKINNY_WIDE_ROWS;
+            if (d * (qn + d + 3 * F) * (size_t)w->n_layers <= SKINNY_SMALL_WEIGHTS) c->skinny_rows_decode = SKINNY_WIDE_ROWS;
+        }
+        if (ok && c->tail_rows_min < SKINNY_ROWS_MAX) c->skinny_rows_prefill = c->skinny_rows_decode = SKINNY_ROWS_MAX / 2;
+        if (const char* e = getenv("CZIP_SKINNY_ROWS")) c->skinny_rows_prefill = c->skinny_rows_decode = std::max(0, atoi(e));
         if (const char* e = getenv("CZIP_TAIL_ROWS")) c->tail_rows = ok ? std::max(0ll, atoll(e)) : 0;
     }
     czip_ctx* C = c.get();
@@ -681,7 +697,7 @@ extern "C" czip_status czip_create(const czip_model_desc* w, int device, czip_ct
         GemmArgs g{};
         g.A = c->embed_xn; g.W = L0.qkv_w; g.M = (int)V; g.N = L0.qkv_n; g.K = (int)d;
         g.out8 = c->qkv_tab; g.ldo = L0.qkv_n; set_requant(g, L0.qkv_mult, L0.qkv_shift);
-        gemm(C, g, EPI_REQ, c->stream);
+        gemm(C, g, EPI_REQ, 0, c->stream);
         HIPCHECK(C, hipGetLastError());
         HIPCHECK(C, hipStreamSynchronize(c->stream));
     }
@@ -785,6 +801,7 @@ struct RowBufs {
     int8_t *xn, *q8, *attn, *y8, *r8;
     int32_t* rn_ws;
     size_t rn_ws_bytes;
+    int skinny_rows;  // the pass's limit of the few-row GEMMs
 };
 
 RowBufs row_bufs(const czip_ctx* c, const czip_job* j, int64_t r0 = 0, int ws_parts = 1, int ws_part = 0) {
@@ -792,7 +809,8 @@ RowBufs row_bufs(const czip_ctx* c, const czip_job* j, int64_t r0 = 0, int ws_pa
     const size_t wb = j->rn_ws_bytes / (size_t)ws_parts / 16 * 16;
     return RowBufs{j->inp + r, j->x + r * d, j->xn + r * d, j->q8 + r * d, j->attn + r * d,
                    j->y8 ? j->y8 + r * d : nullptr, j->r8 ? j->r8 + r * F : nullptr,
-                   j->rn_ws ? j->rn_ws + wb / 4 * (size_t)ws_part : nullptr, wb};
+                   j->rn_ws ? j->rn_ws + wb / 4 * (size_t)ws_part : nullptr, wb,
+                   j->kind == 0 ? c->skinny_rows_prefill : c->skinny_rows_decode};
 }
 
 // next_qkv: the next layer's Q/K/V projection of a decode step (or nullptr);
@@ -803,7 +821,7 @@ bool post_attention(czip_ctx* c, const RowBufs& r, int l, int M, hipStream_t s, 
     const DevLayer& L = c->layers[(size_t)l];
     const bool last = l + 1 == c->cfg.n_layers;
     const int8_t* next = last ? c->final_norm : c->layers[(size_t)l + 1].attn_norm;
-    if (M > c->skinny_rows && M >= c->tail_rows_min && M <= c->tail_rows) {
+    if (M > r.skinny_rows && M >= c->tail_rows_min && M <= c->tail_rows) {
         GemmArgs o{}, u{}, dn{};  // requantization scales (the fast path, checked at czip_create)
         o.K = d; set_requant(o, L.out_mult, L.out_shift);
         u.K = d; set_requant(u, L.up_mult, L.up_shift);
@@ -827,12 +845,12 @@ bool post_attention(czip_ctx* c, const RowBufs& r, int l, int M, hipStream_t s, 
         o.w1 = L.ffn_norm; o.w2 = L.post_attn_norm;
         o.x_in = l == 0 ? nullptr : r.x; o.tok = r.inp; o.embed = c->embed;
         o.x_out = r.x; o.xn = r.xn; o.ws = r.rn_ws; o.ws_bytes = r.rn_ws_bytes; o.y8 = r.y8;
-        { Timed t(c, "gemm_o_norm"); gemm_rn(c, o, s); }
+        { Timed t(c, "gemm_o_norm"); gemm_rn(c, o, r.skinny_rows, s); }
     } else {
         GemmArgs o{};
         o.A = r.attn; o.W = L.out_w; o.Wf = L.out_wf; o.M = M; o.N = d; o.K = d; o.out8 = r.y8; o.ldo = d;
         set_requant(o, L.out_mult, L.out_shift);
-        { Timed t(c, "gemm_o"); gemm(c, o, EPI_REQ, s); }
+        { Timed t(c, "gemm_o"); gemm(c, o, EPI_REQ, r.skinny_rows, s); }
         { Timed t(c, "row_norm"); launch_resid_norm(r.x, r.y8, L.ffn_norm, L.post_attn_norm, M, d, r.xn, s); }
     }
     // the fused FFN walks 128-row strips with one workgroup per CU: it pays
@@ -856,19 +874,19 @@ bool post_attention(czip_ctx* c, const RowBufs& r, int l, int M, hipStream_t s, 
     GemmArgs u{};
     u.A = r.xn; u.W = L.up_w; u.Wf = L.up_wf; u.M = M; u.N = 2 * F; u.K = d; u.out8 = r.r8; u.ldo = F;
     set_requant(u, L.up_mult, L.up_shift);
-    { Timed t(c, "gemm_up"); gemm(c, u, EPI_REGLU, s); }
+    { Timed t(c, "gemm_up"); gemm(c, u, EPI_REGLU, r.skinny_rows, s); }
     if (c->rn_fused) {
         RowGemmArgs dn{};
         dn.A = r.r8; dn.W = L.down_w; dn.Wf = L.down_wf; dn.M = M; dn.K = F; dn.d = d;
         set_requant(dn, L.down_mult, L.down_shift);
         dn.w1 = L.post_ffn_norm; dn.w2 = next;
         dn.x_in = r.x; dn.x_out = last ? nullptr : r.x; dn.xn = r.xn; dn.ws = r.rn_ws; dn.ws_bytes = r.rn_ws_bytes; dn.y8 = r.y8;
-        { Timed t(c, "gemm_down_norm"); gemm_rn(c, dn, s); }
+        { Timed t(c, "gemm_down_norm"); gemm_rn(c, dn, r.skinny_rows, s); }
     } else {
         GemmArgs dn{};
         dn.A = r.r8; dn.W = L.down_w; dn.Wf = L.down_wf; dn.M = M; dn.N = d; dn.K = F; dn.out8 = r.y8; dn.ldo = d;
         set_requant(dn, L.down_mult, L.down_shift);
-        { Timed t(c, "gemm_down"); gemm(c, dn, EPI_REQ, s); }
+        { Timed t(c, "gemm_down"); gemm(c, dn, EPI_REQ, r.skinny_rows, s); }
         { Timed t(c, "row_norm"); launch_resid_norm(r.x, r.y8, L.post_ffn_norm, next, M, d, r.xn, s); }
     }
     return false;
@@ -905,7 +923,7 @@ void layer0_qkv(czip_ctx* c, GemmArgs& g, const uint32_t* tok, hipStream_t s) {
     }
     g.A = c->embed_xn; g.a_rows = tok; g.a_nrows = c->cfg.vocab;
     Timed t(c, "gemm_qkv");
-    gemm(c, g, EPI_QKV, s);
+    gemm(c, g, EPI_QKV, 0, s);
 }
 
 // Run every layer on rows [0, nb*T) whose inputs are j->inp / j->lens; leaves
@@ -930,7 +948,7 @@ czip_status forward_batch(czip_ctx* c, czip_job* j, int nb, int T, bool head = t
             layer0_qkv(c, g, j->inp, s);
         } else {
             Timed t(c, "gemm_qkv");
-            gemm(c, g, EPI_QKV, s);
+            gemm(c, g, EPI_QKV, c->skinny_rows_prefill, s);
         }
         AttnArgs a{};
         a.q = j->q8; a.kc = j->kc; a.vc = j->vc; a.TP = pad64(T); a.lens = j->lens; a.score_mult = L.score_mult;
@@ -944,7 +962,7 @@ czip_status forward_batch(czip_ctx* c, czip_job* j, int nb, int T, bool head = t
         GemmArgs h{};
         h.A = j->xn; h.W = c->head_w; h.Wf = c->head_wf; h.M = M; h.N = V; h.K = d; h.out32 = j->logits; h.ldo = V;
         Timed t(c, "gemm_head");
-        gemm(c, h, EPI_RAW, s);
+        gemm(c, h, EPI_RAW, c->skinny_rows_prefill, s);
     }
     return CZIP_OK;
 }
@@ -1412,7 +1430,7 @@ static czip_status run_decompress(czip_job* j) {
                         layer0_qkv(c, g, Ln.r.inp, s);
                     } else if (!have_qkv) {
                         Timed t(c, "gemm_qkv");
-                        gemm(c, g, EPI_QKV, s);
+                        gemm(c, g, EPI_QKV, c->skinny_rows_decode, s);
                     }
                     AttnArgs a{};
                     a.q = Ln.r.q8; a.kc = kc; a.vc = vc; a.TP = TP; a.lens = Ln.ds.ntok; a.score_mult = L.score_mult;
@@ -1434,7 +1452,7 @@ static czip_status run_decompress(czip_job* j) {
                     GemmArgs hd{};
                     hd.A = Ln.r.xn; hd.W = c->head_w; hd.Wf = c->head_wf; hd.M = M; hd.N = V; hd.K = d;
                     hd.out32 = j->logits + (size_t)Ln.r0 * V; hd.ldo = V;
-                    { Timed t(c, "gemm_head"); gemm(c, hd, EPI_RAW, s); }
+                    { Timed t(c, "gemm_head"); gemm(c, hd, EPI_RAW, c->skinny_rows_decode, s); }
                     {
                         Timed t(c, "cdf_decode");
                         launch_cdf_decode(hd.out32, M, V, c->lut, c->cfg.coef_q24, c->cfg.target_total, p, Ln.st, Ln.ds, Ln.r.inp, s);
@@ -1588,7 +1606,7 @@ extern "C" czip_status czip_decode_step(czip_ctx* c, const uint32_t* tok_in, con
             layer0_qkv(c, g, j->inp, s);
         } else if (!have_qkv) {
             Timed t(c, "gemm_qkv");
-            gemm(c, g, EPI_QKV, s);
+            gemm(c, g, EPI_QKV, c->skinny_rows_decode, s);
         }
         AttnArgs a{};
         a.q = j->q8; a.kc = kc; a.vc = vc; a.TP = TP; a.lens = j->d_ntok; a.score_mult = L.score_mult;
@@ -1603,7 +1621,7 @@ extern "C" czip_status czip_decode_step(czip_ctx* c, const uint32_t* tok_in, con
     {
         GemmArgs hd{};
         hd.A = j->xn; hd.W = c->head_w; hd.Wf = c->head_wf; hd.M = S; hd.N = V; hd.K = d; hd.out32 = j->logits; hd.ldo = V;
-        { Timed t(c, "gemm_head"); gemm(c, hd, EPI_RAW, s); }
+        { Timed t(c, "gemm_head"); gemm(c, hd, EPI_RAW, c->skinny_rows_decode, s); }
         Timed t(c, "cdf");
         launch_cdf(j->logits, S, V, value_or_null ? j->d_val : nullptr, nullptr, 1, c->lut, c->cfg.coef_q24,
                    c->cfg.target_total, value_or_null ? 2 : 1, j->d_out, 0, s);
@@ -1661,7 +1679,7 @@ int32_t* carve_prefill(czip_ctx* c, czip_job* j, Carve& cv, int B, int T) {
     j->logits = c->head_fused ? nullptr : cv.take<int32_t>(M * V);
     // the few-row GEMMs' projection output, where the buffer has room for it
     // (without it those launches take the row GEMM)
-    if (!j->y8 && M <= (size_t)c->skinny_rows && cv.off + M * d + 256 <= NOALLOC_SCRATCH_BYTES) j->y8 = cv.take<int8_t>(M * d);
+    if (!j->y8 && M <= (size_t)c->skinny_rows_prefill && cv.off + M * d + 256 <= NOALLOC_SCRATCH_BYTES) j->y8 = cv.take<int8_t>(M * d);
     return err;
 }
 

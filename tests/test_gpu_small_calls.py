@@ -358,14 +358,46 @@ def test_decode_step_wave_counts(amd, orc, tmp_path, monkeypatch, vocab, env):
     assert np.array_equal(gm.decompress_chunks(cut, [13] * 24), om.decompress_many(cut, [13] * 24))
 
 
-@pytest.mark.parametrize("heads,kv,d_ff", [(4, 2, 4160), (12, 4, 448)])
-def test_few_row_gemms_row_limit(amd, orc, tmp_path, heads, kv, d_ff):
-    """Row counts up to the few-row GEMMs' limit of 1024 and just past it."""
+@pytest.mark.parametrize("heads,kv,d_ff,most", [(4, 2, 4160, 1024), (11, 1, 448, 1024), (12, 4, 448, 768)])
+def test_few_row_gemms_row_limit(amd, orc, tmp_path, heads, kv, d_ff, most):
+    """Row counts up to the few-row GEMMs' limit and just past it: 1024, and
+    768 where a row GEMM of 640 columns or more takes over."""
     import test_gpu_parity as parity
     from czip_amd import synth
     path = synth.write_random_model(str(tmp_path / "l.czm"), d=64 * heads, n_layers=2, n_heads=heads, n_kv=kv,
                                     d_ff=d_ff, vocab=1088, ctx=600, seed=800 + heads)
     gm = amd.Model(amd.ModelWeights(path, amd.KV_GQA))
     om = orc.Model.from_file(path, amd.KV_GQA)
-    for lens in ([520], [385, 385], [512, 300], [513, 512]):
+    gm.set_profiling(True)
+    for lens in ([520], [384, 384], [385, 385], [512, 300], [513, 512]):
+        seen = gm.kernel_stats("few_row_gemm")[0]
         parity._check_logits(gm, om, max(lens), lens, 17 + len(lens), 1088)
+        assert (gm.kernel_stats("few_row_gemm")[0] > seen) == (len(lens) * max(lens) <= most)
+
+
+@pytest.mark.parametrize("layers,most", [(2, 768), (24, 1024)])
+def test_few_row_gemms_decode_limit(amd, tmp_path, monkeypatch, layers, most):
+    """Decode steps of a wide model take the few-row GEMMs up to 768 streams,
+    and up to 1024 with weights of more than 48 MB; the intervals are those of
+    the other kernels."""
+    from czip_amd import synth
+    path = synth.write_random_model(str(tmp_path / "s.czm"), d=640, n_layers=layers, n_heads=10, n_kv=2, d_ff=1152,
+                                    vocab=1024, ctx=8, seed=850)
+    gm = amd.Model(amd.ModelWeights(path, amd.KV_GQA))
+    monkeypatch.setenv("CZIP_SKINNY_ROWS", "0")
+    other = amd.Model(amd.ModelWeights(path, amd.KV_GQA))
+    gm.set_profiling(True)
+    other.set_profiling(True)
+    for S in (768, 769, 1024, 1025):
+        rng = np.random.default_rng(S)
+        values = rng.integers(0, gm.target_total, (3, S)).astype(np.uint32)
+        toks = rng.integers(0, 1024, (3, S)).astype(np.uint32)
+        out = []
+        seen = gm.kernel_stats("few_row_gemm")[0]
+        for m in (gm, other):
+            m.decode_begin(S, 3)
+            out.append([m.decode_step(toks[p], np.full(S, p, np.int32), values[p]) for p in range(3)])
+            m.decode_end()
+        assert np.array_equal(out[0], out[1])
+        assert (gm.kernel_stats("few_row_gemm")[0] > seen) == (S <= most)
+    assert other.kernel_stats("few_row_gemm")[0] == 0
