@@ -35,8 +35,9 @@ constexpr int DEC_LANES_MAX = 4;  // most HIP streams a decode group is split ov
 // bytes span 256 bytes with 4-key blocks (1 KB with the prefill caches' 16-key blocks); the
 // decode attention reads this layout
 constexpr int DEC_VL = 2;
-// decode steps of at most this many (stream, head) rows take the attention
-// kernel with one row per wavefront (CZIP_ATTN_ROWS).  It gains up to 2.7x
+// decode steps of at most this many (stream, head) rows (three quarters where a
+// KV head has more than 8 query heads) take the attention kernel with one row
+// per wavefront (CZIP_ATTN_ROWS).  It gains up to 2.7x
 // while the rows leave SIMDs idle and loses once they queue: 4096 rows 118 ->
 // 64 ms (d512), 12288 rows 16.7 -> 18.3 (v001) and 81 -> 91 ms (d768)
 constexpr long long ATTN_ROWS_MAX = 8192;
@@ -432,6 +433,10 @@ void count_gemm(czip_ctx* c, GemmKernel k) {
     if (!c->profiling) return;
     if (k == GEMM_FEW_ROWS) c->stats["few_row_gemm"].launches++;
     if (k == GEMM_WIDE) c->stats["wide_gemm"].launches++;
+}
+
+void attn_decode(czip_ctx* c, const AttnArgs& a, int S, int p, hipStream_t s) {
+    if (launch_attn_decode(a, S, p, s) && c->profiling) c->stats["attn_decode_rows"].launches++;
 }
 
 // the GEMM launches with the context's kernel switches; skinny_rows: the pass's
@@ -1437,7 +1442,7 @@ static czip_status run_decompress(czip_job* j) {
                     a.sink = L.sink; a.lut = c->lut; a.etab = c->etab; a.out = Ln.r.attn; a.M = M; a.T = TP; a.H = H;
                     a.G = c->cfg.n_kv_heads; a.KH = c->KH; a.kv_mode = c->cfg.kv_mode; a.coef = 378194u;
                     a.general = L.attn_general; a.row_max = c->attn_rows;
-                    { Timed t(c, "attn_decode"); launch_attn_decode(a, M, p, s); }
+                    { Timed t(c, "attn_decode"); attn_decode(c, a, M, p, s); }
                     GemmArgs nq{};
                     if (l + 1 < c->cfg.n_layers) nq = qkv_args(l + 1);
                     have_qkv = post_attention(c, Ln.r, l, M, s, nl > 1, l + 1 < c->cfg.n_layers ? &nq : nullptr);
@@ -1613,7 +1618,7 @@ extern "C" czip_status czip_decode_step(czip_ctx* c, const uint32_t* tok_in, con
         a.sink = L.sink; a.lut = c->lut; a.etab = c->etab; a.out = j->attn; a.M = S; a.T = TP; a.H = c->cfg.n_heads; a.G = c->cfg.n_kv_heads;
         a.KH = c->KH; a.kv_mode = c->cfg.kv_mode; a.coef = 378194u;  // ATTN_COEF_Q24 (attention.rs:17-19)
         a.general = L.attn_general; a.row_max = c->attn_rows;
-        { Timed t(c, "attn_decode"); launch_attn_decode(a, S, p, s); }
+        { Timed t(c, "attn_decode"); attn_decode(c, a, S, p, s); }
         GemmArgs nq{};
         if (l + 1 < c->cfg.n_layers) nq = qkv_args(l + 1);
         have_qkv = post_attention(c, rows, l, S, s, false, l + 1 < c->cfg.n_layers ? &nq : nullptr);

@@ -379,19 +379,25 @@ __global__ __launch_bounds__(256) void k_attn_decode_row(AttnArgs a, int p) {
     a.out[((size_t)b * a.H + h) * 64 + lane] = attn_row_out(st);
 }
 
-void launch_attn_decode(const AttnArgs& a, int S, int p, hipStream_t s) {
+bool launch_attn_decode(const AttnArgs& a, int S, int p, hipStream_t s) {
     // heads per KV group: all of them in rust-compat mode (one KV head), H / G
     // in GQA mode (n_heads is a multiple of n_kv_heads); at most 16
     const int G = a.kv_mode == 1 ? a.H / a.G : a.H;
     AttnArgs g = a;
     g.B = S;
-    if ((long long)S * a.H <= a.row_max) {
+    const bool two = 2 * G <= 16;
+    // A stream with a wave of its own (more than 8 heads a group) costs the tile
+    // kernel three quarters of what two streams a wave do, and the rows pay up to
+    // as much less.  1024 steps of 2 layers, rows -> tiles: 16 heads a group 5000
+    // rows 57 -> 62 ms, 6144 62.0 -> 61.7, 8192 75.5 -> 62.3; 10 heads 6144 rows
+    // 63.8 -> 61.0, 8192 77.6 -> 62.5; 256 steps of 16 heads 6144 rows 9.0 -> 9.2, 8192
+    // 9.7 -> 9.5; with two streams, 1024 steps of 8 heads 8192 rows 79.1 -> 81.7
+    if ((long long)S * a.H <= (two ? a.row_max : a.row_max / 4 * 3)) {
         const dim3 grid((unsigned)(((long long)S * a.H + 3) / 4));
         if (a.general) hipLaunchKernelGGL(k_attn_decode_row<true>, grid, dim3(256), 0, s, g, p);
         else hipLaunchKernelGGL(k_attn_decode_row<false>, grid, dim3(256), 0, s, g, p);
-        return;
+        return true;
     }
-    const bool two = 2 * G <= 16;
     const long long waves = (long long)(two ? (S + 1) / 2 : S) * a.KH;
     dim3 grid((unsigned)((waves + 3) / 4));
     // rows in use per wave (NS G of 16), rounded up to 8, 12 or 16
@@ -411,6 +417,7 @@ void launch_attn_decode(const AttnArgs& a, int S, int p, hipStream_t s) {
         else CZIP_ATTN_DEC(false, 2, 16);
     }
 #undef CZIP_ATTN_DEC
+    return false;
 }
 
 // ---------------------------------------------------------------------------

@@ -227,7 +227,8 @@ void launch_dec_init(DecState st, DecStreams ds, int S, hipStream_t s);
 // interval in st.pend_lo / pend_hi); total = the frequency total
 void launch_dec_prep(DecStreams ds, DecState st, int S, int p, bool upd, unsigned total, uint32_t* inp, hipStream_t s);
 // one query per (stream, head) at position p over cached keys 0..p
-void launch_attn_decode(const AttnArgs& a, int S, int p, hipStream_t s);
+// (returns whether the one-row-per-wave kernel took it)
+bool launch_attn_decode(const AttnArgs& a, int S, int p, hipStream_t s);
 // logits -> cumulative frequencies -> one arithmetic-decode step (arith_coder.rs:195-264)
 void launch_cdf_decode(const int32_t* logits, int S, int V, const uint16_t* lut, unsigned coef, unsigned total,
                        int p, DecState st, DecStreams ds, uint32_t* inp, hipStream_t s);

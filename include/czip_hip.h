@@ -269,7 +269,8 @@ void        czip_set_profiling(czip_ctx* ctx, int32_t on);
  * "cdf"; decode: "dec_init","dec_prep","attn_decode","head_dec" (or, unfused,
  * "gemm_head","cdf_decode"), or "dec_fused" for every step in one launch.
  * "few_row_gemm" and "wide_gemm" count the GEMMs among them (under the names
- * above, with their time) that ran by the few-row kernel or in 128 x 256 tiles. */
+ * above, with their time) that ran by the few-row kernel or in 128 x 256 tiles,
+ * "attn_decode_rows" the decode attentions that took a row a wavefront. */
 czip_status czip_kernel_stats(czip_ctx* ctx, const char* name, int64_t* launches, double* total_ms);
 void        czip_reset_stats(czip_ctx* ctx);
 

@@ -113,7 +113,26 @@ def test_decode_attention_row_general(amd, orc, tmp_path, sink, kv, n_kv):
     toks = synth.zipf_ids(3 * 150 - 41, 1024, seed=431)
     chunks = om.compress_many(toks, 150, threads=4)
     assert np.array_equal(gm.decompress_chunks(chunks, [150, 150, 109]), toks)
-    assert gm.kernel_stats("dec_fused")[0] == 0 and gm.kernel_stats("attn_decode")[0] == 2 * 150
+    assert gm.kernel_stats("dec_fused")[0] == 0 and gm.kernel_stats("attn_decode_rows")[0] == 2 * 150
+
+
+@pytest.mark.parametrize("heads,most", [(8, 4), (16, 1), (10, 2)])
+def test_decode_attention_rows_limit(amd, orc, tmp_path, monkeypatch, heads, most):
+    """The most streams whose attention takes a row a wave: as many rows as the
+    limit, three quarters of it for groups of more than 8 heads."""
+    from czip_amd import synth
+    path = synth.write_random_model(str(tmp_path / "l.czm"), d=64 * heads, n_layers=2, n_heads=heads, n_kv=1, d_ff=64,
+                                    vocab=1024, ctx=70, seed=440 + heads)
+    monkeypatch.setenv("CZIP_ATTN_ROWS", "32")
+    gm, om = amd.Model(amd.ModelWeights(path, amd.KV_GQA)), orc.Model.from_file(path, amd.KV_GQA)
+    gm.set_profiling(True)
+    toks = synth.zipf_ids((most + 1) * 66, 1024, seed=441)
+    chunks = om.compress_many(toks, 66, threads=4)
+    for S in (most, most + 1):
+        gm.reset_stats()
+        assert np.array_equal(gm.decompress_chunks(chunks[:S], [66] * S), toks[:66 * S])
+        assert gm.kernel_stats("attn_decode")[0] == 2 * 66
+        assert gm.kernel_stats("attn_decode_rows")[0] == (2 * 66 if S == most else 0)
 
 
 def test_decode_attention_tile_edge_cases(amd, orc, tmp_path, monkeypatch):
@@ -150,7 +169,7 @@ def test_decode_attention_rows_key_counts(amd, pair, monkeypatch, n):
         for s in (1, 2, 3):
             assert np.array_equal(gm.decompress_chunks(chunks[:s], [n] * s), toks[:s * n])
         assert gm.kernel_stats("dec_fused")[0] == (3 if fused else 0)
-        assert gm.kernel_stats("attn_decode")[0] == (0 if fused else 3 * n)
+        assert gm.kernel_stats("attn_decode_rows")[0] == (0 if fused else 3 * n)
 
 
 @pytest.mark.parametrize("heads,kv,d_ff", [(1, 1, 64), (5, 1, 1600), (6, 2, 128), (14, 7, 832), (16, 4, 3136)])
