@@ -244,7 +244,8 @@ struct czip_ctx {
     int wide_rows = WIDE_ROWS_MIN;        // CZIP_WIDE_ROWS
     int64_t tail_rows = 0;        // most and least rows of a launch whose layers end in the tail
     int64_t tail_rows_min = 0;    // kernel (most 0: never)
-    int dec_fused_max = 0;        // most streams per group decoded by the whole-stream kernel (CZIP_DECODE_FUSED)
+    int dec_fused_max = 0;        // most streams per group decoded by the whole-stream kernel (CZIP_DECODE_FUSED),
+    bool dec_fused_line = true;   // and no more than decode_fused_streams of them (not with that switch)
     int decode_lanes = 0;         // CZIP_DECODE_LANES: lanes per decode group (0: by group size)
     bool lut0_max = false;        // exp2_lut[0] == 65535: the heads' table step 0 is E(0) (HeadCdfArgs::e0)
     std::vector<Alloc> allocs;
@@ -604,7 +605,10 @@ extern "C" czip_status czip_create(const czip_model_desc* w, int device, czip_ct
             ok = o.rq_fast && u.rq_fast && dn.rq_fast;
         }
         c->dec_fused_max = ok ? DECODE_FUSED_MAX_STREAMS : 0;
-        if (const char* e = getenv("CZIP_DECODE_FUSED")) c->dec_fused_max = std::min(c->dec_fused_max, std::max(0, atoi(e)));
+        if (const char* e = getenv("CZIP_DECODE_FUSED")) {
+            c->dec_fused_max = std::min(c->dec_fused_max, std::max(0, atoi(e)));
+            c->dec_fused_line = false;
+        }
     }
     {
         // the layer tail: its shapes, fast-path requantization, weights that stay in an L2
@@ -1342,9 +1346,11 @@ static czip_status run_decompress(czip_job* j) {
     // longest stream rounded up to whole 64-key tiles
     const int TP = pad64(Tc);
     const size_t layer_kv = (size_t)j->S * c->KH * TP * 64, stream_kv = (size_t)c->KH * TP * 64;
+    int fused_max = c->dec_fused_max;
+    if (c->dec_fused_line) fused_max = std::min(fused_max, decode_fused_streams(d, H, c->cfg.kv_mode == CZIP_KV_GQA ? c->cfg.n_kv_heads : 1, Tc));
     for (int64_t g0 = 0; g0 < j->nchunks; g0 += j->S) {
         const int S = (int)std::min<int64_t>(j->S, j->nchunks - g0);
-        if (S <= c->dec_fused_max) {
+        if (S <= fused_max) {
             const DevLayer& L = c->layers[0];
             GemmArgs o{}, u{}, dn{};  // requantization scales (the fast path, checked at czip_create)
             o.K = d; set_requant(o, L.out_mult, L.out_shift);

@@ -21,7 +21,7 @@
 //
 // Measured (shipped model, 512 steps, step kernels -> here): 1 stream 21.8 ->
 // 12.1 ms, 115 26.4 -> 12.2, 512 30.8 -> 14.5, 1024 36.8 -> 17.6, 2048 41.9 ->
-// 25.7, 4096 49.4 -> 42.6 ms; 115 streams of 64 steps 3.4 -> 1.3 ms.
+// 25.7 ms, 3500 42.6 -> 37.0; 115 streams of 64 steps 3.4 -> 1.3 ms.
 #include <algorithm>
 
 #include "czip_attn_row.h"
@@ -477,9 +477,24 @@ __global__ __launch_bounds__(64 * FNW) void k_decode_fused(FusedDecArgs a) {
 }
 
 // Streams per workgroup: one while they fit the CUs (the weights' stream per
-// step is the same for 1 and 16, the attention is not).  Past 16 a workgroup
-// (4096 streams) its row-wise attention is no match for the tile kernel's.
+// step is the same for 1 and 16, the attention is not), 16 at most.
 int decode_fused_rows(int S) { return std::max(1, (S + 255) / 256); }
+
+// Its row-wise attention is no match for the step kernels' tiles once there are
+// many rows and many keys, the sooner the more query heads share a KV head (the
+// tiles share their keys; with one or two they have no more to share).  The line
+// is rows^2 T, where both sides meet, in ms, steps -> here: shipped model, 1024
+// tokens 2560 streams 105.6 -> 87.7, 3072 107 -> 105, 4096 117 -> 142, 512 tokens
+// 4096 44.2 -> 41.2; d512, 4 heads a KV head, 512 tokens 2048 42.6 -> 39.3, 3072
+// 50.1 -> 51.3, 1024 tokens 2048 122 -> 118, 4096 175 -> 211; 8 heads a KV head, 512
+// tokens 2048 39.4 -> 36.5, 3072 42.6 -> 45.6, 1024 tokens 1536 90 -> 84, 2048 96 ->
+// 102, 64 tokens 4096 4.5 -> 3.9; 2 heads, 1024 tokens 4096 294 -> 284.
+int decode_fused_streams(int d, int H, int G, int T) {
+    const int share = H / G;
+    if (share <= 2) return DECODE_FUSED_MAX_STREAMS;
+    const double line = d >= 512 && share > 4 ? 1.6e11 : 2.9e11;
+    return std::min(DECODE_FUSED_MAX_STREAMS, (int)(__builtin_sqrt(line / (T < 1 ? 1 : T)) / H));
+}
 
 bool decode_fused_supported(int d, int F, int V) {
     return (d == 256 || d == 384 || d == 512) && F % 64 == 0 && F <= FMAXF && V == FV;

@@ -267,6 +267,8 @@ struct FusedDecArgs {
     unsigned coef, total;
 };
 constexpr int DECODE_FUSED_MAX_STREAMS = 256 * 16;
+// most streams of T steps for which it is the faster way (G: KV heads)
+int decode_fused_streams(int d, int H, int G, int T);
 bool decode_fused_supported(int d, int F, int V);
 void launch_decode_fused(const FusedDecArgs& a, int d, bool general, hipStream_t s);
 

@@ -233,6 +233,21 @@ def test_fused_decode_shapes(amd, orc, tmp_path, monkeypatch, i):
         assert np.array_equal(gm.decompress_chunks(coded, lens), np.concatenate(part))
 
 
+@pytest.mark.parametrize("T,most", [(1024, 2804), (800, 3173)])
+def test_fused_decode_stream_limit(amd, pair, T, most):
+    """The shipped model's streams decode as a whole up to the line where its
+    row-wise attention falls behind, and step by step past it."""
+    from czip_amd import synth
+    gm = amd.Model(amd.ModelWeights(MODEL_PATH))
+    gm.set_profiling(True)
+    toks = synth.zipf_ids((most + 1) * T, 1024, seed=T)
+    chunks = gm.compress_chunks(toks, T)
+    for S in (most, most + 1):
+        gm.reset_stats()
+        assert np.array_equal(gm.decompress_chunks(chunks[:S], [T] * S), toks[:S * T])
+        assert gm.kernel_stats("dec_fused")[0] == (1 if S == most else 0)
+
+
 def test_fused_decode_truncated_bytes(amd, pair):
     """Streams cut short read zeros past their end, as the step kernels do."""
     gm, om = pair
