@@ -52,6 +52,30 @@ constexpr long long ATTN_ROWS_MAX = 8192;
 // 18944 0.511 -> 0.505, 26752 0.277 -> 0.280, 65536 0.82 -> 0.84
 constexpr int64_t TAIL_ROWS_MAX = 20480;
 constexpr size_t TAIL_WEIGHTS_MAX = (size_t)4 << 20, TAIL_WEIGHT_BYTES_PER_ROW = 2500;
+// A workgroup's time is the weights' stream whatever its rows, so past one round
+// of the 256 CUs the tail loses where the next round is nearly empty, the more
+// the larger the weights.  Rows of a round: 8192, or 4096 where a feed-forward
+// past 2048 leaves LDS for 16 rows a workgroup only.  4 to 8 layers, separate
+// kernels -> tail:
+//  - 16 rows only: up to one round and the fuller half of the second.  d384 / F =
+//    3072 prefill 4096 rows 462 -> 438 us, 4200 510 -> 583, 6400 625 -> 596, 8192 647
+//    -> 622, 8400 665 -> 770; 32 decode steps 4200 10.7 -> 13.2 ms, 6400 14.3 -> 13.5,
+//    8400 15.7 -> 19.1; d256 / 4096 prefill 12288 570 -> 587, 20480 791 -> 862
+//  - more than 3 MB (d512 / 2048): prefills up to one round (8192 rows 1.28 -> 1.08
+//    ms, 8320 1.30 -> 1.43, 12288 1.48 -> 1.55, 18432 2.17 -> 2.15); decode steps
+//    not in the emptier half of the second (8200 33.8 -> 35.0 ms, 11000 37.4 ->
+//    37.7, 13300 40.9 -> 39.6, 16500 57.5 -> 56.5)
+//  - 2 to 3 MB: prefills likewise without that half (d512 / 1536 8320 rows 739 ->
+//    769 us, 12288 831 -> 834, 16640 1093 -> 1058; d384 / 2048 8200 596 -> 605, 13300
+//    662 -> 646), decode steps all (d512 / 1024 8200 14.4 -> 13.8 ms)
+//  - less: all (shipped model 8200 rows 253 -> 243 us, 16500 306 -> 295)
+constexpr size_t TAIL_WEIGHTS_LARGE = (size_t)3 << 20, TAIL_WEIGHTS_MEDIUM = (size_t)2 << 20;
+bool tail_rounds_pay(int64_t M, int F, size_t weights, bool decode) {
+    if (F > 2048) return M <= 4096 || (M >= 6144 && M <= 8192);
+    if (M <= 8192 || weights <= TAIL_WEIGHTS_MEDIUM) return true;
+    if (weights <= TAIL_WEIGHTS_LARGE) return decode || M >= 12288;
+    return decode && M >= 12288;
+}
 // GEMMs of at most this many rows split K over a workgroup's waves and the
 // columns over the chip (CZIP_SKINNY_ROWS); half of it where the layer tail
 // takes over below it.  A step-wise decode step, other kernels -> these: d768
@@ -243,7 +267,9 @@ struct czip_ctx {
     int skinny_rows_prefill = SKINNY_ROWS_MAX, skinny_rows_decode = SKINNY_ROWS_MAX;
     int wide_rows = WIDE_ROWS_MIN;        // CZIP_WIDE_ROWS
     int64_t tail_rows = 0;        // most and least rows of a launch whose layers end in the tail
-    int64_t tail_rows_min = 0;    // kernel (most 0: never)
+    int64_t tail_rows_min = 0;    // kernel (most 0: never),
+    bool tail_rounds = true;      // and not where its last round does not pay (CZIP_TAIL_ROWS: regardless)
+    size_t layer_weights = 0;     // bytes of a layer's weights
     int dec_fused_max = 0;        // most streams per group decoded by the whole-stream kernel (CZIP_DECODE_FUSED),
     bool dec_fused_line = true;   // and no more than decode_fused_streams of them (not with that switch)
     int decode_lanes = 0;         // CZIP_DECODE_LANES: lanes per decode group (0: by group size)
@@ -632,7 +658,11 @@ extern "C" czip_status czip_create(const czip_model_desc* w, int device, czip_ct
         }
         if (ok && c->tail_rows_min < SKINNY_ROWS_MAX) c->skinny_rows_prefill = c->skinny_rows_decode = SKINNY_ROWS_MAX / 2;
         if (const char* e = getenv("CZIP_SKINNY_ROWS")) c->skinny_rows_prefill = c->skinny_rows_decode = std::max(0, atoi(e));
-        if (const char* e = getenv("CZIP_TAIL_ROWS")) c->tail_rows = ok ? std::max(0ll, atoll(e)) : 0;
+        if (const char* e = getenv("CZIP_TAIL_ROWS")) {
+            c->tail_rows = ok ? std::max(0ll, atoll(e)) : 0;
+            c->tail_rounds = false;
+        }
+        c->layer_weights = d * (qn + d + 3 * F);
     }
     czip_ctx* C = c.get();
 #define UP(dst, src, n) if ((rc = upload(C, &dst, src, n))) return rc;
@@ -811,6 +841,7 @@ struct RowBufs {
     int32_t* rn_ws;
     size_t rn_ws_bytes;
     int skinny_rows;  // the pass's limit of the few-row GEMMs
+    bool decode;      // a decode step's rows
 };
 
 RowBufs row_bufs(const czip_ctx* c, const czip_job* j, int64_t r0 = 0, int ws_parts = 1, int ws_part = 0) {
@@ -819,7 +850,7 @@ RowBufs row_bufs(const czip_ctx* c, const czip_job* j, int64_t r0 = 0, int ws_pa
     return RowBufs{j->inp + r, j->x + r * d, j->xn + r * d, j->q8 + r * d, j->attn + r * d,
                    j->y8 ? j->y8 + r * d : nullptr, j->r8 ? j->r8 + r * F : nullptr,
                    j->rn_ws ? j->rn_ws + wb / 4 * (size_t)ws_part : nullptr, wb,
-                   j->kind == 0 ? c->skinny_rows_prefill : c->skinny_rows_decode};
+                   j->kind == 0 ? c->skinny_rows_prefill : c->skinny_rows_decode, j->kind != 0};
 }
 
 // next_qkv: the next layer's Q/K/V projection of a decode step (or nullptr);
@@ -830,7 +861,8 @@ bool post_attention(czip_ctx* c, const RowBufs& r, int l, int M, hipStream_t s, 
     const DevLayer& L = c->layers[(size_t)l];
     const bool last = l + 1 == c->cfg.n_layers;
     const int8_t* next = last ? c->final_norm : c->layers[(size_t)l + 1].attn_norm;
-    if (M > r.skinny_rows && M >= c->tail_rows_min && M <= c->tail_rows) {
+    if (M > r.skinny_rows && M >= c->tail_rows_min && M <= c->tail_rows &&
+        (!c->tail_rounds || tail_rounds_pay(M, F, c->layer_weights, r.decode))) {
         GemmArgs o{}, u{}, dn{};  // requantization scales (the fast path, checked at czip_create)
         o.K = d; set_requant(o, L.out_mult, L.out_shift);
         u.K = d; set_requant(u, L.up_mult, L.up_shift);

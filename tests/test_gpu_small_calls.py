@@ -288,6 +288,40 @@ def test_layer_tail(amd, orc, tmp_path, monkeypatch, d, kv, d_ff, mode):
         assert gm.kernel_stats("layer_tail")[0] > seen
 
 
+@pytest.mark.parametrize("d,kv,d_ff,prefill,decode", [
+    (512, 2, 2048, {8192: 1, 8193: 0, 12288: 0, 16400: 0}, {8192: 1, 8193: 0, 12287: 0, 12288: 1, 20480: 1, 20481: 0}),
+    (512, 2, 1536, {8192: 1, 12287: 0, 12288: 1, 20481: 0}, {8193: 1, 20480: 1}),
+    (384, 1, 3072, {4096: 1, 4097: 0, 6143: 0, 6144: 1, 8192: 1, 8193: 0}, {4096: 1, 4097: 0, 6144: 1, 8193: 0}),
+    (256, 1, 512, {8193: 1, 20480: 1, 20481: 0}, {8193: 1, 20480: 1})])
+def test_layer_tail_rounds(amd, tmp_path, monkeypatch, d, kv, d_ff, prefill, decode):
+    """Row counts on both sides of the tail's rounds: the kernel expected there,
+    and the bytes and intervals of the separate kernels."""
+    from czip_amd import synth
+    path = synth.write_random_model(str(tmp_path / "t.czm"), d=d, n_layers=2, n_heads=d // 64, n_kv=kv, d_ff=d_ff,
+                                    vocab=1024, ctx=64, seed=900 + d_ff)
+    gm = amd.Model(amd.ModelWeights(path, amd.KV_GQA))
+    monkeypatch.setenv("CZIP_TAIL_ROWS", "0")
+    other = amd.Model(amd.ModelWeights(path, amd.KV_GQA))
+    gm.set_profiling(True)
+    for rows, tail in prefill.items():
+        toks = np.random.default_rng(rows).integers(0, 1024, rows).astype(np.uint32)
+        gm.reset_stats()
+        chunk = next(c for c in (32, 31, 29, 23, 19, 17, 13, 11, 7, 5, 3, 1) if rows % c == 0)  # whole chunks: rows rows
+        assert gm.compress_chunks(toks, chunk) == other.compress_chunks(toks, chunk)
+        assert gm.kernel_stats("layer_tail")[0] == 2 * tail
+    for S, tail in decode.items():
+        rng = np.random.default_rng(S)
+        toks, values = rng.integers(0, 1024, (2, S)).astype(np.uint32), rng.integers(0, gm.target_total, (2, S)).astype(np.uint32)
+        gm.reset_stats()
+        out = []
+        for m in (gm, other):
+            m.decode_begin(S, 2)
+            out.append([m.decode_step(toks[p], np.full(S, p, np.int32), values[p]) for p in range(2)])
+            m.decode_end()
+        assert np.array_equal(out[0], out[1])
+        assert gm.kernel_stats("layer_tail")[0] == 4 * tail
+
+
 def test_row_gemm_16_without_tail(amd, shipped, monkeypatch):
     """The 16-row row GEMM behind the tail (shapes whose weights outgrow an L2 take it)."""
     import test_gpu_parity as parity
