@@ -91,8 +91,11 @@ bool tail_rounds_pay(int64_t M, int F, size_t weights, bool decode) {
 // 321 -> 307, 323 -> 349; d704 (2, no row GEMM) 288 -> 261, 292 -> 271.  Decode
 // steps of 800 and 1024 streams: d640 (12 layers, 71 MB) 920 -> 795, 883 -> 878
 // us; d1024 (12) 1419 -> 1289, 1459 -> 1454; d768 (2 layers, 17 MB) 212 -> 208, 224
-// -> 231; d1024 (2, 31 MB) 1024 streams 264 -> 289
-constexpr int SKINNY_ROWS_MAX = 1024, SKINNY_WIDE_ROWS = 768, SKINNY_WIDE_D = 640;
+// -> 231; d1024 (2, 31 MB) 1024 streams 264 -> 289.  Decode steps of a feed-forward
+// past RN16_KMAX, whose down projection has a split-K kernel there: 512 rows
+// (F = 8192, 2 layers, 400 streams d512 206 -> 190 us, d1024 292 -> 259; 760 220
+// -> 237, 307 -> 350; 1000 223 -> 274, 305 -> 406; d1024 12 layers 760 1578 -> 1777)
+constexpr int SKINNY_ROWS_MAX = 1024, SKINNY_WIDE_ROWS = 768, SKINNY_WIDE_D = 640, SKINNY_SPLITK_ROWS = 512;
 constexpr size_t SKINNY_SMALL_WEIGHTS = (size_t)48 << 20;
 // GEMMs of at least this many rows, where no W-stationary kernel takes them,
 // run 128 x 256 tiles with the weights straight from L2 (CZIP_WIDE_ROWS)
@@ -656,6 +659,7 @@ extern "C" czip_status czip_create(const czip_model_desc* w, int device, czip_ct
             c->skinny_rows_prefill = SKINNY_WIDE_ROWS;
             if (d * (qn + d + 3 * F) * (size_t)w->n_layers <= SKINNY_SMALL_WEIGHTS) c->skinny_rows_decode = SKINNY_WIDE_ROWS;
         }
+        if (c->rn_fused && w->d_ff > RN16_KMAX) c->skinny_rows_decode = SKINNY_SPLITK_ROWS;
         if (ok && c->tail_rows_min < SKINNY_ROWS_MAX) c->skinny_rows_prefill = c->skinny_rows_decode = SKINNY_ROWS_MAX / 2;
         if (const char* e = getenv("CZIP_SKINNY_ROWS")) c->skinny_rows_prefill = c->skinny_rows_decode = std::max(0, atoi(e));
         if (const char* e = getenv("CZIP_TAIL_ROWS")) {

@@ -1022,7 +1022,6 @@ __global__ __launch_bounds__(64 * NW) void k_gemm_rn_ws(RowGemmArgs a) {
 // ahead, every W operand used by one MFMA.  The epilogue is rn_epilogue over
 // one row tile.
 // ---------------------------------------------------------------------------
-constexpr int RN16_KMAX = 4096;
 constexpr int RN16_WP = 3;  // K steps of W in flight per wave
 
 template <int NW, int CT, bool FAST>

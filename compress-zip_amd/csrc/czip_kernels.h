@@ -109,6 +109,7 @@ struct RowGemmArgs {
     int skinny_rows = 0, wide_rows = 0;
 };
 bool gemm_rn_supported(int d);
+constexpr int RN16_KMAX = 4096;  // longest K of the 16-row row GEMM
 // bytes of workspace the split-K row GEMM wants for M rows of width d (0: M is large enough without)
 size_t gemm_rn_ws_bytes(int M, int d);
 // the row GEMM's epilogue from the requantized projection a.y8

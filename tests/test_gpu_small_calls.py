@@ -443,20 +443,21 @@ def test_few_row_gemms_row_limit(amd, orc, tmp_path, heads, kv, d_ff, most):
         assert (gm.kernel_stats("few_row_gemm")[0] > seen) == (len(lens) * max(lens) <= most)
 
 
-@pytest.mark.parametrize("layers,most", [(2, 768), (24, 1024)])
-def test_few_row_gemms_decode_limit(amd, tmp_path, monkeypatch, layers, most):
+@pytest.mark.parametrize("heads,layers,d_ff,most", [(10, 2, 1152, 768), (10, 24, 1152, 1024), (8, 2, 4160, 512)])
+def test_few_row_gemms_decode_limit(amd, tmp_path, monkeypatch, heads, layers, d_ff, most):
     """Decode steps of a wide model take the few-row GEMMs up to 768 streams,
-    and up to 1024 with weights of more than 48 MB; the intervals are those of
-    the other kernels."""
+    up to 1024 with weights of more than 48 MB, and up to 512 with a
+    feed-forward of more than 4096; the intervals are those of the other
+    kernels."""
     from czip_amd import synth
-    path = synth.write_random_model(str(tmp_path / "s.czm"), d=640, n_layers=layers, n_heads=10, n_kv=2, d_ff=1152,
+    path = synth.write_random_model(str(tmp_path / "s.czm"), d=64 * heads, n_layers=layers, n_heads=heads, n_kv=2, d_ff=d_ff,
                                     vocab=1024, ctx=8, seed=850)
     gm = amd.Model(amd.ModelWeights(path, amd.KV_GQA))
     monkeypatch.setenv("CZIP_SKINNY_ROWS", "0")
     other = amd.Model(amd.ModelWeights(path, amd.KV_GQA))
     gm.set_profiling(True)
     other.set_profiling(True)
-    for S in (768, 769, 1024, 1025):
+    for S in (512, 513, 768, 769, 1024, 1025):
         rng = np.random.default_rng(S)
         values = rng.integers(0, gm.target_total, (3, S)).astype(np.uint32)
         toks = rng.integers(0, 1024, (3, S)).astype(np.uint32)
