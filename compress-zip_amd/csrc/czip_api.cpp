@@ -848,6 +848,11 @@ struct RowBufs {
     bool decode;      // a decode step's rows
 };
 
+// workspace bytes of a decode job or session of S streams
+size_t decode_ws_bytes(const czip_ctx* c, int S) {
+    return gemm_rn_ws_bytes(S, c->cfg.d_model, std::max(c->cfg.d_model, c->cfg.d_ff), c->gemm_tiled ? 0 : c->skinny_rows_decode);
+}
+
 RowBufs row_bufs(const czip_ctx* c, const czip_job* j, int64_t r0 = 0, int ws_parts = 1, int ws_part = 0) {
     const size_t d = (size_t)c->cfg.d_model, F = (size_t)c->cfg.d_ff, r = (size_t)r0;
     const size_t wb = j->rn_ws_bytes / (size_t)ws_parts / 16 * 16;
@@ -1338,13 +1343,13 @@ extern "C" czip_status czip_decompress_plan(czip_ctx* c, const uint8_t* data, co
         (rc = dalloc(c, A, &j->q8, (size_t)S * d)) || (rc = dalloc(c, A, &j->attn, (size_t)S * d)) ||
         (rc = dalloc(c, A, &j->y8, (size_t)S * d)) || (rc = dalloc(c, A, &j->r8, (size_t)S * c->cfg.d_ff)) ||
         (rc = dalloc(c, A, &j->logits, c->head_fused ? 1 : (size_t)S * c->cfg.vocab)) ||
-        (rc = dalloc(c, A, &j->rn_ws, std::max<size_t>(gemm_rn_ws_bytes((int)S, (int)d) / 4, 1))) ||
+        (rc = dalloc(c, A, &j->rn_ws, std::max<size_t>(decode_ws_bytes(c, (int)S) / 4, 1))) ||
         (rc = dalloc(c, A, &j->kc, L * (size_t)S * c->KH * pad64(Tcap) * 64)) ||
         (rc = dalloc(c, A, &j->vc, L * (size_t)S * c->KH * pad64(Tcap) * 64))) {
         free_job_mem(j.get());
         return rc;
     }
-    j->rn_ws_bytes = gemm_rn_ws_bytes((int)S, (int)d);
+    j->rn_ws_bytes = decode_ws_bytes(c, (int)S);
     hipError_t e = hipSuccess;
     if (total_bytes > 0) e = hipMemcpy(j->d_data, data, (size_t)total_bytes, hipMemcpyHostToDevice);
     if (e == hipSuccess && nchunks > 0) e = hipMemcpy(j->d_offs, offs, (size_t)nchunks * 8, hipMemcpyHostToDevice);
@@ -1581,12 +1586,12 @@ extern "C" czip_status czip_decode_begin(czip_ctx* c, int32_t S, int32_t T) {
         (rc = dalloc(c, A, &j->q8, (size_t)S * d)) || (rc = dalloc(c, A, &j->attn, (size_t)S * d)) ||
         (rc = dalloc(c, A, &j->y8, (size_t)S * d)) || (rc = dalloc(c, A, &j->r8, (size_t)S * c->cfg.d_ff)) ||
         (rc = dalloc(c, A, &j->logits, (size_t)S * V)) ||
-        (rc = dalloc(c, A, &j->rn_ws, std::max<size_t>(gemm_rn_ws_bytes(S, (int)d) / 4, 1))) ||
+        (rc = dalloc(c, A, &j->rn_ws, std::max<size_t>(decode_ws_bytes(c, S) / 4, 1))) ||
         (rc = dalloc(c, A, &j->kc, kv)) || (rc = dalloc(c, A, &j->vc, kv))) {
         free_job_mem(j.get());
         return rc;
     }
-    j->rn_ws_bytes = gemm_rn_ws_bytes(S, (int)d);
+    j->rn_ws_bytes = decode_ws_bytes(c, S);
     j->h_lens.assign((size_t)S, -1);
     j->h_done.assign((size_t)S, -1);
     c->dec = j.release();

@@ -1113,6 +1113,7 @@ __global__ __launch_bounds__(64 * NW) void k_gemm_rn_part(RowGemmArgs a, int ks_
 }
 
 constexpr int RN_MAX_SPLITS = 16;
+constexpr int RN16_MIN_BLOCKS = 24;
 
 // K slices for M rows: enough (row block, slice) workgroups for the 256 CUs, at
 // least two K steps per slice; 1 = no split
@@ -1122,7 +1123,10 @@ static int rn_splits(int M, int K) {
     return std::max(1, std::min(std::min(RN_MAX_SPLITS, K / 128), (384 + nblk - 1) / nblk));
 }
 
-size_t gemm_rn_ws_bytes(int M, int d) {
+size_t gemm_rn_ws_bytes(int M, int d, int K, int skinny_rows) {
+    // launches of up to skinny_rows rows are the few-row GEMM's, and of at least
+    // RN16_MIN_BLOCKS blocks and up to RN16_KMAX deep the 16-row kernel's
+    if (M <= skinny_rows || (K <= RN16_KMAX && skinny_rows >= 16 * (RN16_MIN_BLOCKS - 1))) return 0;
     return (size_t)RN_MAX_SPLITS * (size_t)M * (size_t)d * 4u * ((M + RBM - 1) / RBM < 96 ? 1u : 0u);
 }
 
@@ -1158,7 +1162,6 @@ static void launch_rn_ws(const RowGemmArgs& a, hipStream_t s) {
 // workgroup per 16 rows, K unsplit.  From 24 blocks it beats the split-K
 // kernels (d768/L12 decode groups of 1,272 and 776 streams: O projection
 // 1.70 vs 2.61 s, down projection 3.58 vs 4.14 s per 8 M-token job)
-constexpr int RN16_MIN_BLOCKS = 24;
 static bool use_rn16(const RowGemmArgs& a) {
     const int nblk = (a.M + RBM - 1) / RBM;
     return nblk < 96 && (a.M + 15) / 16 >= RN16_MIN_BLOCKS && a.K <= RN16_KMAX;

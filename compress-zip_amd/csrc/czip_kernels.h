@@ -110,8 +110,9 @@ struct RowGemmArgs {
 };
 bool gemm_rn_supported(int d);
 constexpr int RN16_KMAX = 4096;  // longest K of the 16-row row GEMM
-// bytes of workspace the split-K row GEMM wants for M rows of width d (0: M is large enough without)
-size_t gemm_rn_ws_bytes(int M, int d);
+// bytes of workspace the split-K row GEMM wants for launches of up to M rows of width
+// d and a longest K, the few-row GEMMs taking skinny_rows (0: none of them gets there)
+size_t gemm_rn_ws_bytes(int M, int d, int K, int skinny_rows);
 // the row GEMM's epilogue from the requantized projection a.y8
 void launch_rn_rows(const RowGemmArgs& a, hipStream_t s);
 void launch_rn_splitk_epi(const RowGemmArgs& a, const int32_t* part, int splits, hipStream_t s);

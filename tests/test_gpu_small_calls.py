@@ -3,6 +3,8 @@ their limits, against the oracle: the arithmetic encoder's load groups, decode
 attention by rows, few-row GEMMs, whole-stream decode, layer tail, 128 x 256
 tiles and the wave counts of the unfused decoder step; and device memory that
 jobs hand on."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -22,6 +24,14 @@ def amd():
 @pytest.fixture(scope="module")
 def pair(amd, orc):
     return amd.Model(amd.ModelWeights(MODEL_PATH)), orc.Model.from_file(MODEL_PATH)
+
+
+def free_device_memory():
+    """Free bytes of the device, from the HIP runtime that the library links."""
+    hip = C.CDLL("libamdhip64.so.7")
+    free, total = C.c_size_t(), C.c_size_t()
+    assert hip.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+    return free.value
 
 
 @pytest.mark.parametrize("chunk", [1, 7, 8, 9, 16, 65])
@@ -56,6 +66,25 @@ def test_job_memory_reuse(pair):
     for j, (_, _, want) in zip(jobs, ref):
         assert j.fetch() == want
         j.free()
+
+
+@pytest.mark.parametrize("d_ff,env,want", [(1024, None, 0), (4160, None, 1), (1024, "0", 1)])
+def test_split_k_workspace_only_where_used(amd, tmp_path, monkeypatch, d_ff, env, want):
+    """A session's split-K workspace (64 KB a stream at d1024) is there where a
+    launch can take the split-K row GEMM: K past 4096, or the few-row GEMMs off."""
+    from czip_amd import synth
+    path = synth.write_random_model(str(tmp_path / "w.czm"), d=1024, n_layers=1, n_heads=16, n_kv=1, d_ff=d_ff,
+                                    vocab=1024, ctx=8, seed=860)
+    if env is not None:
+        monkeypatch.setenv("CZIP_SKINNY_ROWS", env)
+    S = 4000
+    gm = amd.Model(amd.ModelWeights(path, amd.KV_GQA))
+    before = free_device_memory()
+    gm.decode_begin(S, 4)
+    used = before - free_device_memory()
+    gm.decode_end()
+    rest = S * (2 * 4 * 1024 + 7 * 1024 + d_ff + 2 * 64 * 64)  # tables and logits, rows, caches
+    assert (used > rest + S * 32 * 1024) == bool(want), (used, rest)
 
 
 def test_job_memory_threads(amd, pair):
