@@ -157,11 +157,12 @@ struct Alloc {
 // frees its tens of GB on every call waits for that clearing as soon as the
 // already cleared memory is used up: repeated 24 MiB text compressions took
 // 1.60 s a call around 0.134 s of kernels (now 0.139 s), and calls of a few MB
-// spent 0.5-2.8 ms in hipFree (418 chunks of 64: 1.07 -> 0.35 ms a call).  At most POOL_SCRATCH_SHARE of the context's scratch
-// budget is kept (least recently used blocks go first), all of it is given
-// back at czip_destroy, and an allocation that fails gives back what every
-// context holds before it is tried again.  Only idle blocks are here: a job
-// waits for the context's streams before it returns its memory.
+// spent 0.5-2.8 ms in hipFree (418 chunks of 64: 1.07 -> 0.35 ms a call).  At
+// most POOL_SCRATCH_SHARE of the context's scratch budget is kept (least
+// recently used blocks go first), all of it is given back at czip_trim and
+// czip_destroy, and an allocation that fails gives back what every context
+// holds before it is tried again.  Only idle blocks are here: a job waits for
+// the context's streams before it returns its memory.
 constexpr double POOL_SCRATCH_SHARE = 1.25;  // a job's inputs and outputs lie beside its scratch
 class DevicePool {
 public:
@@ -771,6 +772,12 @@ extern "C" void czip_destroy(czip_ctx* c) {
     for (auto q : c->lane_s) if (q) hipStreamDestroy(q);
     if (c->stream) hipStreamDestroy(c->stream);
     delete c;
+}
+
+extern "C" void czip_trim(czip_ctx* c) {
+    if (!c) return;
+    hipSetDevice(c->device);
+    c->pool.trim();
 }
 
 extern "C" void czip_set_profiling(czip_ctx* c, int32_t on) {

@@ -80,6 +80,7 @@ SIGNATURES = {
     "czip_model_free": (None, [_P]),
     "czip_create": (C.c_int32, [C.POINTER(ModelDesc), C.c_int, C.POINTER(C.c_void_p)]),
     "czip_destroy": (None, [_P]),
+    "czip_trim": (None, [_P]),
     "czip_last_error": (C.c_char_p, [_P]),
     "czip_device_count": (C.c_int, []),
     "czip_forward_logits": (C.c_int32, [_P, _P, _P, C.c_int32, C.c_int32, _P]),
@@ -239,6 +240,10 @@ class Model:
 
     def __del__(self):
         self.close()
+
+    def trim(self):
+        """Give the device memory of freed jobs back to the driver."""
+        lib().czip_trim(self._ctx)
 
     # --- batched forward (debug / parity) ---
     def forward_logits(self, inputs: np.ndarray, lens) -> np.ndarray:

@@ -9,8 +9,9 @@
  * stream and all device memory it allocates; it is not thread-safe, but
  * several contexts may coexist (one per host thread / device).  The device
  * memory of a freed job or session stays with the context for its next ones
- * (at most 1.25 times CZIP_SCRATCH_GB, 80 GB by default) until czip_destroy,
- * or until an allocation of any context in the process would fail without it.
+ * (at most 1.25 times CZIP_SCRATCH_GB, 80 GB by default) until czip_trim or
+ * czip_destroy, or until an allocation of any context in the process would
+ * fail without it; other allocators and processes do not get it before.
  *
  * The reference has no FFI; each entry point names the Rust API it stands in
  * for (file:line in the reference crate, rust/src).
@@ -98,6 +99,9 @@ void czip_model_free(czip_model* m);
  *      (attention.rs:172).  Weights are copied; the caller keeps ownership. ---- */
 czip_status czip_create(const czip_model_desc* w, int device, czip_ctx** out);
 void        czip_destroy(czip_ctx* ctx);
+/* Gives the device memory of freed jobs and sessions that the context keeps
+ * back to the driver (live jobs and an open session keep theirs). */
+void        czip_trim(czip_ctx* ctx);
 const char* czip_last_error(const czip_ctx* ctx);   /* never NULL */
 int         czip_device_count(void);
 

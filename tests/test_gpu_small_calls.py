@@ -68,6 +68,28 @@ def test_job_memory_reuse(pair):
         j.free()
 
 
+def test_job_memory_trim(amd, pair):
+    """Freed jobs' memory goes back to the driver on demand, the live ones' stays."""
+    _, om = pair
+    gm = amd.Model(amd.ModelWeights(MODEL_PATH))
+    toks = np.random.default_rng(8).integers(0, 1024, 300_000).astype(np.uint32)
+    gm.compress_chunks(toks[:2000], 512)  # what a first launch takes for itself
+    gm.trim()
+    before = free_device_memory()
+    gm.compress_chunks(toks, 512)
+    live = gm.compress_plan(toks[:2000], 512)
+    kept = before - free_device_memory()
+    assert kept > 500e6  # 300 thousand rows of about 4 KB
+    gm.trim()
+    assert 0 <= before - free_device_memory() < 100e6  # the live job's
+    live.run()
+    assert live.fetch() == om.compress_many(toks[:2000], 512, threads=4)
+    live.free()
+    gm.trim()
+    assert before - free_device_memory() < 16 << 20  # the runtime keeps a few pieces of 2 MB for small allocations
+    assert gm.compress_chunks(toks[:2000], 512) == om.compress_many(toks[:2000], 512, threads=4)
+
+
 @pytest.mark.parametrize("d_ff,env,want", [(1024, None, 0), (4160, None, 1), (1024, "0", 1)])
 def test_split_k_workspace_only_where_used(amd, tmp_path, monkeypatch, d_ff, env, want):
     """A session's split-K workspace (64 KB a stream at d1024) is there where a
