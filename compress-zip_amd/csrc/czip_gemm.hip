@@ -459,9 +459,9 @@ __global__ __launch_bounds__(256, 2) void k_gemm_ws(GemmArgs a, int ncg) {
 // WIDE_GROUP row blocks are neighbours, so that an XCD's workgroups share both
 // operands in its L2.  d768, 200 thousand rows, 12 layers, against k_gemm: up +
 // ReGLU 16.4 -> 10.8 ms (1.4 -> 2.1 POP/s), QKV 4.3 -> 3.1, head (V = 8192) 2.7 ->
-// 2.2; 4096 rows: up 0.42 -> 0.35, QKV 0.19 -> 0.22; 2048 rows 0.26 -> 0.29 and
-// 0.16 -> 0.20.  (K = 512: the W-stationary kernel is faster, up 14.9 against 18.4
-// ms at a million rows.)  Fast requantization only (try_wide).  A whole pass of 2
+// 2.2; 4096 rows: up 0.42 -> 0.35; 2048 rows up 0.26 -> 0.29.  (K = 512: the
+// W-stationary kernel is faster, up 14.9 against 18.4 ms at a million rows.)
+// Fast requantization only, QKV from 256 tiles on (try_wide).  A whole pass of 2
 // layers, 4096 / 65536 rows: d640 449 -> 443 us / 2.33 -> 2.12 ms, d704 511 -> 488
 // / 2.75 -> 2.36, d768 487 -> 474 / 2.90 -> 2.31, d896 543 -> 532 / 3.62 -> 2.86,
 // d1024 586 -> 566 / 4.12 -> 3.27.
@@ -588,6 +588,13 @@ static bool try_wide(const GemmArgs& a, hipStream_t s) {
     if (a.tiled || !a.Wf || a.a_rows || a.M < a.wide_rows || a.N % 64 != 0 || (long long)a.N * a.K >= (1ll << 31) - (1 << 20) ||
         (long long)WIDE_BM * a.K >= (1ll << 31) || (long long)WIDE_BM * a.ldo * (EPI == EPI_RAW ? 4 : 1) >= (1ll << 31))
         return false;
+    // QKV, the narrowest of the projections: as many full tiles as CUs (by default
+    // wide_rows / 16 = 256).  Per launch, 128 x 128 tiles -> these: d256 / N = 512
+    // 4096 rows 11.0 -> 12.5 us, 8192 11.7 -> 13.5, 16384 15.6 -> 15.1; d448 / 576
+    // 10240 14.7 -> 17.3, 16384 19.0 -> 18.7; d768 / 1280 4096 17.2 -> 18.7, 8192 23.8
+    // -> 20.0; d1024 / 1280 6144 20.3 -> 22.5, 8192 25.7 -> 23.7.  (The others gain
+    // with fewer: d768 O and down, 192 tiles, 8192 rows 31.8 -> 22.8 and 56.6 -> 36.1)
+    if (EPI == EPI_QKV && (long long)a.M * a.N < (long long)(a.wide_rows / 16) * WIDE_BM * WIDE_BN) return false;
     // 32-bit offsets into the caches from a block's first chunk
     if (EPI == EPI_QKV && (((long long)WIDE_BM / a.T + 2) * a.KH * a.TP * 64 >= (1ll << 31) || a.T > a.TP || a.pos >= 0)) return false;
     const int ntm = (a.M + WIDE_BM - 1) / WIDE_BM, ntn = (a.N + WIDE_BN - 1) / WIDE_BN;

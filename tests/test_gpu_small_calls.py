@@ -434,6 +434,23 @@ def test_wide_gemms(amd, orc, tmp_path, monkeypatch, heads, kv, d_ff, vocab, per
         assert gm.kernel_stats("wide_gemm")[0] - seen == n
 
 
+def test_wide_qkv_least_tiles(amd, tmp_path, monkeypatch):
+    """A narrow QKV projection takes the 128 x 256 tiles from 256 of them on; the
+    bytes are those of the other kernel."""
+    from czip_amd import synth
+    path = synth.write_random_model(str(tmp_path / "q.czm"), d=256, n_layers=2, n_heads=4, n_kv=2, d_ff=512, vocab=1024,
+                                    ctx=64, seed=640)
+    gm = amd.Model(amd.ModelWeights(path, amd.KV_GQA))
+    monkeypatch.setenv("CZIP_WIDE_ROWS", str(1 << 30))
+    other = amd.Model(amd.ModelWeights(path, amd.KV_GQA))
+    gm.set_profiling(True)
+    for rows, wide in ((8192, 0), (16352, 0), (16384, 1), (16416, 1)):
+        toks = np.random.default_rng(rows).integers(0, 1024, rows).astype(np.uint32)
+        gm.reset_stats()
+        assert gm.compress_chunks(toks, 32) == other.compress_chunks(toks, 32)
+        assert gm.kernel_stats("wide_gemm")[0] == wide
+
+
 def test_general_requantization_leaves_the_wide_tiles(amd, orc, tmp_path, monkeypatch):
     """Projections off the fast requantization path (|mult| >= 2^26) keep the
     128 x 128 tiles, which are faster there; the head has none and does not."""
