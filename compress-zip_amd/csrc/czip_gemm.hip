@@ -711,11 +711,19 @@ static void launch_skinny_nw(const GemmArgs& a, hipStream_t s) {
 
 template <int EPI, bool FAST>
 static void launch_skinny(const GemmArgs& a, hipStream_t s) {
-    // about SKINNY_U K steps a wave
+    // about SKINNY_U K steps a wave (all but the down projection have K = d_model <= 1024)
     const int nks = a.K / 64;
-    if (nks <= 4 * SKINNY_U) launch_skinny_nw<EPI, FAST, 4>(a, s);
-    else if (EPI == EPI_QKV || EPI == EPI_REGLU || nks <= 8 * SKINNY_U) launch_skinny_nw<EPI, FAST, 8>(a, s);
-    else launch_skinny_nw<EPI, FAST, 16>(a, s);
+    if (nks <= 4 * SKINNY_U) {
+        launch_skinny_nw<EPI, FAST, 4>(a, s);
+        return;
+    }
+    if constexpr (EPI == EPI_REQ) {
+        if (nks > 8 * SKINNY_U) {
+            launch_skinny_nw<EPI, FAST, 16>(a, s);
+            return;
+        }
+    }
+    launch_skinny_nw<EPI, FAST, 8>(a, s);
 }
 
 template <int EPI>
@@ -726,8 +734,8 @@ static bool try_skinny(const GemmArgs& a, hipStream_t s) {
     if (a.tiled || !a.Wf || a.a_rows || a.M <= 0 || a.M > most || a.N % 64 != 0 || a.K % 64 != 0 ||
         (long long)a.N * a.K >= (1ll << 31))
         return false;
-    if (a.rq_fast) launch_skinny<EPI, true>(a, s);
-    else launch_skinny<EPI, false>(a, s);
+    if (EPI == EPI_RAW || a.rq_fast) launch_skinny<EPI, true>(a, s);
+    else if constexpr (EPI != EPI_RAW) launch_skinny<EPI, false>(a, s);
     return true;
 }
 

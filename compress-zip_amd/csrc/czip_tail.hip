@@ -105,8 +105,9 @@ __global__ __launch_bounds__(64 * TNW) void k_layer_tail(TailArgs a) {
                 }
             }
     }
-    // a share of the weights ahead of their streaming: 2 MB of the up rows, 1 MB
-    // each of the others with 32 workgroups an XCD
+    // a share of the weights ahead of their streaming, 64 KB a workgroup and
+    // request: with 32 workgroups an XCD up to 4 MB of the up rows (the second
+    // request lies past those of most models), 2 MB each of the others
     int touched[4] = {0, 0, 0, 0};
     const int tns = min((int)gridDim.x, 256) >> 3, ts = (int)blockIdx.x >> 3;
     if (ts < tns) {
