@@ -297,12 +297,14 @@ struct czip_ctx {
     std::vector<Pending> pending;
     std::vector<hipEvent_t> event_pool;
     czip_job* dec = nullptr;  // step-wise decode session (czip_decode_begin)
+    czip_job* jobs = nullptr; // the live jobs (a list through next / prev)
     uint8_t* noalloc = nullptr;  // this device's copy of `scratch` (czip_prefill_cdf_noalloc)
     std::string noalloc_err;
 };
 
 struct czip_job {
-    czip_ctx* ctx = nullptr;
+    czip_ctx* ctx = nullptr;  // nullptr once the context is destroyed: the job holds nothing any more
+    czip_job *next = nullptr, *prev = nullptr;
     int kind = 0;  // 0 prefill (compress, rows in and out), 1 decompress, 2 decode session
     int64_t n_tokens = 0, nchunks = 0;
     int T = 0, BC = 0;
@@ -759,12 +761,21 @@ extern "C" czip_status czip_create(const czip_model_desc* w, int device, czip_ct
 }
 
 static void free_decode_session(czip_ctx* c);
+namespace {
+void free_job_mem(czip_job* j);
+void detach_job(czip_job* j);
+}  // namespace
 
 extern "C" void czip_destroy(czip_ctx* c) {
     if (!c) return;
     hipSetDevice(c->device);
     if (c->stream) hipStreamSynchronize(c->stream);
     free_decode_session(c);
+    while (czip_job* j = c->jobs) {
+        free_job_mem(j);
+        detach_job(j);
+        j->ctx = nullptr;
+    }
     for (auto& p : c->pending) { hipEventDestroy(p.a); hipEventDestroy(p.b); }
     for (auto e : c->event_pool) hipEventDestroy(e);
     for (auto& a : c->allocs) hipFree(a.p);
@@ -1048,6 +1059,20 @@ czip_status check_tokens(czip_ctx* c, const uint32_t* t, int64_t n) {
 
 void free_job_mem(czip_job* j) { release(j->ctx, j->allocs); }
 
+// The context knows its live jobs: one that outlives it (a garbage collector
+// may finalize either first) gives its memory back at czip_destroy.
+void attach_job(czip_ctx* c, czip_job* j) {
+    j->next = c->jobs;
+    if (c->jobs) c->jobs->prev = j;
+    c->jobs = j;
+}
+void detach_job(czip_job* j) {
+    if (j->prev) j->prev->next = j->next;
+    else j->ctx->jobs = j->next;
+    if (j->next) j->next->prev = j->prev;
+    j->next = j->prev = nullptr;
+}
+
 // Debug paths (forward_logits / prefill_cdf / prefill_cumfreqs): one job
 // over caller-given input rows, processed in sub-batches.
 czip_status run_rows(czip_ctx* c, const uint32_t* rows_in, const uint32_t* rows_tgt, const int32_t* lens, int B, int T,
@@ -1179,6 +1204,7 @@ extern "C" czip_status czip_compress_plan(czip_ctx* c, const uint32_t* tokens, i
         hipError_t e = hipMemcpy(j->tok, tokens, (size_t)n * 4, hipMemcpyHostToDevice);
         if (e != hipSuccess) { free_job_mem(j.get()); return fail(c, CZIP_E_HIP, hipGetErrorString(e)); }
     }
+    attach_job(c, j.get());
     *out = j.release();
     return CZIP_OK;
 }
@@ -1226,7 +1252,7 @@ static czip_status run_compress(czip_job* j) {
 static czip_status run_decompress(czip_job* j);
 
 extern "C" czip_status czip_job_run(czip_job* j) {
-    if (!j) return CZIP_E_ARG;
+    if (!j || !j->ctx) return CZIP_E_ARG;
     j->ran = false;
     HIPCHECK(j->ctx, hipSetDevice(j->ctx->device));
     czip_status rc;
@@ -1238,7 +1264,7 @@ extern "C" czip_status czip_job_run(czip_job* j) {
 }
 
 extern "C" czip_status czip_compress_fetch(czip_job* j, uint8_t* out, int64_t slot, int32_t* lens) {
-    if (!j || j->kind != 0 || !lens || (j->nchunks > 0 && !out)) return CZIP_E_ARG;
+    if (!j || !j->ctx || j->kind != 0 || !lens || (j->nchunks > 0 && !out)) return CZIP_E_ARG;
     czip_ctx* c = j->ctx;
     if (j->nchunks == 0) return CZIP_OK;
     if (!j->ran) return fail(c, CZIP_E_ARG, "fetch before a successful czip_job_run");
@@ -1258,7 +1284,7 @@ extern "C" czip_status czip_compress_fetch(czip_job* j, uint8_t* out, int64_t sl
 }
 
 extern "C" czip_status czip_compress_fetch_packed(czip_job* j, uint8_t* out, int64_t cap, int64_t* offs) {
-    if (!j || j->kind != 0 || !offs) return CZIP_E_ARG;
+    if (!j || !j->ctx || j->kind != 0 || !offs) return CZIP_E_ARG;
     czip_ctx* c = j->ctx;
     offs[0] = 0;
     if (j->nchunks == 0) return CZIP_OK;
@@ -1367,6 +1393,7 @@ extern "C" czip_status czip_decompress_plan(czip_ctx* c, const uint8_t* data, co
         free_job_mem(j.get());
         return fail(c, CZIP_E_HIP, hipGetErrorString(e));
     }
+    attach_job(c, j.get());
     *out = j.release();
     return CZIP_OK;
 }
@@ -1531,7 +1558,7 @@ static czip_status run_decompress(czip_job* j) {
 }
 
 extern "C" czip_status czip_decompress_fetch(czip_job* j, uint32_t* tokens_out, const int64_t* tok_offs) {
-    if (!j || j->kind != 1 || (j->total_tokens > 0 && !tokens_out)) return CZIP_E_ARG;
+    if (!j || !j->ctx || j->kind != 1 || (j->total_tokens > 0 && !tokens_out)) return CZIP_E_ARG;
     czip_ctx* c = j->ctx;
     if (j->total_tokens == 0) return CZIP_OK;
     if (!j->ran) return fail(c, CZIP_E_ARG, "fetch before a successful czip_job_run");
@@ -1552,8 +1579,11 @@ extern "C" czip_status czip_decompress_fetch(czip_job* j, uint32_t* tokens_out, 
 
 extern "C" void czip_job_free(czip_job* j) {
     if (!j) return;
-    hipSetDevice(j->ctx->device);
-    free_job_mem(j);
+    if (j->ctx) {
+        hipSetDevice(j->ctx->device);
+        free_job_mem(j);
+        detach_job(j);
+    }
     delete j;
 }
 

@@ -165,6 +165,8 @@ czip_status czip_compress_fetch(czip_job* job, uint8_t* out, int64_t slot, int32
  * below that gives CZIP_E_OVERFLOW.  (The same bytes as czip_compress_fetch,
  * which keeps the reference's one-Vec-per-chunk shape, main.rs:206-238.) */
 czip_status czip_compress_fetch_packed(czip_job* job, uint8_t* out, int64_t cap, int64_t* offs);
+/* A job of a destroyed context holds nothing any more: it can only be freed
+ * (its other calls give CZIP_E_ARG). */
 void        czip_job_free(czip_job* job);
 /* Upper bound of one chunk's coded size for `chunk` tokens. */
 int64_t     czip_chunk_slot_bytes(int32_t chunk);

@@ -68,6 +68,36 @@ def test_job_memory_reuse(pair):
         j.free()
 
 
+def test_jobs_outlive_their_context(amd, pair):
+    """A collector may finalize a model before its jobs: their memory goes with
+    the context, and all that is left to do with them is to free them."""
+    _, om = pair
+    toks = np.random.default_rng(12).integers(0, 1024, 2000).astype(np.uint32)
+    want = om.compress_many(toks, 64, threads=4)
+    gm = amd.Model(amd.ModelWeights(MODEL_PATH))
+    jobs = [gm.compress_plan(toks, 64), gm.decompress_plan(want, [64] * 31 + [16]), gm.compress_plan(toks, 64),
+            gm.compress_plan(toks, 64)]
+    for j in jobs[:3]:
+        j.run()
+    jobs[2].free()
+    gm.close()
+    for j in (jobs[0], jobs[1], jobs[3]):
+        for call in (j.run, j.fetch):
+            with pytest.raises(amd.CzipError) as e:
+                call()
+            assert e.value.code == -1
+        j.free()
+    # a context after it, and a job freed out of order in it
+    gm = amd.Model(amd.ModelWeights(MODEL_PATH))
+    a, b, c = (gm.compress_plan(toks, 64) for _ in range(3))
+    b.free()
+    for j in (a, c):
+        j.run()
+        assert j.fetch() == want
+        j.free()
+    gm.close()
+
+
 def test_job_memory_trim(amd, pair):
     """Freed jobs' memory goes back to the driver on demand, the live ones' stays."""
     _, om = pair
