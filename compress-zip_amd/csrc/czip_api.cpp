@@ -52,30 +52,6 @@ constexpr long long ATTN_ROWS_MAX = 8192;
 // 18944 0.511 -> 0.505, 26752 0.277 -> 0.280, 65536 0.82 -> 0.84
 constexpr int64_t TAIL_ROWS_MAX = 20480;
 constexpr size_t TAIL_WEIGHTS_MAX = (size_t)4 << 20, TAIL_WEIGHT_BYTES_PER_ROW = 2500;
-// A workgroup's time is the weights' stream whatever its rows, so past one round
-// of the 256 CUs the tail loses where the next round is nearly empty, the more
-// the larger the weights.  Rows of a round: 8192, or 4096 where a feed-forward
-// past 2048 leaves LDS for 16 rows a workgroup only.  4 to 8 layers, separate
-// kernels -> tail:
-//  - 16 rows only: up to one round and the fuller half of the second.  d384 / F =
-//    3072 prefill 4096 rows 462 -> 438 us, 4200 510 -> 583, 6400 625 -> 596, 8192 647
-//    -> 622, 8400 665 -> 770; 32 decode steps 4200 10.7 -> 13.2 ms, 6400 14.3 -> 13.5,
-//    8400 15.7 -> 19.1; d256 / 4096 prefill 12288 570 -> 587, 20480 791 -> 862
-//  - more than 3 MB (d512 / 2048): prefills up to one round (8192 rows 1.28 -> 1.08
-//    ms, 8320 1.30 -> 1.43, 12288 1.48 -> 1.55, 18432 2.17 -> 2.15); decode steps
-//    not in the emptier half of the second (8200 33.8 -> 35.0 ms, 11000 37.4 ->
-//    37.7, 13300 40.9 -> 39.6, 16500 57.5 -> 56.5)
-//  - 2 to 3 MB: prefills likewise without that half (d512 / 1536 8320 rows 739 ->
-//    769 us, 12288 831 -> 834, 16640 1093 -> 1058; d384 / 2048 8200 596 -> 605, 13300
-//    662 -> 646), decode steps all (d512 / 1024 8200 14.4 -> 13.8 ms)
-//  - less: all (shipped model 8200 rows 253 -> 243 us, 16500 306 -> 295)
-constexpr size_t TAIL_WEIGHTS_LARGE = (size_t)3 << 20, TAIL_WEIGHTS_MEDIUM = (size_t)2 << 20;
-bool tail_rounds_pay(int64_t M, int F, size_t weights, bool decode) {
-    if (F > 2048) return M <= 4096 || (M >= 6144 && M <= 8192);
-    if (M <= 8192 || weights <= TAIL_WEIGHTS_MEDIUM) return true;
-    if (weights <= TAIL_WEIGHTS_LARGE) return decode || M >= 12288;
-    return decode && M >= 12288;
-}
 // GEMMs of at most this many rows split K over a workgroup's waves and the
 // columns over the chip (CZIP_SKINNY_ROWS); half of it where the layer tail
 // takes over below it.  A step-wise decode step, other kernels -> these: d768
@@ -889,7 +865,7 @@ bool post_attention(czip_ctx* c, const RowBufs& r, int l, int M, hipStream_t s, 
     const bool last = l + 1 == c->cfg.n_layers;
     const int8_t* next = last ? c->final_norm : c->layers[(size_t)l + 1].attn_norm;
     if (M > r.skinny_rows && M >= c->tail_rows_min && M <= c->tail_rows &&
-        (!c->tail_rounds || tail_rounds_pay(M, F, c->layer_weights, r.decode))) {
+        (!c->tail_rounds || tail_rounds_pay(M, F, c->layer_weights, r.decode, beside_lanes))) {
         GemmArgs o{}, u{}, dn{};  // requantization scales (the fast path, checked at czip_create)
         o.K = d; set_requant(o, L.out_mult, L.out_shift);
         u.K = d; set_requant(u, L.up_mult, L.up_shift);

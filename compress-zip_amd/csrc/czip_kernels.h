@@ -293,6 +293,9 @@ struct TailArgs {
     GemmArgs qkv;
 };
 bool tail_supported(int d, int F);
+// whether it is the faster way for a launch of M rows (weights: a layer's bytes;
+// decode: a decode step, lanes: beside others)
+bool tail_rounds_pay(int64_t M, int F, size_t weights, bool decode, bool lanes);
 void launch_layer_tail(const TailArgs& a, int d, hipStream_t s);
 
 }  // namespace czip

@@ -316,6 +316,36 @@ static int tail_rt(int M, int F) { return M > 16 * 256 && 32 * F <= TAIL_R8_BYTE
 
 bool tail_supported(int d, int F) { return (d == 256 || d == 384 || d == 512) && F % 64 == 0 && 16 * F <= TAIL_R8_BYTES; }
 
+// A workgroup's time is the weights' stream whatever its rows, so past one round
+// of the 256 CUs the tail loses where the next round is nearly empty, the more
+// the larger the weights.  Rows of a round: 8192, or 4096 where a feed-forward
+// past 2048 leaves LDS for 16 rows a workgroup only.  4 to 8 layers, separate
+// kernels -> tail:
+//  - 16 rows only: up to one round and the fuller half of the second.  d384 / F =
+//    3072 prefill 4096 rows 462 -> 438 us, 4200 510 -> 583, 6400 625 -> 596, 8192 647
+//    -> 622, 8400 665 -> 770; 32 decode steps 4200 10.7 -> 13.2 ms, 6400 14.3 -> 13.5,
+//    8400 15.7 -> 19.1; d256 / 4096 prefill 12288 570 -> 587, 20480 791 -> 862
+//  - more than 3 MB (d512 / 2048): prefills up to one round (8192 rows 1.28 -> 1.08
+//    ms, 8320 1.30 -> 1.43, 12288 1.48 -> 1.55, 18432 2.17 -> 2.15); decode steps
+//    not in the emptier half of the second (8200 33.8 -> 35.0 ms, 11000 37.4 ->
+//    37.7, 13300 40.9 -> 39.6, 16500 57.5 -> 56.5)
+//  - 2 to 3 MB: prefills likewise without that half (d512 / 1536 8320 rows 739 ->
+//    769 us, 12288 831 -> 834, 16640 1093 -> 1058; d384 / 2048 8200 596 -> 605, 13300
+//    662 -> 646), decode steps all (d512 / 1024 8200 14.4 -> 13.8 ms)
+//  - less: all (shipped model 8200 rows 253 -> 243 us, 16500 306 -> 295)
+// Beside other decode lanes, whose kernels fill the separate ones' last rounds,
+// only with weights of up to 2 MB (32 steps of 40 thousand streams in two lanes:
+// d512 / 2048, 8 layers 91.1 -> 97.5 ms, d384 / 2048 37.8 -> 40.8, d512 / 1024 38.9 ->
+// 40.0; shipped model 7.69 -> 7.42, d256 / 1024 21.3 -> 20.8).
+static constexpr size_t TAIL_WEIGHTS_LARGE = (size_t)3 << 20, TAIL_WEIGHTS_MEDIUM = (size_t)2 << 20;
+bool tail_rounds_pay(int64_t M, int F, size_t weights, bool decode, bool lanes) {
+    if (lanes && weights > TAIL_WEIGHTS_MEDIUM) return false;
+    if (F > 2048) return M <= 4096 || (M >= 6144 && M <= 8192);
+    if (M <= 8192 || weights <= TAIL_WEIGHTS_MEDIUM) return true;
+    if (weights <= TAIL_WEIGHTS_LARGE) return decode || M >= 12288;
+    return decode && M >= 12288;
+}
+
 template <int KS>
 static void launch_tail(const TailArgs& a, hipStream_t s) {
     const int rt = tail_rt(a.M, a.F);

@@ -15,8 +15,8 @@ void launch_rn_splitk_epi(const RowGemmArgs&, const int32_t*, int, hipStream_t) 
 using namespace czip;
 
 namespace {
-std::vector<int8_t> mem((size_t)192 << 20);  // plain loads and stores land here
-int8_t* at(size_t mb) { return mem.data() + (mb << 20); }
+int8_t* const mem = (int8_t*)std::calloc(192, 1 << 20);  // plain loads and stores land here
+int8_t* at(size_t mb) { return mem + (mb << 20); }
 
 GemmArgs gemm_args(int M, int N, int K, int T) {
     GemmArgs g{};
@@ -91,6 +91,7 @@ int main(int argc, char** argv) {
     else if (!std::strcmp(argv[1], "tail")) tail(v[0], v[1], v[2], v[3] != 0);
     else if (!std::strcmp(argv[1], "fused")) fused(v[0], v[1], v[2]);
     else if (!std::strcmp(argv[1], "attention")) attention(v[0], v[1], v[2]);
+    else if (!std::strcmp(argv[1], "tail_rounds")) return std::printf("%d\n", tail_rounds_pay(v[0], v[1], (size_t)v[2], v[3], v[4])) < 0;
     else return 2;
     std::printf("%ld accesses, %ld bad\n", bounds::accesses, bounds::bad);
     return bounds::bad ? 1 : 0;

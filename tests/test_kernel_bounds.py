@@ -1,7 +1,8 @@
-"""Buffer accesses of the kernels that request operands ahead of their use,
-checked in a CPU build (kernel_bounds/): the range check of a buffer resource
-is specified for the vector offset only, so every access must be masked by its
-vector offset alone or lie inside its resource, scalar offset included."""
+"""Kernel sources in a CPU build (kernel_bounds/): the layer tail's rule, and the
+buffer accesses of the kernels that request operands ahead of their use.  The
+range check of a buffer resource is specified for the vector offset only, so
+every access must be masked by its vector offset alone or lie inside its
+resource, scalar offset included."""
 import glob
 import os
 import subprocess
@@ -48,6 +49,29 @@ def program(tmp_path_factory):
     subprocess.run([CLANG, "-O0", "-std=c++17", "-w", "-x", "c++", "-I", HERE, "-I", str(src), "-I", os.path.join(ROOT, "include"),
                     os.path.join(HERE, "bounds.cpp"), "-o", exe], check=True)
     return exe
+
+
+def _tail_rounds(M, F, weights, decode, lanes):
+    """The layer tail's rule on its rounds, restated from its measurements."""
+    mb = weights / (1 << 20)
+    if lanes and mb > 2:
+        return False
+    if F > 2048:  # 16 rows a workgroup: one round, and the fuller half of the second
+        return M <= 4096 or 6144 <= M <= 8192
+    if M <= 8192 or mb <= 2:
+        return True
+    half = M >= 12288  # the second round is at least half full
+    return half if decode and mb > 3 else decode or (half and mb <= 3)
+
+
+def test_layer_tail_rounds_rule(program):
+    for F, weights in ((512, 1 << 20), (2048, 2 << 20), (2048, (2 << 20) + 1), (1536, 3 << 20), (2048, (3 << 20) + 1), (3072, 1 << 20),
+                       (3072, 4 << 20)):
+        for M in (600, 4096, 4097, 6143, 6144, 8192, 8193, 12287, 12288, 20480):
+            for decode in (0, 1):
+                for lanes in (0, decode):
+                    r = subprocess.run([program, "tail_rounds", *map(str, (M, F, weights, decode, lanes))], capture_output=True, text=True)
+                    assert int(r.stdout) == _tail_rounds(M, F, weights, decode, lanes), (M, F, weights, decode, lanes)
 
 
 @pytest.mark.parametrize("case", CASES)
