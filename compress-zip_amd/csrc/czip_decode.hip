@@ -427,9 +427,9 @@ bool launch_attn_decode(const AttnArgs& a, int S, int p, hipStream_t s) {
 // value = ((code - low + 1) * total - 1) / range.  Also leaves the next step's
 // forward input (main.rs:386-388) in inp.  A step of few streams is one
 // chain: the decoder's state and stream words are requested with the logits,
-// and a row takes as many waves as a workgroup holds.  V = 8192, against four
-// waves a row and stream bits read one by one: 59 streams 21.6 -> 13.5 us, 512
-// 31.5 -> 23.8; with four waves still, 1024 41.2 -> 26.5.
+// and a row takes as many waves as a workgroup holds (up to CDF_FEW_ROWS rows).
+// V = 8192, against four waves a row and stream bits read one by one: 59 streams
+// 21.6 -> 13.5 us; with four waves still, 512 31.5 -> 20.8, 1024 41.2 -> 26.5.
 // ---------------------------------------------------------------------------
 template <int WPR, int EPL>
 __global__ __launch_bounds__(64 * WPR) void k_cdf_decode(const int32_t* __restrict__ logits, int V,
@@ -574,7 +574,7 @@ void launch_cdf_decode(const int32_t* logits, int S, int V, const uint16_t* lut,
                        DecState st, DecStreams ds, uint32_t* inp, hipStream_t s) {
 #define CZIP_CDF_DEC(W, E) \
     hipLaunchKernelGGL((k_cdf_decode<W, E>), dim3((unsigned)S), dim3(64 * W), 0, s, logits, V, lut, coef, total, p, st, ds, inp)
-    const bool few = S <= CDF_FEW_ROWS;
+    const bool few = S <= CDF_FEW_ROWS * (V <= 1024 ? 2 : 1);
     if (V <= 1024) { if (few) CZIP_CDF_DEC(4, 4); else CZIP_CDF_DEC(1, 16); }
     else if (V <= 4096) { if (few) CZIP_CDF_DEC(16, 4); else CZIP_CDF_DEC(4, 16); }
     else { if (few) CZIP_CDF_DEC(16, 8); else CZIP_CDF_DEC(4, 32); }

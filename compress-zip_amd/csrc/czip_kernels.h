@@ -188,10 +188,14 @@ void launch_attention(const AttnArgs& a, int B, hipStream_t s);
 // mode 0: (lo, hi) of targets; mode 1: full inclusive cumfreqs; mode 2:
 // targets are decoder values, out rows (sym, cum_lo, cum_hi).  Row r of the
 // launch is written at output row out_row0 + r.
-// Launches of at most this many rows (two workgroups of 16 waves a CU) give a
-// row to as many waves as hold its logits at 4 or 8 a lane: they are bound by
-// one row's chain of reductions
-constexpr int CDF_FEW_ROWS = 512;
+// Launches of few rows give a row to as many waves as hold its logits at 4 or 8 a
+// lane: they are bound by one row's chain of reductions.  Up to a workgroup of 16
+// waves a CU; up to two where the waves are 4 (V <= 1024), and for k_cdf past V =
+// 4096.  us a launch, one or four waves a row -> four or sixteen: V = 1024 512 rows
+// 11.3 -> 8.9 (k_cdf), 11.9 -> 10.1 (k_cdf_decode); 2048 256 rows 11.5 -> 9.9, 12.7 ->
+// 12.1; 300 rows 12.0 -> 12.3, 13.2 -> 15.0; 4096 512 rows 13.0 -> 13.4, 14.1 -> 16.3;
+// 8192 256 rows 17.0 -> 12.7, 18.0 -> 14.7; 512 rows 18.9 -> 17.1, 20.8 -> 23.4
+constexpr int CDF_FEW_ROWS = 256;
 void launch_cdf(const int32_t* logits, int M, int V, const uint32_t* targets, const int32_t* lens, int T,
                 const uint16_t* lut, unsigned coef, unsigned total, int mode, uint32_t* out, int64_t out_row0,
                 hipStream_t s);

@@ -650,7 +650,7 @@ void launch_cdf(const int32_t* logits, int M, int V, const uint32_t* targets, co
 #define CZIP_CDF(W, E)                                                                                             \
     hipLaunchKernelGGL((k_cdf<W, E>), dim3((unsigned)M), dim3(64 * W), 0, s, logits, V, targets, lens, T, lut, coef, \
                        total, mode, out, (long long)out_row0)
-    const bool few = M <= CDF_FEW_ROWS;
+    const bool few = M <= CDF_FEW_ROWS * (V <= 1024 || V > 4096 ? 2 : 1);
     if (V <= 1024) { if (few) CZIP_CDF(4, 4); else CZIP_CDF(1, 16); }
     else if (V <= 4096) { if (few) CZIP_CDF(16, 4); else CZIP_CDF(4, 16); }
     else { if (few) CZIP_CDF(16, 8); else CZIP_CDF(4, 32); }

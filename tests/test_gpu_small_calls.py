@@ -503,7 +503,7 @@ def test_general_requantization_leaves_the_wide_tiles(amd, orc, tmp_path, monkey
 @pytest.mark.parametrize("vocab,env", [(1024, "CZIP_UNFUSED_HEAD"), (1088, None), (4096, None), (4160, None), (8192, None)])
 def test_decode_step_wave_counts(amd, orc, tmp_path, monkeypatch, vocab, env):
     """The unfused head's decoder step with a row's logits over one, four and
-    sixteen waves (up to 512 rows, then more), at the edges of their vocabulary
+    sixteen waves (up to 256 or 512 rows, then more), at the edges of their vocabulary
     ranges; streams that end at different steps and streams cut short."""
     from czip_amd import synth
     if env:
@@ -515,7 +515,7 @@ def test_decode_step_wave_counts(amd, orc, tmp_path, monkeypatch, vocab, env):
     rng = np.random.default_rng(vocab)
     toks = rng.integers(0, vocab, 24 * 13).astype(np.uint32)
     coded = om.compress_many(toks, 13, threads=8)
-    for S in (24, 512, 513):
+    for S in (24, 256, 257, 512, 513):
         pick = rng.integers(0, 24, S)
         lens = rng.integers(0, 14, S).astype(np.int32)
         want = np.concatenate([toks[13 * c:13 * c + n] for c, n in zip(pick, lens)])
