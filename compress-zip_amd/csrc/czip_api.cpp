@@ -274,6 +274,7 @@ struct czip_ctx {
     std::vector<hipEvent_t> event_pool;
     czip_job* dec = nullptr;  // step-wise decode session (czip_decode_begin)
     czip_job* jobs = nullptr; // the live jobs (a list through next / prev)
+    std::mutex jobs_mu;       // a collector may free a job on a thread of its own
     uint8_t* noalloc = nullptr;  // this device's copy of `scratch` (czip_prefill_cdf_noalloc)
     std::string noalloc_err;
 };
@@ -1038,11 +1039,13 @@ void free_job_mem(czip_job* j) { release(j->ctx, j->allocs); }
 // The context knows its live jobs: one that outlives it (a garbage collector
 // may finalize either first) gives its memory back at czip_destroy.
 void attach_job(czip_ctx* c, czip_job* j) {
+    std::lock_guard<std::mutex> lock(c->jobs_mu);
     j->next = c->jobs;
     if (c->jobs) c->jobs->prev = j;
     c->jobs = j;
 }
 void detach_job(czip_job* j) {
+    std::lock_guard<std::mutex> lock(j->ctx->jobs_mu);
     if (j->prev) j->prev->next = j->next;
     else j->ctx->jobs = j->next;
     if (j->next) j->next->prev = j->prev;

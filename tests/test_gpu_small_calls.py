@@ -4,6 +4,8 @@ attention by rows, few-row GEMMs, whole-stream decode, layer tail, 128 x 256
 tiles and the wave counts of the unfused decoder step; and device memory that
 jobs hand on."""
 import ctypes as C
+import queue
+import threading
 
 import numpy as np
 import pytest
@@ -87,6 +89,22 @@ def test_jobs_outlive_their_context(amd, pair):
                 call()
             assert e.value.code == -1
         j.free()
+    # jobs freed by another thread while this one makes more
+    gm = amd.Model(amd.ModelWeights(MODEL_PATH))
+    made = queue.Queue()
+
+    def free_all():
+        while (j := made.get()) is not None:
+            j.free()
+
+    t = threading.Thread(target=free_all)
+    t.start()
+    for _ in range(300):
+        made.put(gm.compress_plan(toks[:64], 64))
+    made.put(None)
+    t.join()
+    assert gm.compress_chunks(toks, 64) == want
+    gm.close()
     # a context after it, and a job freed out of order in it
     gm = amd.Model(amd.ModelWeights(MODEL_PATH))
     a, b, c = (gm.compress_plan(toks, 64) for _ in range(3))
@@ -141,7 +159,6 @@ def test_split_k_workspace_only_where_used(amd, tmp_path, monkeypatch, d_ff, env
 
 def test_job_memory_threads(amd, pair):
     """A context per thread, both taking and returning device memory at the same time."""
-    import threading
     _, om = pair
     toks = np.random.default_rng(6).integers(0, 1024, 5000).astype(np.uint32)
     want = {c: om.compress_many(toks, c, threads=4) for c in (64, 200)}
